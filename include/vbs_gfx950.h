@@ -220,8 +220,8 @@ int vbs_gfx950_linear_batch(int type, const void *w, const float *x, uint32_t x_
 /* Up to three matrices of one type and column count over the same vectors
  * (Q, K and V, or gate and up): for m < n_mat, Y_m[b*y_stride[m] + r] =
  * sum_c deq(W_m[r,c]) * X[b*x_stride + c], b < batch (<= 16). Equal to n_mat
- * calls of vbs_gfx950_linear_batch; for Q4_K and Q6_K the vectors are
- * prepared once and every matrix shares one matrix-core launch, as the
+ * calls of vbs_gfx950_linear_batch; for Q4_K, Q6_K, Q4_0, Q4_1, Q8_0 and F16 the
+ * vectors are prepared once and every matrix shares one matrix-core launch, as the
  * batched decoder runs a layer's Q/K/V and gate/up. w, rows, y and y_stride
  * are host arrays of n_mat entries (w[m] and y[m] device pointers). No
  * counterpart in the reference (it has no batched matvec). */
@@ -253,8 +253,8 @@ int vbs_gfx950_checksum_variant(const void *p, size_t bytes, uint32_t *partials,
 /* The library's stream (a hipStream_t), for callers that time kernels with
  * HIP events or capture the stream into a graph.
  *
- * Capture and the library's scratch: vbs_gfx950_linear_batch (Q4_K / Q6_K)
- * and vbs_gfx950_attention keep intermediate results in a device scratch
+ * Capture and the library's scratch: vbs_gfx950_linear_batch (Q4_K / Q6_K; the
+ * other types run without it where it cannot grow) and vbs_gfx950_attention keep intermediate results in a device scratch
  * that the library owns. It only grows, and a buffer that a larger call
  * replaces stays allocated until the process ends, so a captured graph keeps
  * valid memory whatever is called after the capture. Growing allocates, so a

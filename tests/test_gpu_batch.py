@@ -197,6 +197,57 @@ def test_batch_multi_matrix_launch(dev, host, oracle, mem, t, shapes, cols, batc
                 assert lin_err(Y[b, lo:hi], want) <= LIN_TOL, (m, lo, b)
 
 
+BLK = [V.Q4_0, V.Q4_1, V.Q8_0, V.F16]
+
+
+@pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
+@pytest.mark.parametrize("shapes,cols,batch", [
+    ([1], 2304, 3), ([16], 256, 16), ([17, 33], 96, 9), ([300], 4384, 8), ([4097], 288, 2),
+    ([4113, 80, 15], 544, 5), ([8209], 256, 7), ([12301], 320, 11)])
+def test_batch_block_types(dev, host, oracle, mem, t, shapes, cols, batch):
+    """The matrix-core batched kernel of the 32-element block types and F16:
+    one, two and three tiles per workgroup (up to 256, 512 and more tiles),
+    launches across matrix boundaries, partial last tiles, workgroups and
+    256-element units (rows of 96 to 4384 elements at every 2-byte offset),
+    one and two groups of eight vectors, strides wider than the row; every
+    row against the oracle, the padding untouched."""
+    xs, pad = cols + 4, 3
+    ws = [V.synth_matrix(host, t, r, cols, SEED, 180 + m) for m, r in enumerate(shapes)]
+    X = vectors(host, batch, cols, 190)
+    Xp = np.zeros((batch, xs), np.float32)
+    Xp[:, :cols] = X
+    pws = [mem.up(w) for w in ws]
+    pys = [mem.up(np.full(batch * (r + pad), -3.0, np.float32)) for r in shapes]
+    dev.linear_batch_multi(t, pws, shapes, mem.up(Xp), xs, pys, [r + pad for r in shapes], cols, batch)
+    for m, (w, r) in enumerate(zip(ws, shapes)):
+        Y = dev.download(pys[m], (batch, r + pad), np.float32)
+        assert np.all(Y[:, r:] == -3.0), m
+        for b in range(batch):
+            want = oracle.linear(t, w, X[b], cols, r)
+            assert lin_err(Y[b, :r], want) <= LIN_TOL, (m, b)
+
+
+@pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
+def test_batch_block_types_non_finite(dev, host, oracle, mem, t):
+    """inf and NaN in a vector and in a row's scales give the oracle's inf and
+    NaN rows; the other vectors and rows stay within the bar."""
+    rows, cols = 64, 1024
+    w = V.synth_matrix(host, t, rows, cols, SEED, 74)
+    w[7, :2] = np.array([0x7C00], np.uint16).view(np.uint8)  # an infinite scale (F16: weight)
+    w[9, :2] = np.array([0x7E00], np.uint16).view(np.uint8)  # NaN
+    X = vectors(host, 6, cols, 110)
+    X[1, 300], X[2, 5], X[3, 1000] = np.inf, np.nan, -np.inf
+    Y = run_batch(dev, mem, t, w, X, rows, cols)
+    for b in range(6):
+        with np.errstate(invalid="ignore"):
+            want = oracle.linear(t, w, X[b], cols, rows)
+        fine = np.isfinite(want)
+        assert np.array_equal(np.isnan(Y[b]), np.isnan(want)), b
+        assert np.array_equal(Y[b][~fine & ~np.isnan(want)], want[~fine & ~np.isnan(want)]), b
+        if fine.any():
+            assert lin_err(Y[b][fine], want[fine]) <= LIN_TOL, b
+
+
 def test_scratch_growth_keeps_captured_graphs(dev, host, oracle, mem):
     """The batched matvec keeps its prepared x in the library's scratch. A
     graph captured from the library's stream holds the scratch address of the

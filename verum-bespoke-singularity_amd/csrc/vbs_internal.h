@@ -98,6 +98,15 @@ hipError_t launch_kq_linear_batch(int type, const uint8_t *w, const float *x, ui
                                   uint32_t ys, uint32_t cols, uint32_t rows, uint32_t batch,
                                   hipStream_t s);
 
+// Y_m[t] = W_m * X[t] for m < nmat <= 3 matrices of one type (Q4_0, Q4_1, Q8_0;
+// F16 with rows of a multiple of 8 elements at 16-byte alignment) and t < batch
+// <= 16 on the f16 matrix cores, the weights read once, x prepared into the
+// runtime scratch first; hipErrorNotSupported (nothing launched) otherwise.
+hipError_t launch_blk_linear_batch(int type, uint32_t nmat, const uint8_t *const w[],
+                                   const uint32_t rows[], const float *x, uint32_t xs,
+                                   float *const y[], const uint32_t ys[], uint32_t cols,
+                                   uint32_t batch, hipStream_t s);
+
 struct MvArgs;
 // Q4_K matvec with each workgroup's whole row range in flight (rows of 16
 // blocks, 4096-12288 rows, 16-byte aligned w and x); hipErrorNotSupported

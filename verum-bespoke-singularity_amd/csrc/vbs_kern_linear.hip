@@ -191,7 +191,8 @@ hipError_t launch_linear(int type, const uint8_t *w, const float *x, float *y, u
     return hipGetLastError();
 }
 
-// Batched: a wavefront owns one row and loops the batch, so each weight unit
+// Batched, for what the matrix cores do not take (F32, LNS8, F16 rows off 8
+// elements or 16 bytes, little work): a wavefront owns one row and loops the batch, so each weight unit
 // is decoded once and used `batch` times (weights read once from HBM).
 template <int T, int NB>
 __global__ __launch_bounds__(256) void k_linear_batch(const uint8_t *__restrict__ w,
@@ -252,6 +253,10 @@ hipError_t launch_linear_batch(int type, const uint8_t *w, const float *x, uint3
             e = launch_kq_linear_batch(type, w, x + (uint64_t)b0 * xs, xs, y + (uint64_t)b0 * ys, ys,
                                        cols, rows, min(8u, batch - b0), s);
         if (e != hipErrorNotSupported) return e;  // the shape check fails on the first launch
+    }
+    {  // Q4_0, Q4_1, Q8_0 and F16: the matrix cores again, all vectors in one launch
+        const hipError_t e = launch_blk_linear_batch(type, 1u, &w, &rows, x, xs, &y, &ys, cols, batch, s);
+        if (e != hipErrorNotSupported) return e;
     }
     uint64_t rb = row_bytes(type, cols);
     dim3 grid((rows + 3u) / 4u), block(256);

@@ -4,6 +4,7 @@
 #include "vbs_attn_common.h"
 #include "vbs_lds_dma.h"
 #include "vbs_mfma.h"
+#include "vbs_mfma_batch.h"
 
 namespace vbs {
 
@@ -47,72 +48,12 @@ namespace vbs {
 // next block are in flight while one block is computed. The waves' partial
 // sums are added in wave order at the end.
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-constexpr uint32_t kBatchMax = 8;
-
-// Prepared x: [cols/8][16 planes][8] f16 | [cols/256][16 planes][8] f16
-// sub-block sums of x'/32 | int s[cols/256][8] (block, vector).
-struct XbLayout {
-    uint32_t msum, expo, bytes;
-};
-__host__ __device__ inline XbLayout xb_layout(uint32_t cols) {
-    XbLayout L;
-    L.msum = 32u * cols;
-    L.expo = 33u * cols;
-    L.bytes = 33u * cols + cols / 8u;
-    return L;
-}
-
 // What the prep reads (XP_* in vbs_internal.h): x itself, rms_norm(x) * w
 // (k_rms_norm's arithmetic and block order, src/vbs_host_math.h:28-36), or
 // silu(gate) * up (src/vbs_host_math.h:53-57, the E_SILU epilogue's expression).
 // One wave per (256-element block, vector): lane l holds elements 4l..4l+3.
 // XP_NORM: the workgroup first sums the squares of the whole vector (blocks
 // split over its waves, added in block order).
-// Block b of vector t (one wave, lane l: elements 4l..4l+3 of the block in v)
-// into the prepared form: its exponent, f16 hi/lo planes 2t and 2t + 1 and the
-// sub-block sums of x'/32.
-__device__ __forceinline__ void xprep_block(const float v[4], uint32_t lane, uint32_t t, uint32_t b,
-                                            uint32_t cols, uint8_t *xp) {
-    const uint32_t e0 = 256u * b + 4u * lane;
-    const float amax = wave_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
-    int e = 0;
-    (void)frexpf(amax, &e);  // amax < 2^e
-    const int s = amax > 0.f ? 15 - e : 0;
-    h2 hi[2], lo[2];
-    float sum = 0.f;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float xs2 = ldexpf(v[k], s);
-        const _Float16 h = (_Float16)xs2;
-        hi[k >> 1][k & 1] = h;
-        lo[k >> 1][k & 1] = (_Float16)(xs2 - (float)h);
-        sum += xs2;
-    }
-    const XbLayout L = xb_layout(cols);
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    // elements e0..e0+3: chunk e0 / 8, half lane & 1; planes 2t and 2t + 1
-    _Float16 *ph = reinterpret_cast<_Float16 *>(xp) + 128u * (e0 >> 3) + 8u * (2u * t) + 4u * (lane & 1u);
-    *reinterpret_cast<u32x2 *>(ph) = u32x2{__builtin_bit_cast(uint32_t, hi[0]), __builtin_bit_cast(uint32_t, hi[1])};
-    *reinterpret_cast<u32x2 *>(ph + 8u) = u32x2{__builtin_bit_cast(uint32_t, lo[0]), __builtin_bit_cast(uint32_t, lo[1])};
-    // sub-block sums of x'/32: eight lanes per 32 elements
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    sum += __shfl_xor(sum, 4, 64);
-    if ((lane & 7u) == 0) {
-        const float m = sum * 0.03125f;
-        const _Float16 h = (_Float16)m;
-        _Float16 *pm = reinterpret_cast<_Float16 *>(xp + L.msum) + 128u * b + 8u * (2u * t) + lane / 8u;
-        pm[0] = h;
-        pm[8] = (_Float16)(m - (float)h);
-    }
-    if (lane == 0) reinterpret_cast<int *>(xp + L.expo)[8u * b + t] = s;
-}
-
 template <int MODE>
 __global__ __launch_bounds__(256) void k_xprep_b(const float *x, const float *x2, uint32_t xs,
                                                  const float *norm_w, float eps, uint32_t cols,
@@ -191,30 +132,6 @@ struct MbArgs {
     // (cumulative), each taking rpw[m] rows of it (the last one of a matrix fewer)
     uint32_t rwg_end[3], rpw[3];
 };
-
-// This lane's A row: its plane's first eight elements and first eight
-// sub-block sums; element chunk c of the plane is at plane + 128 c, block b's
-// sums at msum + 128 b.
-struct XbView {
-    const _Float16 *plane, *msum;
-    const int *expo;
-};
-
-// {1024 + byte, 1024 + byte'} as an f16 pair: bytes (0, 1) of w for sel
-// 0x00050004, (2, 3) for 0x00070006, (k, k) for 0x00040004 + 0x00010001 k.
-__device__ __forceinline__ h2 f16_bytes(uint32_t w, uint32_t sel) {
-    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(w, 0x64646464u, sel));
-}
-__device__ __forceinline__ h8 join8(h2 a, h2 b, h2 c, h2 d) {
-    const u32x4 v = {__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
-                     __builtin_bit_cast(uint32_t, c), __builtin_bit_cast(uint32_t, d)};
-    return __builtin_bit_cast(h8, v);
-}
-__device__ __forceinline__ h4 join4(h2 a, h2 b) {
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    const u32x2 v = {__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b)};
-    return __builtin_bit_cast(h4, v);
-}
 
 struct Q4KB {
     typedef Q4K Load;
@@ -1078,6 +995,10 @@ hipError_t launch_linear_batch_multi(int type, uint32_t n_mat, const uint8_t *co
                                      uint32_t batch, hipStream_t s) {
     if (n_mat == 0 || n_mat > 3u) return hipErrorInvalidValue;
     if (batch == 0) return hipSuccess;
+    {
+        const hipError_t e = launch_blk_linear_batch(type, n_mat, w, rows, x, xs, y, ys, cols, batch, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     bool mfma = type == kQ4_K || type == kQ6_K;
     for (uint32_t m = 0; m < n_mat && mfma; m++)
         mfma = rows[m] != 0 && mv_fits(type, w[m], x, cols, rows[m]);
