@@ -202,7 +202,7 @@ BLK = [V.Q4_0, V.Q4_1, V.Q8_0, V.F16]
 
 @pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
 @pytest.mark.parametrize("shapes,cols,batch", [
-    ([1], 2304, 3), ([16], 256, 16), ([17, 33], 96, 9), ([300], 4384, 8), ([4097], 288, 2),
+    ([1], 2304, 3), ([16], 256, 16), ([17, 33], 96, 9), ([300], 4384, 8), ([3000], 4384, 8), ([4097], 288, 2),
     ([4113, 80, 15], 544, 5), ([8209], 256, 7), ([12301], 320, 11)])
 def test_batch_block_types(dev, host, oracle, mem, t, shapes, cols, batch):
     """The matrix-core batched kernel of the 32-element block types and F16:

@@ -614,6 +614,42 @@ def test_linear_random_shapes(dev, host, oracle, mem, t, rows, cols):
     assert lin_err(got, want) <= LIN_TOL, (V.TYPE_NAMES[t], rows, cols)
 
 
+@pytest.mark.parametrize("t", [V.Q4_0, V.Q4_1, V.Q8_0, V.F16, V.F32, V.LNS8],
+                         ids=lambda t: V.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (511, 544), (513, 1056), (3071, 96), (3074, 2016),
+                                       (3077, 2080), (5, 16416)])
+@pytest.mark.parametrize("batch", [1, 3, 9])
+def test_general_linear(dev, host, oracle, mem, t, rows, cols, batch):
+    """The general kernel's splits (a row on sixteen, four and one waves; two
+    and four rows sharing x; one, 4 and 16 vectors), on both sides of each
+    limit: rows that leave a group of rows, a workgroup or a wave's step
+    partly idle, F16 and F32 rows with a tail of up to seven elements at
+    element alignment, x off 16 bytes, accumulating into y."""
+    if t in (V.F16, V.F32):
+        cols += 5
+    if t == V.LNS8:
+        rng = np.random.default_rng(SEED)
+        w = rng.integers(0, 12, size=(rows, cols // 32, 36), dtype=np.uint8)
+        w[:, :, 32:36] = rng.random((rows, cols // 32, 1), np.float32).view(np.uint8)
+        w = w.reshape(rows, -1)
+    else:
+        w = V.synth_matrix(host, t, rows, cols, SEED, 51)
+    X = np.stack([synth_x(host, cols + 3, 52 + b) for b in range(batch)])
+    pw, px = mem.up(w), mem.up(X)
+    want = [oracle.linear(t, w, X[b, 3:].copy(), cols, rows) for b in range(batch)]
+    if batch > 1:
+        py = mem.zeros(batch * rows)
+        dev.linear_batch(t, pw, px + 12, cols + 3, py, rows, cols, rows, batch)
+        got = dev.download(py, (batch, rows), np.float32)
+        for b in range(batch):
+            assert lin_err(got[b], want[b]) <= LIN_TOL, b
+        return
+    y0 = synth_x(host, rows, 60)
+    py = mem.up(y0)
+    dev.linear(t, pw, px, py, cols, rows, col_off=3, accumulate=True)
+    assert lin_err(dev.download(py, rows, np.float32), y0 + want[0]) <= LIN_TOL
+
+
 def _attention_draws(n=12, seed=SEED + 6):
     rng = np.random.default_rng(seed)
     out = []

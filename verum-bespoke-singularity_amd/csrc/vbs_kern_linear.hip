@@ -1,168 +1,317 @@
-// vbs_kern_linear.hip — batch-1 linear (matvec) kernels for every hot-path
-// weight type, plus the batched (skinny) variant.
+// vbs_kern_linear.hip — the general linear (matvec) kernel, k_rows: every
+// hot-path weight type, one vector or up to 16, any shape; and the dispatch
+// of the linear entry points to the matrix-core kernels or to it.
 //
 // Semantics: vbs_host_linear_tile (src/vbs_host_math.h:223-267) —
 // y[r] (+)= sum_c deq(W[r,c]) * x[c]. Each weight is dequantised with the
 // reference's exact roundings (vbs_dev_common.h) and then accumulated in
 // fp32 with fused multiply-adds; rows are reduced across the wavefront.
-//
-// Work split: a wavefront owns one row; its 64 lanes walk the row's 32-element
-// units (a legacy block, or one sub-block of a 256-element super-block).
 #include "vbs_dev_common.h"
 #include "vbs_internal.h"
+#include "vbs_lds_dma.h"
 
 namespace vbs {
 
-// Dot of unit u (elements 32u .. 32u+31) of a packed row with x.
-template <int T> __device__ __forceinline__ float unit_dot(const uint8_t *row, uint32_t u,
-                                                          const float *x);
+namespace {
 
-template <> __device__ __forceinline__ float unit_dot<kQ4_0>(const uint8_t *row, uint32_t u,
-                                                            const float *x) {
-    const uint8_t *b = row + 18u * u;
-    const float *xb = x + 32u * u;
-    float d = h2f(ld16(b));
-    float acc = 0.f;
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t __attribute__((aligned(2))) u32h;  // words at a 2-byte aligned address
+typedef uint32_t u2h __attribute__((ext_vector_type(2), aligned(2)));
+
+// A step's share of a row: a lane takes eight elements. Blocks of 32: lane l
+// takes block l >> 2 of the step's sixteen, its quarter q = l & 3 being the
+// elements lo(q) .. + 3 and hi(q) .. + 3 (the two nibbles of four bytes; else
+// eight in a row). raw() loads the bytes, value() makes the eight weights.
+template <int T> struct Row8 {  // K-quants: element by element
+    struct Raw {
+        float w[8];
+    };
+    static constexpr uint32_t E = 32;
+    __device__ static uint32_t lo(uint32_t q) { return 8u * q; }
+    __device__ static uint32_t hi(uint32_t q) { return 8u * q + 4u; }
+    __device__ static Raw raw(const uint8_t *row, uint32_t u, uint32_t q) {
+        const uint8_t *b = row + (uint64_t)(u >> 3) * Geo<T>::B;
+        Raw r;
 #pragma unroll
-    for (int i = 0; i < 16; i += 2) {
-        uint16_t two = ld16(b + 2 + i);
+        for (uint32_t k = 0; k < 8u; k++) r.w[k] = deq_elem<T>(b, 32u * (u & 7u) + 8u * q + k);
+        return r;
+    }
+    __device__ static void value(const Raw &r, float (&w)[8]) {
 #pragma unroll
-        for (int k = 0; k < 2; k++) {
-            uint32_t byte = (two >> (8 * k)) & 255u;
-            float lo = __fmul_rn((float)(byte & 15u) - 8.0f, d);
-            float hi = __fmul_rn((float)(byte >> 4) - 8.0f, d);
-            acc = fmaf(lo, xb[i + k], acc);
-            acc = fmaf(hi, xb[16 + i + k], acc);
+        for (int k = 0; k < 8; k++) w[k] = r.w[k];
+    }
+};
+template <int T> struct Nib8 {  // Q4_0, Q4_1
+    struct Raw {
+        uint32_t q;
+        uint16_t d, m;
+    };
+    static constexpr uint32_t E = 32;
+    __device__ static uint32_t lo(uint32_t q) { return 4u * q; }
+    __device__ static uint32_t hi(uint32_t q) { return 16u + 4u * q; }
+    __device__ static Raw raw(const uint8_t *row, uint32_t u, uint32_t q) {
+        const uint8_t *b = row + (uint64_t)u * Geo<T>::B;
+        return Raw{*reinterpret_cast<const u32h *>(b + (T == kQ4_0 ? 2u : 4u) + 4u * q), ld16(b),
+                   T == kQ4_0 ? (uint16_t)0 : ld16(b + 2)};
+    }
+    __device__ static void value(const Raw &r, float (&w)[8]) {
+        const float d = h2f(r.d), m = h2f(r.m);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float n = (float)((r.q >> (8 * (k & 3) + (k >> 2) * 4)) & 15u);
+            w[k] = T == kQ4_0 ? __fmul_rn(n - 8.0f, d) : __fadd_rn(__fmul_rn(d, n), m);
         }
     }
-    return acc;
-}
-
-template <> __device__ __forceinline__ float unit_dot<kQ4_1>(const uint8_t *row, uint32_t u,
-                                                            const float *x) {
-    const uint8_t *b = row + 20u * u;
-    const float *xb = x + 32u * u;
-    float d = h2f(ld16(b)), m = h2f(ld16(b + 2));
-    float acc = 0.f;
+};
+template <> struct Row8<kQ4_0> : Nib8<kQ4_0> {};
+template <> struct Row8<kQ4_1> : Nib8<kQ4_1> {};
+template <> struct Row8<kQ8_0> {
+    struct Raw {
+        uint32_t q[2];
+        uint16_t d;
+    };
+    static constexpr uint32_t E = 32;
+    __device__ static uint32_t lo(uint32_t q) { return 8u * q; }
+    __device__ static uint32_t hi(uint32_t q) { return 8u * q + 4u; }
+    __device__ static Raw raw(const uint8_t *row, uint32_t u, uint32_t q) {
+        const uint8_t *b = row + (uint64_t)u * 34u;
+        const u32h *p = reinterpret_cast<const u32h *>(b + 2u + 8u * q);
+        return Raw{{p[0], p[1]}, ld16(b)};
+    }
+    __device__ static void value(const Raw &r, float (&w)[8]) {
+        const float d = h2f(r.d);
 #pragma unroll
-    for (int i = 0; i < 16; i += 2) {
-        uint16_t two = ld16(b + 4 + i);
+        for (int k = 0; k < 8; k++)
+            w[k] = __fmul_rn(d, (float)(int8_t)(r.q[k >> 2] >> (8 * (k & 3))));
+    }
+};
+template <> struct Row8<kLNS8> {  // exp2f(code) * scale, as deq_elem<kLNS8>
+    struct Raw {
+        u2h q;
+        float s;
+    };
+    static constexpr uint32_t E = 32;
+    __device__ static uint32_t lo(uint32_t q) { return 8u * q; }
+    __device__ static uint32_t hi(uint32_t q) { return 8u * q + 4u; }
+    __device__ static Raw raw(const uint8_t *row, uint32_t u, uint32_t q) {
+        const uint8_t *b = row + (uint64_t)u * 36u;
+        return Raw{*reinterpret_cast<const u2h *>(b + 8u * q), *reinterpret_cast<const float *>(b + 32)};
+    }
+    __device__ static void value(const Raw &r, float (&w)[8]) {
 #pragma unroll
-        for (int k = 0; k < 2; k++) {
-            uint32_t byte = (two >> (8 * k)) & 255u;
-            float lo = __fadd_rn(__fmul_rn(d, (float)(byte & 15u)), m);
-            float hi = __fadd_rn(__fmul_rn(d, (float)(byte >> 4)), m);
-            acc = fmaf(lo, xb[i + k], acc);
-            acc = fmaf(hi, xb[16 + i + k], acc);
+        for (int k = 0; k < 8; k++) {
+            const uint32_t c = (r.q[k >> 2] >> (8 * (k & 3))) & 255u;
+            w[k] = __fmul_rn(c < 128u ? __uint_as_float((c + 127u) << 23) : INFINITY, r.s);
         }
     }
-    return acc;
-}
-
-template <> __device__ __forceinline__ float unit_dot<kQ8_0>(const uint8_t *row, uint32_t u,
-                                                            const float *x) {
-    const uint8_t *b = row + 34u * u;
-    const float *xb = x + 32u * u;
-    float d = h2f(ld16(b));
-    float acc = 0.f;
-#pragma unroll
-    for (int i = 0; i < 32; i += 2) {
-        uint16_t two = ld16(b + 2 + i);
-        acc = fmaf(__fmul_rn(d, (float)(int8_t)(two & 255u)), xb[i], acc);
-        acc = fmaf(__fmul_rn(d, (float)(int8_t)(two >> 8)), xb[i + 1], acc);
+};
+// F16, F32: lane l takes elements 8 l .. 8 l + 7 of the step's 512 ("blocks" of
+// 8); rows may start at any element, so the loads are only element-aligned.
+template <> struct Row8<kF16> {
+    typedef uint32_t u4h __attribute__((ext_vector_type(4), aligned(2)));
+    struct Raw {
+        u4h v;
+    };
+    static constexpr uint32_t E = 8;
+    __device__ static uint32_t lo(uint32_t) { return 0u; }
+    __device__ static uint32_t hi(uint32_t) { return 4u; }
+    __device__ static Raw raw(const uint8_t *row, uint32_t u, uint32_t) {
+        return Raw{*reinterpret_cast<const u4h *>(row + 16ull * u)};
     }
-    return acc;
-}
-
-template <> __device__ __forceinline__ float unit_dot<kQ4_K>(const uint8_t *row, uint32_t u,
-                                                            const float *x) {
-    const uint8_t *b = row + 144u * (u >> 3);
-    uint32_t j = u & 7u;
-    const float *xb = x + 32u * u;
-    float d = h2f(ld16(b)), dmin = h2f(ld16(b + 2));
-    int sc, mn;
-    q4k_scale_min(b + 4, (int)j, sc, mn);
-    float dsc = __fmul_rn(d, (float)sc), dm = __fmul_rn(dmin, (float)mn);
-    const uint8_t *qs = b + 16 + 32 * (j >> 1);
-    uint32_t shift = (j & 1u) * 4u;
-    float acc = 0.f;
+    __device__ static void value(const Raw &r, float (&w)[8]) {
 #pragma unroll
-    for (int l = 0; l < 32; l += 2) {
-        uint16_t two = ld16(qs + l);
-        float w0 = __fsub_rn(__fmul_rn(dsc, (float)((two >> shift) & 15u)), dm);
-        float w1 = __fsub_rn(__fmul_rn(dsc, (float)((two >> (8u + shift)) & 15u)), dm);
-        acc = fmaf(w0, xb[l], acc);
-        acc = fmaf(w1, xb[l + 1], acc);
+        for (int k = 0; k < 8; k++)
+            w[k] = (float)__builtin_bit_cast(_Float16, (uint16_t)(r.v[k >> 1] >> (16 * (k & 1))));
     }
-    return acc;
-}
+};
+template <> struct Row8<kF32> {
+    struct Raw {
+        v4f a, b;
+    };
+    static constexpr uint32_t E = 8;
+    __device__ static uint32_t lo(uint32_t) { return 0u; }
+    __device__ static uint32_t hi(uint32_t) { return 4u; }
+    __device__ static Raw raw(const uint8_t *row, uint32_t u, uint32_t) {
+        const f4u *p = reinterpret_cast<const f4u *>(row + 32ull * u);
+        return Raw{p[0], p[1]};
+    }
+    __device__ static void value(const Raw &r, float (&w)[8]) {
+        w[0] = r.a.x, w[1] = r.a.y, w[2] = r.a.z, w[3] = r.a.w;
+        w[4] = r.b.x, w[5] = r.b.y, w[6] = r.b.z, w[7] = r.b.w;
+    }
+};
 
-template <> __device__ __forceinline__ float unit_dot<kQ6_K>(const uint8_t *row, uint32_t u,
-                                                            const float *x) {
-    const uint8_t *b = row + 210u * (u >> 3);
-    uint32_t j = u & 7u, h = j >> 2, q = j & 3u;
-    const float *xb = x + 32u * u;
-    float d = h2f(ld16(b + 208));
-    float s0 = __fmul_rn(d, (float)(int8_t)b[192 + 8 * h + 2 * q]);
-    float s1 = __fmul_rn(d, (float)(int8_t)b[192 + 8 * h + 2 * q + 1]);
-    const uint8_t *ql = b + 64 * h + 32 * (q & 1u);
-    const uint8_t *qh = b + 128 + 32 * h;
-    uint32_t lsh = q >= 2 ? 4u : 0u, hsh = 2u * q;
-    float acc = 0.f;
+// R rows and NB vectors per group of S waves (S = 1: every wave has rows of its
+// own; else the workgroup's S waves split the row's steps and add their sums
+// in wave order). A step is 512 elements of a row; U steps' loads go out
+// together. With NB > 1 the eight weights serve every vector.
+//
+// Bound: HBM for the large shapes, the latency of one row's loads for the
+// small ones (so few rows are split over sixteen waves). Measured, weights
+// from HBM, against the kernels it replaced (a block or a 2-byte element per
+// lane): 11008 x 4128 F16 120.6 -> 17.5 us (5.2 TB/s), F32 74.5 -> 33.5 (5.4),
+// Q4_0 29.3 -> 13.3, Q8_0 37.0 -> 14.7, LNS8 28.0 -> 15.2; 2049 x 5664 Q4_0 9.4
+// -> 6.1; 256 x 4128 F16 55.2 -> 2.8, Q4_0 5.3 -> 2.5. Vectors of their own
+// loads: F32 11008 x 4128, 4 vectors 179 -> 42, 16 vectors 521 -> 116.
+template <int T, uint32_t R, uint32_t NB, uint32_t S, uint32_t U>
+__global__ __launch_bounds__(S > 4 ? 64 * S : 256) void k_rows(const uint8_t *__restrict__ w,
+                                                               const float *__restrict__ x, uint32_t xs,
+                                                               float *__restrict__ y, uint32_t ys,
+                                                               uint32_t cols, uint32_t rows, uint64_t rb,
+                                                               uint32_t batch, int accumulate) {
+    typedef Row8<T> P;
+    constexpr uint32_t kWaves = S > 4u ? S : 4u, kGroups = kWaves / S, L = P::E / 8u;  // lanes per block
+    __shared__ float red[S > 1 ? kWaves : 1][R * NB];
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t part = S > 1u ? wave % S : 0u;
+    const uint32_t row0 = (blockIdx.x * kGroups + (S > 1u ? wave / S : wave)) * R;
+    const uint32_t q = lane % L, nu = cols / P::E;  // whole blocks (cols of F16 / F32 may have a tail)
+    const uint8_t *rp[R];
 #pragma unroll
-    for (int l = 0; l < 32; l += 2) {
-        uint16_t lo2 = ld16(ql + l), hi2 = ld16(qh + l);
+    for (uint32_t r = 0; r < R; r++) rp[r] = w + (uint64_t)min(row0 + r, rows - 1u) * rb;
+    float acc[R][NB];
 #pragma unroll
-        for (int k = 0; k < 2; k++) {
-            int lo = (lo2 >> (8 * k + lsh)) & 15;
-            int hi = (hi2 >> (8 * k + hsh)) & 3;
-            float s = (l + k) < 16 ? s0 : s1;
-            acc = fmaf(__fmul_rn(s, (float)((lo | (hi << 4)) - 32)), xb[l + k], acc);
+    for (uint32_t r = 0; r < R; r++)
+#pragma unroll
+        for (uint32_t b = 0; b < NB; b++) acc[r][b] = 0.f;
+    if (row0 < rows) {
+        for (uint32_t u0 = lane / L + (64u / L) * part; u0 < nu; u0 += (64u / L) * S * U) {
+            typename P::Raw raw[U][R];
+            v4f xa[U], xb[U];
+#pragma unroll
+            for (uint32_t k = 0; k < U; k++) {
+                const uint32_t u = min(u0 + (64u / L) * S * k, nu - 1u);  // (past the row: its last block)
+#pragma unroll
+                for (uint32_t r = 0; r < R; r++) raw[k][r] = P::raw(rp[r], u, q);
+                if constexpr (NB == 1u) {
+                    const float *xp = x + P::E * u;
+                    xa[k] = *reinterpret_cast<const f4u *>(xp + P::lo(q));
+                    xb[k] = *reinterpret_cast<const f4u *>(xp + P::hi(q));
+                }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < U; k++) {
+                const uint32_t u = u0 + (64u / L) * S * k;
+                if (u >= nu) break;
+                float wv[R][8];
+#pragma unroll
+                for (uint32_t r = 0; r < R; r++) P::value(raw[k][r], wv[r]);
+#pragma unroll
+                for (uint32_t b = 0; b < NB; b++) {
+                    if (NB > 1u && b >= batch) break;  // (uniform)
+                    v4f a, c;
+                    if constexpr (NB == 1u) {
+                        a = xa[k], c = xb[k];
+                    } else {
+                        const float *xp = x + (uint64_t)b * xs + P::E * u;
+                        a = *reinterpret_cast<const f4u *>(xp + P::lo(q));
+                        c = *reinterpret_cast<const f4u *>(xp + P::hi(q));
+                    }
+                    const float xv[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+                    for (uint32_t r = 0; r < R; r++) {
+                        float s = 0.f;
+#pragma unroll
+                        for (int e = 0; e < 8; e++) s = fmaf(wv[r][e], xv[e], s);
+                        acc[r][b] += s;
+                    }
+                }
+            }
+        }
+        if (P::E == 8u && part == 0u) {  // the tail of F16 / F32 rows: up to seven elements
+            const uint32_t c = 8u * nu + lane;
+            if (lane < 8u && c < cols) {
+#pragma unroll
+                for (uint32_t r = 0; r < R; r++)
+#pragma unroll
+                    for (uint32_t b = 0; b < NB; b++)
+                        if (NB == 1u || b < batch)
+                            acc[r][b] = fmaf(deq_elem<T>(rp[r], c), x[(uint64_t)b * xs + c], acc[r][b]);
+            }
         }
     }
-    return acc;
-}
-
-template <> __device__ __forceinline__ float unit_dot<kLNS8>(const uint8_t *row, uint32_t u,
-                                                            const float *x) {
-    const uint8_t *b = row + 36u * u;
-    const float *xb = x + 32u * u;
-    float acc = 0.f;
+    // row r of vector b ends in lane r NB + b (R NB <= 64), or in LDS first
+    float mine = 0.f;
 #pragma unroll
-    for (int i = 0; i < 32; i++) acc = fmaf(deq_elem<kLNS8>(b, i), xb[i], acc);
-    return acc;
+    for (uint32_t r = 0; r < R; r++)
+#pragma unroll
+        for (uint32_t b = 0; b < NB; b++) {
+            if (NB > 1u && b >= batch) break;
+            const float t = wave_sum(acc[r][b]);
+            if (S > 1u) {
+                if (lane == 0u) red[wave][r * NB + b] = t;
+            } else if (lane == r * NB + b) {
+                mine = t;
+            }
+        }
+    if (S > 1u) {
+        __syncthreads();
+        if (part != 0u) return;
+        if (lane < R * NB)
+            for (uint32_t k = 0; k < S; k++) mine += red[wave + k][lane];
+    }
+    const uint32_t r = lane / NB, b = lane % NB;
+    if (lane < R * NB && row0 + r < rows && b < batch) {
+        float *dst = y + (uint64_t)b * ys + row0 + r;
+        *dst = accumulate ? *dst + mine : mine;
+    }
 }
 
+template <int T, uint32_t R, uint32_t NB, uint32_t S, uint32_t U>
+hipError_t launch_rows_t(const uint8_t *w, const float *x, uint32_t xs, float *y, uint32_t ys, uint32_t cols,
+                         uint32_t rows, uint32_t batch, int accumulate, hipStream_t s) {
+    constexpr uint32_t waves = S > 4u ? S : 4u, per = waves / S * R;
+    k_rows<T, R, NB, S, U><<<(rows + per - 1u) / per, 64u * waves, 0, s>>>(w, x, xs, y, ys, cols, rows,
+                                                                        row_bytes(T, cols), batch, accumulate);
+    return hipGetLastError();
+}
+
+// Few rows: one per workgroup of sixteen waves (256 x 4128 F16 2.8 us, four
+// waves 3.5, one 6.5). Up to 3072 rows: two rows per workgroup of four waves
+// (1000 x 10528 Q4_0 6.0 us; one row on sixteen 6.7, four rows 8.7; 2049 x 5664
+// F16 6.7 / 10.3 / 6.4). Above, four rows share x (11008 x 4128 F16 17.5 us,
+// two rows 18.7, one 20.8), by a wave each where a row is under four steps
+// (32000 x 1056 Q4_0 12.0 us against 14.6). Several vectors alike: 4, 16 vectors,
+// F32 256 x 4128 4.1, 7.3 us (a wave per row 10.5, 24.8), 1000 x 10528 13.5, 38.7
+// (29.1, 100), 11008 x 4128 42.1, 115 (55.9, 147).
 template <int T>
-__global__ __launch_bounds__(256) void k_linear_units(const uint8_t *__restrict__ w,
-                                                      const float *__restrict__ x,
-                                                      float *__restrict__ y, uint32_t cols,
-                                                      uint32_t rows, uint64_t rb, int accumulate) {
-    uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
-    uint32_t lane = threadIdx.x & 63u;
-    if (row >= rows) return;  // uniform per wavefront
-    const uint8_t *rp = w + (uint64_t)row * rb;
-    float acc = 0.f;
-    for (uint32_t u = lane; u < cols / 32u; u += 64u) acc += unit_dot<T>(rp, u, x);
-    acc = wave_sum(acc);
-    if (lane == 0) y[row] = accumulate ? y[row] + acc : acc;
+hipError_t launch_rows(const uint8_t *w, const float *x, uint32_t xs, float *y, uint32_t ys, uint32_t cols,
+                       uint32_t rows, uint32_t batch, int accumulate, hipStream_t s) {
+#define VBS_ROWS(R, NB, S, U) \
+    return launch_rows_t<T, R, NB, S, U>(w, x, xs, y, ys, cols, rows, batch, accumulate, s)
+    if (batch == 1u) {
+        if (rows <= 512u) VBS_ROWS(1, 1, 16, 1);
+        if (rows <= 3072u) VBS_ROWS(2, 1, 4, 2);
+        if (cols < 2048u) VBS_ROWS(4, 1, 1, 1);
+        VBS_ROWS(4, 1, 4, 1);
+    }
+    if (batch <= 4u) {
+        if (rows <= 512u) VBS_ROWS(1, 4, 16, 1);
+        if (rows <= 3072u) VBS_ROWS(2, 4, 4, 1);
+        VBS_ROWS(4, 4, 1, 1);
+    }
+    if (rows <= 512u) VBS_ROWS(1, 16, 16, 1);
+    VBS_ROWS(2, 16, 4, 1);
+#undef VBS_ROWS
 }
 
-// F32 / F16 rows: element-granular (cols need not be a multiple of 32).
-template <int T>
-__global__ __launch_bounds__(256) void k_linear_dense(const uint8_t *__restrict__ w,
-                                                      const float *__restrict__ x,
-                                                      float *__restrict__ y, uint32_t cols,
-                                                      uint32_t rows, uint64_t rb, int accumulate) {
-    uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
-    uint32_t lane = threadIdx.x & 63u;
-    if (row >= rows) return;
-    const uint8_t *rp = w + (uint64_t)row * rb;
-    float acc = 0.f;
-    for (uint32_t c = lane; c < cols; c += 64u) acc = fmaf(deq_elem<T>(rp, c), x[c], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) y[row] = accumulate ? y[row] + acc : acc;
+hipError_t launch_rows_any(int type, const uint8_t *w, const float *x, uint32_t xs, float *y, uint32_t ys,
+                           uint32_t cols, uint32_t rows, uint32_t batch, int accumulate, hipStream_t s) {
+    switch (type) {
+        case kF32: return launch_rows<kF32>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        case kF16: return launch_rows<kF16>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        case kQ4_0: return launch_rows<kQ4_0>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        case kQ4_1: return launch_rows<kQ4_1>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        case kQ8_0: return launch_rows<kQ8_0>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        case kQ4_K: return launch_rows<kQ4_K>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        case kQ6_K: return launch_rows<kQ6_K>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        case kLNS8: return launch_rows<kLNS8>(w, x, xs, y, ys, cols, rows, batch, accumulate, s);
+        default: return hipErrorInvalidValue;
+    }
 }
+
+}  // namespace
 
 hipError_t launch_linear(int type, const uint8_t *w, const float *x, float *y, uint32_t cols,
                          uint32_t rows, int accumulate, hipStream_t s) {
@@ -175,71 +324,7 @@ hipError_t launch_linear(int type, const uint8_t *w, const float *x, float *y, u
         hipError_t e = launch_q4k_fast(w, x, y, cols, rows, accumulate, s);
         if (e != hipErrorNotSupported) return e;
     }
-    uint64_t rb = row_bytes(type, cols);
-    dim3 grid((rows + 3u) / 4u), block(256);
-    switch (type) {
-        case kF32: k_linear_dense<kF32><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        case kF16: k_linear_dense<kF16><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        case kQ4_0: k_linear_units<kQ4_0><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        case kQ4_1: k_linear_units<kQ4_1><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        case kQ8_0: k_linear_units<kQ8_0><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        case kQ4_K: k_linear_units<kQ4_K><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        case kQ6_K: k_linear_units<kQ6_K><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        case kLNS8: k_linear_units<kLNS8><<<grid, block, 0, s>>>(w, x, y, cols, rows, rb, accumulate); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-// Batched, for what the matrix cores do not take (F32, LNS8, F16 rows off 8
-// elements or 16 bytes, little work): a wavefront owns one row and loops the batch, so each weight unit
-// is decoded once and used `batch` times (weights read once from HBM).
-template <int T, int NB>
-__global__ __launch_bounds__(256) void k_linear_batch(const uint8_t *__restrict__ w,
-                                                      const float *__restrict__ x, uint32_t xs,
-                                                      float *__restrict__ y, uint32_t ys,
-                                                      uint32_t cols, uint32_t rows, uint64_t rb,
-                                                      uint32_t batch) {
-    uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
-    uint32_t lane = threadIdx.x & 63u;
-    if (row >= rows) return;
-    const uint8_t *rp = w + (uint64_t)row * rb;
-    float acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) acc[b] = 0.f;
-    if (Geo<T>::E == 1) {
-        for (uint32_t c = lane; c < cols; c += 64u) {
-            float wv = deq_elem<T>(rp, c);
-#pragma unroll
-            for (int b = 0; b < NB; b++)
-                if ((uint32_t)b < batch) acc[b] = fmaf(wv, x[(uint64_t)b * xs + c], acc[b]);
-        }
-    } else {
-        float wv[32];
-        for (uint32_t u = lane; u < cols / 32u; u += 64u) {
-            const uint8_t *blk = rp + (uint64_t)(u / (Geo<T>::E / 32u)) * Geo<T>::B;
-            uint32_t e0 = (u % (Geo<T>::E / 32u)) * 32u;
-#pragma unroll
-            for (int i = 0; i < 32; i++) wv[i] = deq_elem<T>(blk, e0 + i);
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                if ((uint32_t)b < batch) {
-                    const float *xb = x + (uint64_t)b * xs + 32u * u;
-                    float a = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 32; i++) a = fmaf(wv[i], xb[i], a);
-                    acc[b] += a;
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        if ((uint32_t)b < batch) {
-            float t = wave_sum(acc[b]);
-            if (lane == 0) y[(uint64_t)b * ys + row] = t;
-        }
-    }
+    return launch_rows_any(type, w, x, cols, y, rows, cols, rows, 1u, accumulate, s);
 }
 
 hipError_t launch_linear_batch(int type, const uint8_t *w, const float *x, uint32_t xs, float *y,
@@ -258,22 +343,7 @@ hipError_t launch_linear_batch(int type, const uint8_t *w, const float *x, uint3
         const hipError_t e = launch_blk_linear_batch(type, 1u, &w, &rows, x, xs, &y, &ys, cols, batch, s);
         if (e != hipErrorNotSupported) return e;
     }
-    uint64_t rb = row_bytes(type, cols);
-    dim3 grid((rows + 3u) / 4u), block(256);
-#define VBS_LB(T) k_linear_batch<T, 16><<<grid, block, 0, s>>>(w, x, xs, y, ys, cols, rows, rb, batch)
-    switch (type) {
-        case kF32: VBS_LB(kF32); break;
-        case kF16: VBS_LB(kF16); break;
-        case kQ4_0: VBS_LB(kQ4_0); break;
-        case kQ4_1: VBS_LB(kQ4_1); break;
-        case kQ8_0: VBS_LB(kQ8_0); break;
-        case kQ4_K: VBS_LB(kQ4_K); break;
-        case kQ6_K: VBS_LB(kQ6_K); break;
-        case kLNS8: VBS_LB(kLNS8); break;
-        default: return hipErrorInvalidValue;
-    }
-#undef VBS_LB
-    return hipGetLastError();
+    return launch_rows_any(type, w, x, xs, y, ys, cols, rows, batch, 0, s);
 }
 
 }  // namespace vbs

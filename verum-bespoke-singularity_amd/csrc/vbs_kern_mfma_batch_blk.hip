@@ -37,7 +37,7 @@
 //
 // Values that are not finite (an inf or NaN in x makes its whole block's
 // planes NaN here) are computed again by the general kernel's arithmetic, so
-// such vectors and weights give what k_linear_batch gave.
+// such vectors and weights give what k_rows gives.
 #include "vbs_mfma_batch.h"
 
 namespace vbs {
@@ -379,12 +379,16 @@ hipError_t launch_blk_linear_batch(int type, uint32_t nmat, const uint8_t *const
         tiles += (rows[m] + 15u) / 16u;
         a.tile_end[m] = tiles;
     }
-    // Little work stays on the general kernel's one launch, which ends before
-    // this path's two would (graph replays, general against matrix cores: Q4_0
-    // 1024 x 1024 one vector 4.7 / 6.1 us, two 5.4 / 6.4, four 6.7 / 6.4; F16
-    // 1024 x 256 two vectors 4.7 / 4.7; Q8_0 never: 1 x 256 5.5 / 5.5)
-    const uint32_t small = f16 ? 512u : type == kQ8_0 ? 0u : 2048u;
-    if (nmat == 1u && rows[0] <= 2048u && cols * batch <= small) return hipErrorNotSupported;
+    // One vector, or few rows, are done sooner by the general kernel's one launch
+    // (this path's two launches take 5 us at the least). Graph replays, matrix
+    // cores / general: one vector 4096 x 11008 Q8_0 17.7 / 15.0 us, F16 24.7 /
+    // 20.3; four, 2048 x 4096 Q8_0 9.3 / 7.5, 2048 x 11008 15.8 / 16.8, 4096 x
+    // 4096 10.0 / 15.8; eight, 512 x 11008 16.4 / 10.5, 1024 x 4096 9.4 / 8.5,
+    // 1024 x 11008 16.7 / 19.5, 2048 x 4096 9.8 / 11.1; sixteen, 512 x 4096 11.3 /
+    // 9.1, 1024 x 4096 11.3 / 12.5.
+    if (nmat == 1u && (batch == 1u || rows[0] <= (batch <= 4u ? 2048u : 512u) ||
+                       (batch <= 8u && rows[0] <= 1024u && cols <= 4096u)))
+        return hipErrorNotSupported;
     const uint32_t pcols = (cols + 255u) & ~255u;
     hipError_t why;
     uint8_t *xp = static_cast<uint8_t *>(rt_scratch((size_t)((batch + kBatchMax - 1u) / kBatchMax) * xb_layout(pcols).bytes, s, &why));
