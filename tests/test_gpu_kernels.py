@@ -680,6 +680,34 @@ def test_attention_random_shapes(dev, host, oracle, mem, nqh, nkh, hd, seq, max_
     assert np.all(np.abs(got - want) <= 1e-4 + 1e-4 * np.abs(want))
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("nqh,nkh", [(1, 1), (6, 2), (8, 1), (35, 5)])
+@pytest.mark.parametrize("seq", [31, 33, 128, 129, 256, 257, 4500])
+def test_attention_chunk_limits(dev, host, oracle, mem, hd, nqh, nkh, seq):
+    """The matrix-core kernel's head sizes on both sides of the one-launch
+    limits (128 positions at head_dim 96 and 128, 256 at 32 and 64), of a tile,
+    and past 128 chunks (4500 positions of one kv head), with groups that
+    leave heads of the eight idle; scores of up to ~170 in the first q head
+    (there a score's rounding to f32, 1e-5 in both, moves a weight by 1e-5 of
+    itself, a tenth of the bar), and of ~1e9 in a second call, where the
+    result must still be a mean of the values."""
+    max_ctx, layer = seq + 5, 1
+    kvd = nkh * hd
+    kc = V.synth_normal_f16(host, 2 * max_ctx * kvd, SEED, 151)
+    vc = V.synth_normal_f16(host, 2 * max_ctx * kvd, SEED, 152)
+    q = synth_x(host, nqh * hd, 153)
+    q[:hd] *= 30.0
+    scale = np.float32(1.0 / math.sqrt(hd))
+    pq, pkc, pvc, po = mem.up(q), mem.up(kc), mem.up(vc), mem.zeros(nqh * hd)
+    dev.attention(pq, pkc, pvc, po, seq, layer, max_ctx, nqh, nkh, hd, scale)
+    got = dev.download(po, nqh * hd, np.float32)
+    want = oracle.attention(q, kc, vc, seq, layer, max_ctx, nqh, nkh, hd, scale)
+    assert np.all(np.abs(got - want) <= 1e-4 + 1e-4 * np.abs(want))
+    dev.attention(mem.up(q * np.float32(1e8)), pkc, pvc, po, seq, layer, max_ctx, nqh, nkh, hd, scale)
+    got = dev.download(po, nqh * hd, np.float32)
+    assert np.max(np.abs(got)) <= 1.001 * np.max(np.abs(vc.view(np.float16).astype(np.float32)))
+
+
 @pytest.mark.parametrize("qscale", [1e-6, 1e4])
 def test_attention_q_magnitude(dev, host, oracle, mem, qscale):
     """q far from unit scale (the matrix-core kernel rescales each head's q

@@ -1,9 +1,9 @@
 // vbs_attn_common.h — the sequence split of split-sequence attention and the
-// head_dim-128 merge of its partial results (vbs_kern_attn.hip).
+// merge of its partial results (vbs_kern_attn.hip).
 //
-// Partials: for q head h and chunk c, at part + (h * stride + c) * 130
-// floats: m (the chunk's maximum score), l (sum of e^(s - m)) and acc[128]
-// (sum of e^(s - m) v). Reference: the online softmax of vbs_host_attention
+// Partials: for q head h and chunk c, at part + (h * stride + c) * (HD + 2)
+// floats: m (the chunk's maximum score; merge_exp), l (sum of e^(s - m)) and
+// acc[HD] (sum of e^(s - m) v). Reference: the online softmax of vbs_host_attention
 // (src/vbs_host_math.h:170-209), merged by log-sum-exp rescaling:
 // out = sum_c acc_c e^(m_c - M) / sum_c l_c e^(m_c - M), M = max_c m_c.
 #pragma once
@@ -55,14 +55,25 @@ __device__ __forceinline__ float fast_exp(float x) {
     return __builtin_amdgcn_exp2f(x * 1.44269504088896341f);
 }
 
-// ---- head_dim-128 merge, one wave's pieces ------------------------------------------
-// The merge of q head h (partials ph = part + h * stride * 130, nc chunks)
-// is M and L, then four interleaved sums, residue r taking chunks r, r + 4,
-// ... in order with lane l holding head dims 2l and 2l + 1, then
-// out = ((a_0 + a_1) + a_2 + a_3) / L. The four-wave merge kernel gives wave
-// r residue r.
+// 2^x, the same way.
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+// The weight of a partial whose m lies x below the largest: head_dim 128 keeps
+// m as the score, the other sizes as a whole power of two (m times log2 e).
+template <uint32_t HD>
+__device__ __forceinline__ float merge_exp(float x) {
+    return HD == 128u ? fast_exp(x) : exp2_fast(x);
+}
+
+// ---- the merge, one wave's pieces --------------------------------------------------
+// The merge of q head h (partials ph = part + h * stride * (HD + 2), nc chunks;
+// HD up to 128) is M and L, then four interleaved sums, residue r taking
+// chunks r, r + 4, ... in order with lane l < HD / 2 holding head dims 2l and
+// 2l + 1, then out = ((a_0 + a_1) + a_2 + a_3) / L. The four-wave merge kernel
+// gives wave r residue r.
 constexpr uint32_t kMergeRes = 4, kMergeBatch = 32;  // residues; chunks of one held in registers
-constexpr uint32_t kPartRow = 130;                   // m, l, acc[128]
+template <uint32_t HD>
+constexpr uint32_t part_row = HD + 2u;               // m, l, acc[HD]
+constexpr uint32_t kPartRow = part_row<128>;
 
 struct MergeStats {
     float M, L;
@@ -73,12 +84,13 @@ struct MergeStats {
 struct MergeMl {
     float m0, l0, m1, l1;
 };
+template <uint32_t HD = 128>
 __device__ __forceinline__ MergeMl merge_ml_load(const float *ph, uint32_t nc, uint32_t lane) {
     MergeMl v;
-    v.m0 = lane < nc ? ph[(uint64_t)lane * kPartRow] : -INFINITY;
-    v.l0 = lane < nc ? ph[(uint64_t)lane * kPartRow + 1u] : 0.f;
-    v.m1 = lane + 64u < nc ? ph[(uint64_t)(lane + 64u) * kPartRow] : -INFINITY;
-    v.l1 = lane + 64u < nc ? ph[(uint64_t)(lane + 64u) * kPartRow + 1u] : 0.f;
+    v.m0 = lane < nc ? ph[(uint64_t)lane * part_row<HD>] : -INFINITY;
+    v.l0 = lane < nc ? ph[(uint64_t)lane * part_row<HD> + 1u] : 0.f;
+    v.m1 = lane + 64u < nc ? ph[(uint64_t)(lane + 64u) * part_row<HD>] : -INFINITY;
+    v.l1 = lane + 64u < nc ? ph[(uint64_t)(lane + 64u) * part_row<HD> + 1u] : 0.f;
     return v;
 }
 // The same loads bounded by `bound` >= nc chunk rows (all inside the
@@ -100,21 +112,22 @@ __device__ __forceinline__ MergeMl merge_ml_mask(MergeMl v, uint32_t nc, uint32_
 
 // Every lane of the wave gets M and L: lane l takes chunks l, l + 64, ... in
 // that order (chunks from 128 on are read here).
+template <uint32_t HD = 128>
 __device__ __forceinline__ MergeStats merge_stats(const float *ph, uint32_t nc, uint32_t lane,
                                                   const MergeMl &v) {
     MergeStats st;
     float M = fmaxf(v.m0, v.m1);
-    for (uint32_t c = lane + 128u; c < nc; c += 64u) M = fmaxf(M, ph[(uint64_t)c * kPartRow]);
+    for (uint32_t c = lane + 128u; c < nc; c += 64u) M = fmaxf(M, ph[(uint64_t)c * part_row<HD>]);
     st.M = wave_max(M);
-    const float w0 = v.m0 == -INFINITY ? 0.f : fast_exp(__fsub_rn(v.m0, st.M));
-    const float w1 = v.m1 == -INFINITY ? 0.f : fast_exp(__fsub_rn(v.m1, st.M));
+    const float w0 = v.m0 == -INFINITY ? 0.f : merge_exp<HD>(__fsub_rn(v.m0, st.M));
+    const float w1 = v.m1 == -INFINITY ? 0.f : merge_exp<HD>(__fsub_rn(v.m1, st.M));
     float L = 0.f;
     if (lane < nc) L = fmaf(v.l0, w0, L);
     if (lane + 64u < nc) L = fmaf(v.l1, w1, L);
     for (uint32_t c = lane + 128u; c < nc; c += 64u) {
-        const float mc = ph[(uint64_t)c * kPartRow];
-        const float wc = mc == -INFINITY ? 0.f : fast_exp(__fsub_rn(mc, st.M));
-        L = fmaf(ph[(uint64_t)c * kPartRow + 1u], wc, L);
+        const float mc = ph[(uint64_t)c * part_row<HD>];
+        const float wc = mc == -INFINITY ? 0.f : merge_exp<HD>(__fsub_rn(mc, st.M));
+        L = fmaf(ph[(uint64_t)c * part_row<HD> + 1u], wc, L);
     }
     st.L = wave_sum(L);
     st.w_lane = lane < nc ? w0 : 0.f;
@@ -125,30 +138,31 @@ __device__ __forceinline__ MergeStats merge_stats(const float *ph, uint32_t nc, 
 // Residue r: the acc rows of chunks c = r + 4 k, k < kMergeBatch, requested
 // at once (lane l: head dims 2l, 2l + 1; rows from nc on, when nc is a bound
 // on the chunk count rather than the count, are read and not used) ...
+template <uint32_t HD = 128>
 __device__ __forceinline__ void merge_residue_load(const float *ph, uint32_t nc, uint32_t r,
                                                    uint32_t lane, float2 av[kMergeBatch]) {
 #pragma unroll
     for (uint32_t k = 0; k < kMergeBatch; k++) {
         const uint32_t c = r + kMergeRes * k;
-        av[k] = c < nc ? *reinterpret_cast<const float2 *>(ph + (uint64_t)c * kPartRow + 2u + 2u * lane)
+        av[k] = c < nc && (HD == 128u || lane < HD / 2u) ? *reinterpret_cast<const float2 *>(ph + (uint64_t)c * part_row<HD> + 2u + 2u * lane)
                        : make_float2(0.f, 0.f);
     }
 }
 // ... and their sum weighted by e^(m_c - M), accumulated in chunk order (later
 // chunks of the residue read here).
+template <uint32_t HD = 128>
 __device__ __forceinline__ float2 merge_residue_sum(const float *ph, uint32_t nc, const MergeStats &st,
                                                    uint32_t r, uint32_t lane,
                                                    const float2 av[kMergeBatch]) {
     float ox = 0.f, oy = 0.f;
-    auto add = [&](uint32_t c, float2 a) {
+    auto add = [&](uint32_t c, float2 a, float mc) {  // (mc, the chunk's m, from chunk 128 on)
         float wc;
         if (c < 128u) {  // (a lane's weight: c is wave-uniform)
             wc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(
                                                __builtin_bit_cast(int, c < 64u ? st.w_lane : st.w_lane64),
                                                (int)(c & 63u)));
         } else {
-            const float mc = ph[(uint64_t)c * kPartRow];
-            wc = mc == -INFINITY ? 0.f : fast_exp(__fsub_rn(mc, st.M));
+            wc = mc == -INFINITY ? 0.f : merge_exp<HD>(__fsub_rn(mc, st.M));
         }
         ox = fmaf(a.x, wc, ox);
         oy = fmaf(a.y, wc, oy);
@@ -156,10 +170,23 @@ __device__ __forceinline__ float2 merge_residue_sum(const float *ph, uint32_t nc
 #pragma unroll
     for (uint32_t k = 0; k < kMergeBatch; k++) {
         const uint32_t c = r + kMergeRes * k;
-        if (c < nc) add(c, av[k]);
+        if (c < nc) add(c, av[k], 0.f);
     }
-    for (uint32_t c = r + kMergeRes * kMergeBatch; c < nc; c += kMergeRes)
-        add(c, *reinterpret_cast<const float2 *>(ph + (uint64_t)c * kPartRow + 2u + 2u * lane));
+    if (HD == 128u || lane < HD / 2u) {  // (sixteen rows requested at a time)
+        for (uint32_t c0 = r + kMergeRes * kMergeBatch; c0 < nc; c0 += 16u * kMergeRes) {
+            float2 tv[16];
+            float tm[16];
+#pragma unroll
+            for (uint32_t k = 0; k < 16u; k++) {
+                const float *row = ph + (uint64_t)min(c0 + kMergeRes * k, nc - 1u) * part_row<HD>;
+                tv[k] = *reinterpret_cast<const float2 *>(row + 2u + 2u * lane);
+                tm[k] = row[0];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 16u; k++)
+                if (c0 + kMergeRes * k < nc) add(c0 + kMergeRes * k, tv[k], tm[k]);
+        }
+    }
     return make_float2(ox, oy);
 }
 
@@ -179,20 +206,20 @@ __device__ __forceinline__ float2 merge_finish(const float2 a[kMergeRes], float 
 // in chunk order (each residue's chunks in its own order, as the four waves
 // take them), the acc rows of B chunks requested at once (B a multiple of
 // kMergeRes), then merge_finish: bit-identical to the four-wave merge.
-template <uint32_t B>
+template <uint32_t B, uint32_t HD = 128>
 __device__ __forceinline__ float2 merge_one_wave(const float *ph, uint32_t nc, uint32_t lane) {
     static_assert(B % kMergeRes == 0u, "batch");
     auto load_batch = [&](uint32_t c0, float2 av[B]) {
 #pragma unroll
         for (uint32_t k = 0; k < B; k++) {
             const uint32_t c = c0 + k;
-            av[k] = c < nc ? *reinterpret_cast<const float2 *>(ph + (uint64_t)c * kPartRow + 2u + 2u * lane)
+            av[k] = c < nc && (HD == 128u || lane < HD / 2u) ? *reinterpret_cast<const float2 *>(ph + (uint64_t)c * part_row<HD> + 2u + 2u * lane)
                            : make_float2(0.f, 0.f);
         }
     };
     float2 av[B];
     load_batch(0u, av);
-    const MergeStats st = merge_stats(ph, nc, lane, merge_ml_load(ph, nc, lane));
+    const MergeStats st = merge_stats<HD>(ph, nc, lane, merge_ml_load<HD>(ph, nc, lane));
     float ox[kMergeRes] = {0.f, 0.f, 0.f, 0.f}, oy[kMergeRes] = {0.f, 0.f, 0.f, 0.f};
     for (uint32_t c0 = 0; c0 < nc; c0 += B) {
         if (c0) load_batch(c0, av);
@@ -206,8 +233,8 @@ __device__ __forceinline__ float2 merge_one_wave(const float *ph, uint32_t nc, u
                                                        __builtin_bit_cast(int, c < 64u ? st.w_lane : st.w_lane64),
                                                        (int)(c & 63u)));
                 } else {
-                    const float mc = ph[(uint64_t)c * kPartRow];
-                    wc = mc == -INFINITY ? 0.f : fast_exp(__fsub_rn(mc, st.M));
+                    const float mc = ph[(uint64_t)c * part_row<HD>];
+                    wc = mc == -INFINITY ? 0.f : merge_exp<HD>(__fsub_rn(mc, st.M));
                 }
                 ox[r] = fmaf(av[k].x, wc, ox[r]);
                 oy[r] = fmaf(av[k].y, wc, oy[r]);

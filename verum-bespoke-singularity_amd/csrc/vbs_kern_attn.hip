@@ -10,28 +10,16 @@
 // and acc[d] = sum exp(score - m) * v[d]; the chunks are merged with
 // log-sum-exp rescaling: out = sum_c acc_c * e^(m_c-M) / sum_c l_c * e^(m_c-M).
 // The chunk length follows the sequence (attn_split) so that about
-// kTargetWgs (512) workgroups of the vector-ALU kernels, or kMfmaTargetWgs
-// (vbs_attn_common.h) of the matrix-core kernel, share it at any length. A second kernel merges (a hand-off
-// inside one kernel, through device-scope stores, loads and an arrival
-// count, measured slower than the kernel boundary on this part).
+// kMfmaTargetWgs (vbs_attn_common.h) workgroups of the matrix-core kernel, or
+// kTargetWgs of the generic one, share it at any length. A second kernel
+// merges (a hand-off inside one kernel, through device-scope stores, loads and
+// an arrival count, measured slower than the kernel boundary on this part);
+// short sequences take one launch that does both, the chunks of a kv head
+// on the waves of one workgroup (k_attn_one).
 //
-// Fast chunk kernel (head_dim 32/64/128, group <= 8): four waves; lanes of a
-// wave split a position's head_dim into 8-element slices (16-byte K and V
-// loads), so one wave step covers 64/(head_dim/8) positions ("slots"). A wave
-// loads four steps at a time (up to four such batches; the next batch's K
-// rows are requested once the scores are taken, its V rows once they are
-// used). q lives in registers (the lane's slice for every q head of the
-// group); the partial dot of a slice is an fp32 FMA chain and the slices are
-// added with DPP row operations, which leaves every lane of a slot with its
-// scores. Each slot keeps a running softmax state (max, sum, acc) over its
-// positions; the slots of a wave are combined with lane shuffles and the four
-// waves in one LDS pass. Scores are fp32 dots of exactly converted f16
-// keys instead of the reference's double dot: a relative difference of order
-// 1e-7 in each score, far inside the 1e-4 the reference's own backend test
-// allows (src/vbs_backend_test.c:617-625).
-//
-// Other shapes use the generic chunk kernel (double dot, one position per
-// four threads).
+// head_dim 32, 64, 96 and 128 with at most eight q heads per kv head take the
+// matrix-core chunk kernel; other shapes the generic one (double dot, one
+// position per four threads).
 #include "vbs_attn_common.h"
 #include "vbs_dev_common.h"
 #include "vbs_internal.h"
@@ -40,9 +28,9 @@ namespace vbs {
 
 constexpr uint32_t kChunk = 64;  // positions per workgroup of the generic kernel
 constexpr uint32_t kMaxGroup = 16;
-constexpr uint32_t kTargetWgs = 512;      // workgroups the vector-ALU split aims for
+constexpr uint32_t kTargetWgs = 512;      // workgroups the generic kernel's split aims for
 
-// (attn_split, the matrix-core split's constants and fast_exp: vbs_attn_common.h)
+// (attn_split, the matrix-core split's constants and the exponentials: vbs_attn_common.h)
 // Chunks per kv head of any split of a sequence of at most max_seq (every
 // len >= 64 or len >= seq * nkh / target, target <= kMfmaTargetWgs).
 inline uint32_t attn_max_chunks(uint32_t max_seq, uint32_t nkh) {
@@ -150,217 +138,7 @@ __global__ __launch_bounds__(256) void k_attn_partial(const float *__restrict__ 
 }
 
 
-// ---- fast chunk kernel ---------------------------------------------------------
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                                                     CTRL, 0xF, 0xF, false));
-}
-
-// Sum over each aligned group of L lanes (L = 4, 8, 16); every lane of the
-// group receives the sum.
-template <uint32_t L>
-__device__ __forceinline__ float group_sum(float v) {
-    v = dpp_add<0xB1>(v);                        // quad_perm [1,0,3,2]
-    v = dpp_add<0x4E>(v);                        // quad_perm [2,3,0,1]
-    if constexpr (L >= 8) v = dpp_add<0x141>(v);  // row_half_mirror
-    if constexpr (L >= 16) v = dpp_add<0x140>(v); // row_mirror
-    return v;
-}
-
-
-// Shape of the fast kernel: four waves; LPP lanes per position (8 head dims
-// each), so a wave step covers PPW positions ("slots"); a wave loads kSteps
-// steps at a time and runs up to kBatches such batches.
-constexpr uint32_t kWaves = 4, kSteps = 4, kBatches = 4;
-template <uint32_t HD>
-struct ChunkShape {
-    static constexpr uint32_t LPP = HD / 8, PPW = 64 / LPP, GRAN = kWaves * PPW,
-                              LMAX = kBatches * kSteps * GRAN;
-};
-
-template <uint32_t HD, uint32_t GMAX>
-__global__ __launch_bounds__(64 * kWaves) void k_attn_chunk(
-    const float *__restrict__ q, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,
-    float *__restrict__ part, uint32_t seq_len, const uint32_t *__restrict__ pos_dev,
-    uint64_t layer_off, uint32_t nkh, uint32_t group, float scale, uint32_t stride_chunks) {
-    using S = ChunkShape<HD>;
-    constexpr uint32_t LPP = S::LPP, PPW = S::PPW;
-    extern __shared__ __align__(16) uint8_t chunk_lds[];
-    float *red = reinterpret_cast<float *>(chunk_lds);  // [kWaves][group][HD] acc per wave
-    __shared__ float sm[kWaves][GMAX], sl[kWaves][GMAX], sf[kWaves][GMAX];
-
-    const uint32_t chunk = blockIdx.x, kvh = blockIdx.y, t = threadIdx.x;
-    const uint32_t wave = t >> 6, lane = t & 63u;
-    const uint32_t slot = lane / LPP, c = lane % LPP;
-    if (pos_dev) seq_len = pos_dev[0] + 1u;  // graph replay: the device holds the position
-    const AttnSplit sp = attn_split(seq_len, nkh, S::GRAN, S::LMAX, kTargetWgs);
-    if (chunk >= sp.n) return;  // past the sequence (the grid covers the longest split)
-    const uint32_t s0 = chunk * sp.len;
-    const uint32_t valid = min(sp.len, seq_len - s0);
-    const uint32_t pw = sp.len / kWaves, ns = pw / PPW;  // positions and steps per wave
-    const uint32_t nb = (ns + kSteps - 1u) / kSteps;     // batches of kSteps steps
-    const uint64_t rstride = (uint64_t)nkh * HD;
-    const uint64_t base = layer_off + (uint64_t)s0 * rstride + (uint64_t)kvh * HD + 8u * c;
-
-    // position of step i of this lane's slot; positions past the chunk re-read
-    // its last row and are masked (score -inf, v zero)
-    auto pos_of = [&](uint32_t i) { return wave * pw + i * PPW + slot; };
-    uint4 kr[kSteps], vr[kSteps];
-    auto load_k = [&](uint32_t bi) {
-#pragma unroll
-        for (uint32_t b = 0; b < kSteps; b++)
-            if (bi * kSteps + b < ns)
-                kr[b] = *reinterpret_cast<const uint4 *>(
-                    kc + base + (uint64_t)min(pos_of(bi * kSteps + b), valid - 1u) * rstride);
-    };
-    auto load_v = [&](uint32_t bi) {
-#pragma unroll
-        for (uint32_t b = 0; b < kSteps; b++) {
-            const uint32_t i = bi * kSteps + b;
-            if (i < ns) {
-                vr[b] = *reinterpret_cast<const uint4 *>(
-                    vc + base + (uint64_t)min(pos_of(i), valid - 1u) * rstride);
-                if (pos_of(i) >= valid) vr[b] = make_uint4(0u, 0u, 0u, 0u);
-            }
-        }
-    };
-    load_k(0);
-    load_v(0);
-    float qv[GMAX][8];
-#pragma unroll
-    for (uint32_t g = 0; g < GMAX; g++) {
-        const uint32_t gg = g < group ? g : 0u;
-        const float4 *qp =
-            reinterpret_cast<const float4 *>(q + ((uint64_t)kvh * group + gg) * HD + 8u * c);
-        const float4 a = qp[0], b4 = qp[1];
-        qv[g][0] = a.x; qv[g][1] = a.y; qv[g][2] = a.z; qv[g][3] = a.w;
-        qv[g][4] = b4.x; qv[g][5] = b4.y; qv[g][6] = b4.z; qv[g][7] = b4.w;
-    }
-
-    // per slot and q head: running max m, sum l of e^(s - m), acc of e^(s - m) v
-    float m[GMAX], l[GMAX], acc[GMAX][8];
-#pragma unroll
-    for (uint32_t g = 0; g < GMAX; g++) {
-        m[g] = -INFINITY;
-        l[g] = 0.f;
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) acc[g][j] = 0.f;
-    }
-    for (uint32_t bi = 0; bi < nb; bi++) {
-        // scores: every lane of a slot holds its position's scores
-        float sc[kSteps][GMAX];
-#pragma unroll
-        for (uint32_t b = 0; b < kSteps; b++) {
-            const uint32_t i = bi * kSteps + b;
-            const bool in = i < ns && pos_of(i) < valid;
-            float kf[8];
-            if (i < ns) {
-                const uint32_t kw[4] = {kr[b].x, kr[b].y, kr[b].z, kr[b].w};
-#pragma unroll
-                for (uint32_t j = 0; j < 8; j++) kf[j] = hcvt(kw[j >> 1] >> (16u * (j & 1u)));
-            }
-#pragma unroll
-            for (uint32_t g = 0; g < GMAX; g++) {
-                float p = 0.f;
-                if (i < ns) {
-#pragma unroll
-                    for (uint32_t j = 0; j < 8; j++) p = fmaf(qv[g][j], kf[j], p);
-                    p = group_sum<LPP>(p);
-                }
-                sc[b][g] = in ? __fmul_rn(p, scale) : -INFINITY;
-            }
-        }
-        if (bi + 1u < nb) load_k(bi + 1u);  // the K registers are free again
-#pragma unroll
-        for (uint32_t g = 0; g < GMAX; g++) {
-            float mb = sc[0][g];
-#pragma unroll
-            for (uint32_t b = 1; b < kSteps; b++) mb = fmaxf(mb, sc[b][g]);
-            const float mn = fmaxf(m[g], mb);
-            const float r = m[g] == -INFINITY ? 0.f : fast_exp(__fsub_rn(m[g], mn));
-            l[g] *= r;
-#pragma unroll
-            for (uint32_t j = 0; j < 8; j++) acc[g][j] *= r;
-#pragma unroll
-            for (uint32_t b = 0; b < kSteps; b++) {
-                if (bi * kSteps + b < ns) {
-                    const float e = sc[b][g] == -INFINITY ? 0.f : fast_exp(__fsub_rn(sc[b][g], mn));
-                    const uint32_t vw[4] = {vr[b].x, vr[b].y, vr[b].z, vr[b].w};
-                    l[g] += e;
-#pragma unroll
-                    for (uint32_t j = 0; j < 8; j++)
-                        acc[g][j] = fmaf(e, hcvt(vw[j >> 1] >> (16u * (j & 1u))), acc[g][j]);
-                }
-            }
-            m[g] = mn;
-        }
-        if (bi + 1u < nb) load_v(bi + 1u);
-    }
-
-    // ---- the wave's slots combined (lanes of equal c across slots): M = max m,
-    // weights e^(m - M) (0 for an empty slot), then sums; every slot ends with
-    // the totals and slot 0 stores them
-#pragma unroll
-    for (uint32_t g = 0; g < GMAX; g++) {
-        float M = m[g];
-#pragma unroll
-        for (uint32_t off = LPP; off < 64u; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-        const float f = m[g] == -INFINITY ? 0.f : fast_exp(__fsub_rn(m[g], M));
-        float L = l[g] * f, a[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) a[j] = acc[g][j] * f;
-#pragma unroll
-        for (uint32_t off = LPP; off < 64u; off <<= 1) {
-            L += __shfl_xor(L, off, 64);
-#pragma unroll
-            for (uint32_t j = 0; j < 8; j++) a[j] += __shfl_xor(a[j], off, 64);
-        }
-        if (g < group && slot == 0) {
-            float *dst = red + ((wave * group + g) * HD + 8u * c);
-            reinterpret_cast<float4 *>(dst)[0] = make_float4(a[0], a[1], a[2], a[3]);
-            reinterpret_cast<float4 *>(dst)[1] = make_float4(a[4], a[5], a[6], a[7]);
-            if (c == 0) {
-                sm[wave][g] = M;
-                sl[wave][g] = L;
-            }
-        }
-    }
-    __syncthreads();
-
-    // ---- combine the waves: M = max m_w, weights e^(m_w - M) (0 for empty waves)
-    if (t < kWaves * GMAX) {
-        const uint32_t w = t / GMAX, g = t % GMAX;
-        if (g < group) {
-            float M = sm[0][g];
-#pragma unroll
-            for (uint32_t i = 1; i < kWaves; i++) M = fmaxf(M, sm[i][g]);
-            const float mw = sm[w][g];
-            sf[w][g] = mw == -INFINITY ? 0.f : fast_exp(__fsub_rn(mw, M));
-        }
-    }
-    __syncthreads();
-    float *const pk = part + (uint64_t)kvh * group * stride_chunks * (HD + 2u);
-    for (uint32_t i = t; i < group * HD; i += 64u * kWaves) {
-        const uint32_t g = i / HD, d = i % HD;
-        float a = 0.f;
-#pragma unroll
-        for (uint32_t w = 0; w < kWaves; w++) a = fmaf(red[(w * group + g) * HD + d], sf[w][g], a);
-        float *dst = pk + ((uint64_t)g * stride_chunks + chunk) * (HD + 2u);
-        dst[2u + d] = a;
-        if (d == 0) {
-            float M = sm[0][g], L = 0.f;
-#pragma unroll
-            for (uint32_t w = 1; w < kWaves; w++) M = fmaxf(M, sm[w][g]);
-#pragma unroll
-            for (uint32_t w = 0; w < kWaves; w++) L = fmaf(sl[w][g], sf[w][g], L);
-            dst[0] = M;
-            dst[1] = L;
-        }
-    }
-}
-
-// ---- matrix-core chunk kernel (head_dim 128, group <= 8) ------------------------
+// ---- matrix-core chunk kernel (head_dim 32, 64, 96, 128; group <= 8) -------------
 // One wave per chunk of up to kMfmaTiles tiles of 32 positions, on
 // v_mfma_f32_16x16x32_f16:
 // * scores, S = K q^T: A = 16 positions x 32 head dims of K (the cache's f16,
@@ -374,11 +152,16 @@ __global__ __launch_bounds__(64 * kWaves) void k_attn_chunk(
 // * online softmax per head over the tiles (running max m, sum l).
 // * P V: A = P, rows n: e^(s - m) of head n & 7 (f16 hi for n < 8, lo for
 //   n >= 8), k slots = exactly the lane's own eight positions; B = V with the
-//   same k slots and column n of dim tile t standing for head dim 8 n + t, so
-//   lane (n, g) takes its B operands from eight 16-byte V rows it loaded
-//   itself (dims 8n..8n+7 of its eight positions) and no transpose is needed.
+//   same k slots and column n of dim tile t standing for head dim D n + t (D =
+//   HD / 16), so lane (n, g) takes its B operands from eight V rows it loaded
+//   itself (dims Dn..Dn+D-1 of its eight positions) and no transpose is needed.
 //   D rows 0-7 (hi) and 8-15 (lo) add up at the end.
-// The chunk's (m, l, acc) go to the same partials as the vector-ALU kernel.
+// Bound: latency (one or a few tiles per wave) up to HBM at long contexts.
+// Measured (chunk + merge) against the vector-ALU kernel that took head_dim 32
+// and 64 before and the generic one that took 96: 32 q heads over 8 kv heads,
+// 3001 positions, head_dim 32 14.1 -> 8.1 us, 64 13.5 -> 9.0, 96 44.3 -> 10.4; 41
+// positions 9.2 -> 3.5, 8.8 -> 3.9, 28.4 -> 4.4 (one launch). Head_dim 128 over one
+// kv head, 16000 positions 37.4 -> 21.1 (the merge's later rows sixteen at a time).
 // The most chunks the matrix-core split gives any sequence of at most max_seq
 // positions: the chunk count grows with the sequence while the chunk length
 // stays put, so the maximum lies at the longest sequence of some chunk length
@@ -406,48 +189,57 @@ typedef uint32_t au4 __attribute__((ext_vector_type(4)));
 // One wave's chunk: positions [s0, s0 + valid) of kv head kvh (valid >= 1,
 // nt tiles of 32) against the q heads of its group. On return every lane
 // holds, for head n & 7 of its lane n = lane & 15, the chunk maximum m and
-// l = sum e^(s - m); and a[dt][r] = the sum of e^(s - m) v[8 n + dt] of head
+// l = sum e^(s - m); and a[dt][r] = the sum of e^(s - m) v[HD / 16 n + dt] of head
 // 4 (lane >> 4) + r (rows hi + lo added; lane groups 0 and 1 carry them).
+template <uint32_t HD>
 __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
                                                const uint16_t *__restrict__ kc,
                                                const uint16_t *__restrict__ vc, uint64_t layer_off,
                                                uint32_t s0, uint32_t valid, uint32_t nt,
                                                uint32_t nkh, uint32_t kvh, uint32_t group,
                                                float scale, uint32_t lane, float &m_out,
-                                               float &l_out, float (&a)[8][4]) {
-    constexpr uint32_t HD = 128;
+                                               float &l_out, float (&a)[HD / 16][4]) {
+    constexpr uint32_t KK = HD / 32u, DPL = HD / 16u, VW = DPL / 2u;  // K slices; V dims and words per lane
+    constexpr bool FINE = HD != 128u;
+    constexpr float PS = FINE ? 16384.f : 1.f;  // P's scale (f16 would drop lo bits of small weights)
     const uint32_t n = lane & 15u, g = lane >> 4;
     const uint64_t rstride = (uint64_t)nkh * HD;
     const uint64_t base = layer_off + (uint64_t)s0 * rstride + (uint64_t)kvh * HD;
 
     // ---- tile loads: K rows (A operand: position 16 hf + n, dims 32 kk + 8 g ..),
-    // V rows (position p_j of this lane group, dims 8 n ..); positions past the
+    // V rows (position p_j of this lane group, dims DPL n ..); positions past the
     // chunk re-read its last row and are masked
     auto pos_of = [&](uint32_t t, uint32_t j) { return 32u * t + 16u * (j >> 2) + 4u * g + (j & 3u); };
-    au4 kr[2][4], vr[8];
+    au4 kr[2][KK];
+    uint32_t vr[8][VW];
     auto load_k = [&](uint32_t t) {
 #pragma unroll
         for (uint32_t hf = 0; hf < 2; hf++) {
             const uint32_t p = min(32u * t + 16u * hf + n, valid - 1u);
 #pragma unroll
-            for (uint32_t kk = 0; kk < 4; kk++)
+            for (uint32_t kk = 0; kk < KK; kk++)
                 kr[hf][kk] = *reinterpret_cast<const au4 *>(kc + base + (uint64_t)p * rstride +
                                                             32u * kk + 8u * g);
         }
     };
     auto load_v = [&](uint32_t t) {
 #pragma unroll
-        for (uint32_t j = 0; j < 8; j++)
-            vr[j] = *reinterpret_cast<const au4 *>(
-                vc + base + (uint64_t)min(pos_of(t, j), valid - 1u) * rstride + 8u * n);
+        for (uint32_t j = 0; j < 8; j++) {
+            const uint16_t *p = vc + base + (uint64_t)min(pos_of(t, j), valid - 1u) * rstride + DPL * n;
+            typedef uint32_t vw __attribute__((ext_vector_type(VW == 3u ? 2u : VW), aligned(4)));
+            const vw w = *reinterpret_cast<const vw *>(p);
+#pragma unroll
+            for (uint32_t i = 0; i < (VW == 3u ? 2u : VW); i++) vr[j][i] = w[i];
+            if (VW == 3u) vr[j][VW - 1u] = reinterpret_cast<const uint32_t *>(p)[VW - 1u];
+        }
     };
     // ---- q' of head n & 7 (heads past the group repeat head 0 and are not stored)
     const uint32_t h = n & 7u, hq = h < group ? h : 0u;
-    float qv[4][8];
+    float qv[KK][8];
     {
         const float4 *qp = reinterpret_cast<const float4 *>(q + ((uint64_t)kvh * group + hq) * HD);
 #pragma unroll
-        for (uint32_t kk = 0; kk < 4; kk++) {
+        for (uint32_t kk = 0; kk < KK; kk++) {
             const float4 a = qp[(32u * kk + 8u * g) / 4u], b = qp[(32u * kk + 8u * g) / 4u + 1u];
             qv[kk][0] = a.x; qv[kk][1] = a.y; qv[kk][2] = a.z; qv[kk][3] = a.w;
             qv[kk][4] = b.x; qv[kk][5] = b.y; qv[kk][6] = b.z; qv[kk][7] = b.w;
@@ -461,7 +253,7 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
     __builtin_amdgcn_sched_barrier(0);
     float amax = 0.f;
 #pragma unroll
-    for (uint32_t kk = 0; kk < 4; kk++)
+    for (uint32_t kk = 0; kk < KK; kk++)
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(qv[kk][j]));
     amax = fmaxf(amax, lane_xor<16>(amax));
@@ -470,9 +262,18 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
     (void)frexpf(amax, &e2);  // amax < 2^e2
     const int sq = amax > 0.f ? 15 - e2 : 0;
     const float csc = ldexpf(scale, -sq);
-    ah8 Qb[4];
+    // FINE (head sizes whose scores were double dots, or sums of eight dims per
+    // lane, before this kernel took them): each dot is a double sum of one
+    // product per 16 dims, and the scores are kept times log2 e, s2 = c (dot)
+    // with c in two parts, the maximum rounded up to a whole number so that
+    // no bits of s2 are lost against it. Error against 64 bits, 32 q heads over 8
+    // kv heads, 300 and 3001 positions: head_dim 64 1.4e-7 and 1.8e-7 (1.5 and 1.8
+    // without; 2.1 and 1.9 before), 96 1.6 and 1.9 (2.2 and 2.3; 1.6 and 2.0).
+    const float c2 = FINE ? csc * 1.44269504088896341f : csc;
+    const float c2lo = fmaf(csc, 1.44269504088896341f, -c2) + csc * 1.92596299e-8f;
+    ah8 Qb[KK];
 #pragma unroll
-    for (uint32_t kk = 0; kk < 4; kk++)
+    for (uint32_t kk = 0; kk < KK; kk++)
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++) {
             const float x = ldexpf(qv[kk][j], sq);
@@ -482,52 +283,88 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
 
 
     float m = -INFINITY, l = 0.f;
-    af4 acc[8];
+    af4 acc[DPL];
 #pragma unroll
-    for (uint32_t t = 0; t < 8; t++) acc[t] = af4{0.f, 0.f, 0.f, 0.f};
+    for (uint32_t t = 0; t < DPL; t++) acc[t] = af4{0.f, 0.f, 0.f, 0.f};
     auto tile = [&](uint32_t t) {
-        af4 S[2];
+        af4 S[2][FINE ? 2u * KK : 1u];
 #pragma unroll
         for (uint32_t hf = 0; hf < 2; hf++) {
-            S[hf] = af4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (FINE) {  // a sum of its own per 16 dims, added in double below
+                typedef _Float16 ah4 __attribute__((ext_vector_type(4)));
+                typedef uint32_t au2 __attribute__((ext_vector_type(2)));
+                const af4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (uint32_t kk = 0; kk < 4; kk++)
-                S[hf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(ah8, kr[hf][kk]),
-                                                              Qb[kk], S[hf], 0, 0, 0);
+                for (uint32_t kk = 0; kk < KK; kk++)
+#pragma unroll
+                    for (uint32_t v = 0; v < 2u; v++) {
+                        const au2 ka = {kr[hf][kk][2u * v], kr[hf][kk][2u * v + 1u]};
+                        const au4 qq = __builtin_bit_cast(au4, Qb[kk]);
+                        const au2 qa = {qq[2u * v], qq[2u * v + 1u]};
+                        S[hf][2u * kk + v] = __builtin_amdgcn_mfma_f32_16x16x16f16(
+                            __builtin_bit_cast(ah4, ka), __builtin_bit_cast(ah4, qa), z, 0, 0, 0);
+                    }
+            } else {
+                S[hf][0] = af4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (uint32_t kk = 0; kk < KK; kk++)
+                    S[hf][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(ah8, kr[hf][kk]),
+                                                                  Qb[kk], S[hf][0], 0, 0, 0);
+            }
         }
         if (t + 1u < nt) load_k(t + 1u);  // the K registers are free again
         // scores of positions p_j: hi + lo columns (lane n and n ^ 8), scaled, masked
-        float sc[8], mt = -INFINITY;
+        float dot[8], sc[8], mt = -INFINITY;
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++) {
-            const float v = S[j >> 2][j & 3u];
+            float v;
+            if constexpr (FINE) {
+                double d = 0.0;
+#pragma unroll
+                for (uint32_t k = 0; k < 2u * KK; k++) d += (double)S[j >> 2][k][j & 3u];
+                v = (float)d;
+            } else {
+                v = S[j >> 2][0][j & 3u];
+            }
             const float w = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
                                                               0, __builtin_bit_cast(int, v), 0x128,
                                                               0xF, 0xF, false));  // row_ror:8
-            sc[j] = pos_of(t, j) < valid ? __fmul_rn(w, csc) : -INFINITY;
+            const bool in = pos_of(t, j) < valid;
+            dot[j] = in ? w : 0.f;
+            sc[j] = in ? __fmul_rn(w, c2) : -INFINITY;
             mt = fmaxf(mt, sc[j]);
         }
         mt = fmaxf(mt, lane_xor<16>(mt));
         mt = fmaxf(mt, lane_xor<32>(mt));
+        if (FINE) mt = ceilf(mt);
         const float mn = fmaxf(m, mt);
-        const float rs = m == -INFINITY ? 0.f : fast_exp(__fsub_rn(m, mn));
+        const float rs = m == -INFINITY ? 0.f : merge_exp<HD>(__fsub_rn(m, mn));
         m = mn;
         l *= rs;
         ah8 P;
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++) {
-            const float e = sc[j] == -INFINITY ? 0.f : fast_exp(__fsub_rn(sc[j], mn));
+            float e;
+            if constexpr (FINE) {  // s2 = n + x, |x| <= 1/2 and a bit: 2^x times an exact 2^(n - m)
+                const float p = __fmul_rn(dot[j], c2), n = rintf(p);
+                const float err = fmaf(dot[j], c2lo, fmaf(dot[j], c2, -p));
+                e = ldexpf(exp2_fast((p - n) + __builtin_amdgcn_fmed3f(err, -0.5f, 0.5f)), (int)(n - mn));
+            } else {
+                e = fast_exp(__fsub_rn(sc[j], mn));
+            }
+            if (sc[j] == -INFINITY) e = 0.f;
             l += e;
-            const _Float16 hi = (_Float16)e;
-            P[j] = n < 8u ? hi : (_Float16)(e - (float)hi);
+            const float es = e * PS;
+            const _Float16 hi = (_Float16)es;
+            P[j] = n < 8u ? hi : (_Float16)(es - (float)hi);
         }
         // D rows 4 g + r of the P V accumulators belong to head (4 g + r) & 7
         float rsr[4];
 #pragma unroll
         for (uint32_t r = 0; r < 4; r++) rsr[r] = __shfl(rs, (4u * g + r) & 7u, 64);
 #pragma unroll
-        for (uint32_t dt = 0; dt < 8; dt++) {
-            // B: element dt (head dim 8 n + dt) of each of the lane's eight V rows
+        for (uint32_t dt = 0; dt < DPL; dt++) {
+            // B: element dt (head dim DPL n + dt) of each of the lane's eight V rows
             const uint32_t sel = (dt & 1u) ? 0x07060302u : 0x05040100u;
             au4 b;
 #pragma unroll
@@ -548,13 +385,40 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
     l += lane_xor<16>(l);
     l += lane_xor<32>(l);
 #pragma unroll
-    for (uint32_t dt = 0; dt < 8; dt++)
+    for (uint32_t dt = 0; dt < DPL; dt++)
 #pragma unroll
-        for (uint32_t r = 0; r < 4; r++) a[dt][r] = acc[dt][r] + lane_xor<32>(acc[dt][r]);
+        for (uint32_t r = 0; r < 4; r++) a[dt][r] = (acc[dt][r] + lane_xor<32>(acc[dt][r])) * (1.f / PS);
     m_out = m;
     l_out = l;
 }
 
+// A chunk's (m, l, acc) to its partials row (chunk rows `stride` apart per q
+// head; HD + 2 floats each).
+template <uint32_t HD>
+__device__ __forceinline__ void attn_mfma_store(float *pk, uint32_t stride, uint32_t chunk, uint32_t group,
+                                                uint32_t lane, float m, float l, const float (&a)[HD / 16][4]) {
+    constexpr uint32_t DPL = HD / 16u;
+    const uint32_t n = lane & 15u, g = lane >> 4;
+    if (g < 2u) {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) {
+            const uint32_t hh = 4u * g + r;
+            if (hh < group) {
+                float *dst = pk + ((uint64_t)hh * stride + chunk) * part_row<HD> + 2u + DPL * n;
+#pragma unroll
+                for (uint32_t i = 0; i < DPL / 2u; i++)
+                    reinterpret_cast<float2 *>(dst)[i] = make_float2(a[2 * i][r], a[2 * i + 1][r]);
+            }
+        }
+    }
+    if (g == 0 && n < group) {
+        float *dst = pk + ((uint64_t)n * stride + chunk) * part_row<HD>;
+        dst[0] = m;
+        dst[1] = l;
+    }
+}
+
+template <uint32_t HD>
 __global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
                                                   const uint16_t *__restrict__ kc,
                                                   const uint16_t *__restrict__ vc,
@@ -566,9 +430,7 @@ __global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
                                                   uint64_t part_bstride, uint32_t target,
                                                   uint32_t *__restrict__ clear, uint32_t nclear,
                                                   uint32_t clear_stride) {
-    constexpr uint32_t HD = 128;
     const uint32_t chunk = blockIdx.x, kvh = blockIdx.y, lane = threadIdx.x, bz = blockIdx.z;
-    const uint32_t n = lane & 15u, g = lane >> 4;
     // the merging launch that follows (k_mvl_attn) starts from cleared flags
     if (clear && chunk == 0u && kvh == 0u && bz == 0u)
         for (uint32_t i = lane; i < nclear; i += 64u) clear[(uint64_t)i * clear_stride] = 0u;
@@ -581,26 +443,40 @@ __global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
     const AttnSplit sp = attn_split(seq_len, nkh, kMfmaGran, kMfmaLmax, target);
     if (chunk >= sp.n) return;  // past the sequence (the grid covers the longest split)
     const uint32_t s0 = chunk * sp.len, valid = min(sp.len, seq_len - s0);
-    float m, l, a[8][4];
-    attn_mfma_wave(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale,
+    float m, l, a[HD / 16][4];
+    attn_mfma_wave<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale,
                    lane, m, l, a);
-    float *const pk = part + (uint64_t)kvh * group * stride_chunks * (HD + 2u);
-    if (g < 2u) {
-#pragma unroll
-        for (uint32_t r = 0; r < 4; r++) {
-            const uint32_t hh = 4u * g + r;
-            if (hh < group) {
-                float *dst = pk + ((uint64_t)hh * stride_chunks + chunk) * (HD + 2u) + 2u + 8u * n;
-#pragma unroll
-                for (uint32_t i = 0; i < 4; i++)
-                    reinterpret_cast<float2 *>(dst)[i] = make_float2(a[2 * i][r], a[2 * i + 1][r]);
-            }
-        }
+    attn_mfma_store<HD>(part + (uint64_t)kvh * group * stride_chunks * part_row<HD>, stride_chunks, chunk,
+                        group, lane, m, l, a);
+}
+
+// Short sequences (at most kOneChunks chunks) in one launch: workgroup kvh
+// takes the kv head's chunks one per wave, as k_attn_mfma does (bit-identical:
+// the same split, arithmetic and merge), leaves the partials in LDS and merges
+// its q heads there.
+constexpr uint32_t kOneChunks = 8;
+
+template <uint32_t HD>
+__global__ __launch_bounds__(64 * kOneChunks) void k_attn_one(
+    const float *__restrict__ q, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,
+    float *__restrict__ out, uint32_t seq_len, const uint32_t *__restrict__ pos_dev, uint64_t layer_off,
+    uint32_t nkh, uint32_t group, float scale) {
+    extern __shared__ __align__(16) float part[];  // [group][kOneChunks][HD + 2]
+    const uint32_t nw = blockDim.x >> 6, kvh = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    if (pos_dev) seq_len = pos_dev[0] + 1u;
+    const AttnSplit sp = attn_split(seq_len, nkh, kMfmaGran, kMfmaLmax, kMfmaTargetWgs);
+    if (wave < sp.n) {
+        const uint32_t s0 = wave * sp.len, valid = min(sp.len, seq_len - s0);
+        float m, l, a[HD / 16][4];
+        attn_mfma_wave<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane,
+                           m, l, a);
+        attn_mfma_store<HD>(part, kOneChunks, wave, group, lane, m, l, a);
     }
-    if (g == 0 && n < group) {
-        float *dst = pk + ((uint64_t)n * stride_chunks + chunk) * (HD + 2u);
-        dst[0] = m;
-        dst[1] = l;
+    __syncthreads();
+    for (uint32_t h = wave; h < group; h += nw) {
+        const float2 o = merge_one_wave<kOneChunks, HD>(part + h * kOneChunks * part_row<HD>, sp.n, lane);
+        if (HD == 128u || lane < HD / 2u)
+            *reinterpret_cast<float2 *>(out + ((uint64_t)kvh * group + h) * HD + 2u * lane) = o;
     }
 }
 
@@ -689,13 +565,14 @@ __global__ __launch_bounds__(kMergeThreads) void k_attn_merge(const float *__res
     }
 }
 
-// Merge for head_dim 128 (the matrix-core chunk kernel's partials): one
+// Merge of the matrix-core chunk kernel's partials: one
 // workgroup of four waves per q head (grid y: the sequences of a batch). Every
 // wave forms M, L and the chunk weights itself from all chunks' (m, l); wave r
 // takes residue r of the chunks (vbs_attn_common.h), its acc rows loaded at
 // once, and one LDS pass adds the four sums in order. No loads wait on a
 // reduction and one barrier ends it (the general merge above has four).
-__global__ __launch_bounds__(64 * kMergeRes) void k_attn_merge_h128(
+template <uint32_t HD>
+__global__ __launch_bounds__(64 * kMergeRes) void k_attn_merge_hd(
     const float *__restrict__ part, float *__restrict__ out, uint32_t stride_chunks,
     const uint32_t *__restrict__ pos_dev, uint32_t seq_len, uint32_t nkh, uint32_t q_bstride,
     uint64_t part_bstride, uint32_t target) {
@@ -705,17 +582,18 @@ __global__ __launch_bounds__(64 * kMergeRes) void k_attn_merge_h128(
     out += (uint64_t)bz * q_bstride;
     if (pos_dev) seq_len = pos_dev[bz] + 1u;  // seq = pos + 1
     const uint32_t nc = mfma_chunks(seq_len, nkh, target);
-    const float *ph = part + (uint64_t)h * stride_chunks * kPartRow;
+    const float *ph = part + (uint64_t)h * stride_chunks * part_row<HD>;
     float2 av[kMergeBatch];
-    merge_residue_load(ph, nc, wave, lane, av);  // with the (m, l) loads: one round trip
-    const MergeStats st = merge_stats(ph, nc, lane, merge_ml_load(ph, nc, lane));
-    red[wave][lane] = merge_residue_sum(ph, nc, st, wave, lane, av);
+    merge_residue_load<HD>(ph, nc, wave, lane, av);  // with the (m, l) loads: one round trip
+    const MergeStats st = merge_stats<HD>(ph, nc, lane, merge_ml_load<HD>(ph, nc, lane));
+    red[wave][lane] = merge_residue_sum<HD>(ph, nc, st, wave, lane, av);
     __syncthreads();
     if (wave == 0) {
         float2 a[kMergeRes];
 #pragma unroll
         for (uint32_t r = 0; r < kMergeRes; r++) a[r] = red[r][lane];
-        *reinterpret_cast<float2 *>(out + (uint64_t)h * 128u + 2u * lane) = merge_finish(a, st.L);
+        if (HD == 128u || lane < HD / 2u)
+            *reinterpret_cast<float2 *>(out + (uint64_t)h * HD + 2u * lane) = merge_finish(a, st.L);
     }
 }
 
@@ -723,23 +601,30 @@ size_t attention_partial_bytes(uint32_t max_seq, uint32_t nqh, uint32_t nkh, uin
     return (size_t)nqh * attn_max_chunks(max_seq, nkh) * (hd + 2u) * sizeof(float);
 }
 
+// The matrix-core path of one sequence: one launch up to kOneChunks chunks
+// (seq_len is the longest that the launch must cover), else chunks and merge.
 template <uint32_t HD>
-static hipError_t launch_chunk_hd(dim3 grid, hipStream_t s, const float *q, const uint16_t *kc,
-                                  const uint16_t *vc, float *part, uint32_t seq_len,
-                                  const uint32_t *pos_dev, uint64_t layer_off, uint32_t nkh,
-                                  uint32_t group, float scale) {
-    const size_t lds = (size_t)kWaves * group * HD * sizeof(float);
-#define VBS_ATTN_G(GG)                                                                          \
-    do {                                                                                        \
-        k_attn_chunk<HD, GG><<<grid, 64u * kWaves, lds, s>>>(q, kc, vc, part, seq_len, pos_dev,   \
-                                                            layer_off, nkh, group, scale, grid.x);\
-        return hipGetLastError();                                                                 \
-    } while (0)
-    if (group <= 1) VBS_ATTN_G(1);
-    if (group <= 2) VBS_ATTN_G(2);
-    if (group <= 4) VBS_ATTN_G(4);
-    VBS_ATTN_G(8);
-#undef VBS_ATTN_G
+static hipError_t launch_mfma_hd(const float *q, const uint16_t *kc, const uint16_t *vc, float *out,
+                                 float *part, uint32_t seq_len, const uint32_t *pos_dev, uint64_t layer_off,
+                                 uint32_t nkh, uint32_t group, float scale, hipStream_t s) {
+    const uint32_t chunks = mfma_grid_chunks(seq_len, nkh), stride = attn_max_chunks(seq_len, nkh);
+    // One launch: 41 positions of 8 kv heads 3.4-4.6 us (chunks and merge 6.5-9),
+    // 256 of head_dim 64 4.8 (8.8); at head_dim 128 and eight q heads per kv head
+    // 256 positions are too many for one workgroup (7.9 against 7.1), 96 alike.
+    if (chunks <= (HD <= 64u ? kOneChunks : kOneChunks / 2u)) {
+        const uint32_t nw = chunks > group ? chunks : group;  // a wave per chunk, then per q head
+        const size_t lds = (size_t)group * kOneChunks * part_row<HD> * sizeof(float);
+        k_attn_one<HD><<<nkh, 64u * nw, lds, s>>>(q, kc, vc, out, seq_len, pos_dev, layer_off, nkh, group,
+                                                     scale);
+        return hipGetLastError();
+    }
+    k_attn_mfma<HD><<<dim3(chunks, nkh), 64, 0, s>>>(q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group,
+                                                    scale, stride, 0u, 0ull, 0ull, kMfmaTargetWgs, nullptr, 0u, 0u);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    k_attn_merge_hd<HD><<<nkh * group, 64 * kMergeRes, 0, s>>>(part, out, stride, pos_dev, seq_len, nkh, 0u, 0ull,
+                                                             kMfmaTargetWgs);
+    return hipGetLastError();
 }
 
 hipError_t launch_attention(const float *q, const uint16_t *kc, const uint16_t *vc, float *out,
@@ -757,44 +642,29 @@ hipError_t launch_attention(const float *q, const uint16_t *kc, const uint16_t *
         part = (float *)rt_scratch(attention_partial_bytes(seq_len, nqh, nkh, hd), s, &why);
         if (!part) return why;
     }
-    const bool fast = (hd == 32u || hd == 64u || hd == 128u) && group <= 8u &&
-                      ((uintptr_t)q & 15u) == 0 && ((uintptr_t)kc & 15u) == 0 &&
-                      ((uintptr_t)vc & 15u) == 0;
-    hipError_t e;
-    uint32_t gran = kChunk, lmax = kChunk, target = kTargetWgs;
-    const dim3 grid(stride, nkh);
-    if (fast && hd == 128u) {
-        k_attn_mfma<<<dim3(mfma_grid_chunks(seq_len, nkh), nkh), 64, 0, s>>>(
-            q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group, scale, stride, 0u, 0ull, 0ull,
-            kMfmaTargetWgs, nullptr, 0u, 0u);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        k_attn_merge_h128<<<nqh, 64 * kMergeRes, 0, s>>>(part, out, stride, pos_dev, seq_len, nkh,
-                                                            0u, 0ull, kMfmaTargetWgs);
-        return hipGetLastError();
-    } else if (fast && hd == 32u) {
-        gran = ChunkShape<32>::GRAN, lmax = ChunkShape<32>::LMAX;
-        e = launch_chunk_hd<32>(grid, s, q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group,
-                                scale);
-    } else if (fast && hd == 64u) {
-        gran = ChunkShape<64>::GRAN, lmax = ChunkShape<64>::LMAX;
-        e = launch_chunk_hd<64>(grid, s, q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group,
-                                scale);
-    } else if (fast) {
-        gran = ChunkShape<128>::GRAN, lmax = ChunkShape<128>::LMAX;
-        e = launch_chunk_hd<128>(grid, s, q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group,
-                                 scale);
-    } else {
-        const size_t lds = ((size_t)group * hd + (size_t)group * kChunk +
-                            (size_t)(256u / hd) * group * hd) * sizeof(float);
-        k_attn_partial<<<grid, 256, lds, s>>>(q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, hd,
-                                              group, scale, stride);
-        e = hipGetLastError();
+    if (group <= 8u && ((uintptr_t)q & 15u) == 0 && ((uintptr_t)kc & 15u) == 0 && ((uintptr_t)vc & 15u) == 0) {
+#define VBS_ATTN_HD(HD)                                                                                \
+    case HD:                                                                                           \
+        return launch_mfma_hd<HD>(q, kc, vc, out, part, seq_len, pos_dev, layer_off, nkh, group, scale, s)
+        switch (hd) {
+            VBS_ATTN_HD(32);
+            VBS_ATTN_HD(64);
+            VBS_ATTN_HD(96);
+            VBS_ATTN_HD(128);
+            default: break;
+        }
+#undef VBS_ATTN_HD
     }
+    const size_t lds = ((size_t)group * hd + (size_t)group * kChunk + (size_t)(256u / hd) * group * hd) *
+                       sizeof(float);
+    k_attn_partial<<<dim3(stride, nkh), 256, lds, s>>>(q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, hd,
+                                                       group, scale, stride);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const uint32_t n_chunks = attn_split(seq_len, nkh, gran, lmax, target).n;
+    const uint32_t n_chunks = attn_split(seq_len, nkh, kChunk, kChunk, kTargetWgs).n;
     const size_t mlds = ((size_t)stride + kMergeThreads) * sizeof(float);
-    k_attn_merge<<<nqh, kMergeThreads, mlds, s>>>(part, out, hd, n_chunks, stride, pos_dev, nkh, gran,
-                                                  lmax, target, 0u, 0ull);
+    k_attn_merge<<<nqh, kMergeThreads, mlds, s>>>(part, out, hd, n_chunks, stride, pos_dev, nkh, kChunk, kChunk,
+                                                  kTargetWgs, 0u, 0ull);
     return hipGetLastError();
 }
 
@@ -812,7 +682,7 @@ hipError_t launch_attention_chunks(const float *q, const uint16_t *kc, const uin
     if (seq_len == 0 || nkh == 0 || nqh % nkh != 0 || hd != 128u || nqh / nkh > 8u || !part ||
         ((uintptr_t)q & 15u) || ((uintptr_t)kc & 15u) || ((uintptr_t)vc & 15u))
         return hipErrorNotSupported;
-    k_attn_mfma<<<dim3(mfma_grid_chunks(seq_len, nkh), nkh), 64, 0, s>>>(
+    k_attn_mfma<128><<<dim3(mfma_grid_chunks(seq_len, nkh), nkh), 64, 0, s>>>(
         q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, nqh / nkh, scale, attn_max_chunks(seq_len, nkh),
         0u, 0ull, 0ull, kMfmaTargetWgs, clear, nclear, stride);
     return hipGetLastError();
@@ -848,12 +718,12 @@ hipError_t launch_attention_batch(const float *q, const uint16_t *kc, const uint
         return hipSuccess;
     }
     const uint32_t stride = attn_max_chunks(max_seq, nkh), target = attn_batch_target(batch);
-    k_attn_mfma<<<dim3(mfma_grid_chunks(max_seq, nkh, target), nkh, batch), 64, 0, s>>>(
+    k_attn_mfma<128><<<dim3(mfma_grid_chunks(max_seq, nkh, target), nkh, batch), 64, 0, s>>>(
         q, kc, vc, part, max_seq, pos_dev, layer_off, nkh, group, scale, stride, q_stride, kv_stride,
         pstride, target, nullptr, 0u, 0u);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !out) return e;  // (no out: the caller merges the partials itself)
-    k_attn_merge_h128<<<dim3(nqh, batch), 64 * kMergeRes, 0, s>>>(part, out, stride, pos_dev,
+    k_attn_merge_hd<128><<<dim3(nqh, batch), 64 * kMergeRes, 0, s>>>(part, out, stride, pos_dev,
                                                                      max_seq, nkh, q_stride, pstride,
                                                                      target);
     return hipGetLastError();

@@ -846,7 +846,7 @@ static hipError_t launch_mvb_plan(const MbArgs &a, hipStream_t s) {
 // The batched decoder's attention merge (head_dim 128, the matrix-core chunk
 // kernel's partials) writing O's prepared x directly: workgroup (pair p,
 // sequence t) merges q heads 2p and 2p + 1 -- block p of the attention output
-// -- as k_attn_merge_h128 does (four waves per head, the same vbs_attn_common.h
+// -- as k_attn_merge_hd does (four waves per head, the same vbs_attn_common.h
 // pieces), then one wave prepares the block with xprep_block: the values and
 // the prepared bytes equal the merge launch followed by k_xprep_b's.
 __global__ __launch_bounds__(512) void k_attn_merge_prep(const float *__restrict__ part,

@@ -492,7 +492,7 @@ hipError_t launch_q4k_mvl(const uint8_t *w, const float *x, float *y, uint32_t c
 // the launch instead of by a merge launch of its own. Workgroups are dealt to
 // the eight XCDs round-robin in flat-index order, so with 8 nqh of them each
 // XCD holds the 8 j + r for one r and every j < nqh: workgroup i merges q head
-// i / 8 (waves 0..3, as k_attn_merge_h128: bit-identical), publishes it to its
+// i / 8 (waves 0..3, as k_attn_merge_hd: bit-identical), publishes it to its
 // XCD's copy of the vector (its XCC_ID register) and raises the head's flag
 // there, a 128-byte line of its own; then its wave 0 waits for all the
 // heads' flags, read in the XCD's L2 by atomic adds of zero, copies the vector
@@ -590,7 +590,7 @@ __global__ __launch_bounds__(64 * kMvlWaves) void k_mvl_attn(const AttnOArgs a) 
         ml = merge_ml_mask(ml, nc, lane);
     }
 
-    // 3. waves 0..3: the merge of head hh, as k_attn_merge_h128
+    // 3. waves 0..3: the merge of head hh, as k_attn_merge_hd
     MergeStats st{};
     if (wave < kMergeRes) {
         st = merge_stats(ph, nc, lane, ml);
