@@ -103,6 +103,21 @@ def test_hot_matvec_bit_exact(dev, host, orc, t, rows, cols):
     assert same_bits(got, want), (t, rows, cols, np.flatnonzero(got != want)[:5])
 
 
+@pytest.mark.parametrize("t", HOT_TYPES, ids=IDS)
+@pytest.mark.parametrize("rows,cols", [(1, 32), (15, 224), (17, 256), (16, 288), (5, 512), (6, 544), (3, 1024),
+                                       (2, 2048), (9, 2080), (4, 16384), (3, 16416), (2, 33824)])
+def test_hot_matvec_tile_edges(dev, host, orc, t, rows, cols):
+    """Rows that end on and past the kernels' steps, tiles of 256 columns,
+    chunks of 512 blocks and groups of 32 terms, in workgroups partly idle;
+    F16 and F32 rows also one element short."""
+    for c in (cols, cols - 1) if t in (V.F32, V.F16) else (cols,):
+        w = V.synth_matrix(host, t, rows, c, 90 + t, 1)
+        x = edge_activations(host, cols, 91 + t)
+        xq, qd, qs = orc.quantize_q8(x)
+        got = dev_hot(dev, t, w, rows, c, xq, qd, qs, x[:c].copy())
+        assert same_bits(got, orc.hot_matvec(t, w, rows, c, xq, qd, qs, x[:c].copy())), c
+
+
 @pytest.mark.parametrize("t", [V.F32, V.F16], ids=["F32", "F16"])
 def test_hot_matvec_ragged_float_rows(dev, host, orc, t):
     rows, cols = 9, 1000  # F32 / F16 rows need not be whole blocks
