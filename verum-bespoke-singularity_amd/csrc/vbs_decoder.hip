@@ -227,6 +227,112 @@ static hipError_t launch_argmax_embed(int type, const float *logits, uint32_t n,
     return hipGetLastError();
 }
 
+// The first step's state and input, from the kernel arguments: for sequence b
+// (of nb) token, position and step 0 into state[b], state[nb + b], state[2 nb +
+// b], and row `token` of the embedding table to x + b * dim (as
+// k_argmax_advance leaves it for the steps after). One launch, no copy to wait
+// for: a copy of the state, the gather and a synchronization before the graph
+// took 40 us of every call.
+constexpr uint32_t kStartMax = 8;
+struct StartArgs {
+    uint32_t token[kStartMax], pos[kStartMax];
+};
+template <int T>
+__global__ __launch_bounds__(256) void k_decoder_start(StartArgs a, uint32_t nb, uint32_t *state,
+                                                       const uint8_t *__restrict__ embd,
+                                                       uint64_t embd_rb, uint32_t dim,
+                                                       float *__restrict__ x) {
+    const uint32_t b = blockIdx.y, e = blockIdx.x * 256u + threadIdx.x;
+    if (e == 0u) {
+        state[b] = a.token[b];
+        state[nb + b] = a.pos[b];
+        state[2u * nb + b] = 0u;
+    }
+    if (e >= dim) return;
+    const uint8_t *row = embd + (uint64_t)a.token[b] * embd_rb;
+    x[(uint64_t)b * dim + e] = deq_elem<T>(row + (uint64_t)(e / Geo<T>::E) * Geo<T>::B, e % Geo<T>::E);
+}
+
+static hipError_t launch_decoder_start(int type, const uint32_t *tokens, const uint32_t *pos, uint32_t nb,
+                                       uint32_t *state, const void *embd, uint32_t dim, float *x,
+                                       hipStream_t s) {
+    if (nb == 0u || nb > kStartMax) return hipErrorInvalidValue;
+    StartArgs a{};
+    for (uint32_t b = 0; b < nb; b++) a.token[b] = tokens[b], a.pos[b] = pos[b];
+    const dim3 grid((dim + 255u) / 256u, nb);
+    const uint64_t rb = row_bytes(type, dim);
+    const uint8_t *e = (const uint8_t *)embd;
+#define VBS_START(TT) k_decoder_start<TT><<<grid, 256, 0, s>>>(a, nb, state, e, rb, dim, x)
+    switch (type) {
+        case kF32: VBS_START(kF32); break;
+        case kF16: VBS_START(kF16); break;
+        case kQ4_0: VBS_START(kQ4_0); break;
+        case kQ4_1: VBS_START(kQ4_1); break;
+        case kQ8_0: VBS_START(kQ8_0); break;
+        case kQ4_K: VBS_START(kQ4_K); break;
+        case kQ6_K: VBS_START(kQ6_K); break;
+        case kLNS8: VBS_START(kLNS8); break;
+        default: return hipErrorInvalidValue;
+    }
+#undef VBS_START
+    return hipGetLastError();
+}
+
+// Results on their way to the caller: a decoder's own pinned buffer, which a
+// kernel of the step's stream writes (NULL if there was none to be had: then
+// copies straight to the caller). A 7B step's 128 KB of logits: 23 us after
+// the graph, 36 through the copy engine, 43 as a copy to pageable memory.
+__global__ __launch_bounds__(256) void k_fetch(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst,
+                                               size_t n) {
+    const size_t step = (size_t)gridDim.x * 256u;
+    size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
+    if ((((uintptr_t)src | (uintptr_t)dst) & 15u) == 0u) {
+        const size_t n4 = n / 4u;
+        for (size_t k = i; k < n4; k += step)
+            reinterpret_cast<uint4 *>(dst)[k] = reinterpret_cast<const uint4 *>(src)[k];
+        i += 4u * n4;
+    }
+    for (; i < n; i += step) dst[i] = src[i];
+}
+
+struct Fetch {
+    uint8_t *pinned = nullptr;
+    size_t used = 0;
+    struct {
+        void *dst;
+        size_t at, bytes;
+    } part[3];
+    int n = 0;
+    hipError_t add(void *dst, const void *src, size_t bytes, hipStream_t s) {
+        if (bytes == 0) return hipSuccess;
+        if (!pinned) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        const size_t words = bytes / 4u, wgs = (words + 1023u) / 1024u;
+        k_fetch<<<(uint32_t)(wgs < 256u ? wgs : 256u), 256, 0, s>>>((const uint32_t *)src, (uint32_t *)(pinned + used),
+                                                                     words);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        part[n++] = {dst, used, bytes};
+        used += (bytes + 255u) & ~(size_t)255u;
+        return e;
+    }
+    hipError_t finish(hipStream_t s) {
+        const hipError_t e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
+        for (int i = 0; i < n; i++) memcpy(part[i].dst, pinned + part[i].at, part[i].bytes);
+        return e;
+    }
+};
+// Room for the logits of `nb` sequences and for a greedy run's tokens and margins.
+static void *fetch_buffer(uint32_t vocab, uint32_t nb, uint32_t max_steps) {
+    void *p = nullptr;
+    const size_t bytes = ((size_t)vocab + 2u * (size_t)max_steps) * nb * 4u + 3u * 256u;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
 // ---- decoder -------------------------------------------------------------------
 
 struct Decoder {
@@ -250,6 +356,7 @@ struct Decoder {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     void *arena = nullptr;
+    void *pinned = nullptr;  // Fetch
 };
 
 // Polls of a workgroup's bounded wait for its XCD's merged heads in the O launch:
@@ -396,6 +503,10 @@ static void decoder_free(Decoder *d) {
         (void)hipStreamSynchronize(rt_stream());
         (void)hipFree(d->arena);
     }
+    if (d->pinned) {
+        (void)hipStreamSynchronize(rt_stream());
+        (void)hipHostFree(d->pinned);
+    }
     delete d;
 }
 
@@ -490,6 +601,7 @@ int vbs_gfx950_decoder_create(const vbs_gfx950_model_t *m, uint32_t max_steps, v
         decoder_free(d);
         return 0;
     }
+    d->pinned = fetch_buffer(m->vocab, 1u, d->max_steps);
     // capture one token step
     if (!rt_hip_ok(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture")) {
         decoder_free(d);
@@ -516,14 +628,9 @@ int vbs_gfx950_decoder_create(const vbs_gfx950_model_t *m, uint32_t max_steps, v
 static int set_state(Decoder *d, uint32_t token, uint32_t pos) {
     if (token >= d->m.vocab) return rt_fail("decoder: token %u >= vocab %u", token, d->m.vocab);
     if (pos >= d->m.max_ctx) return rt_fail("decoder: pos %u >= max_ctx %u", pos, d->m.max_ctx);
-    const uint32_t st[3] = {token, pos, 0};
-    hipStream_t s = rt_stream();
-    return rt_hip_ok(hipMemcpyAsync(d->state, st, sizeof(st), hipMemcpyHostToDevice, s),
-                     "decoder: state") &&
-           rt_hip_ok(launch_dequant_rows(d->m.embd_type, (const uint8_t *)d->m.tok_embd, d->state,
-                                         0, 1, d->m.hidden, d->stream, s),
-                     "decoder: first embedding") &&
-           rt_hip_ok(hipStreamSynchronize(s), "decoder: state");
+    return rt_hip_ok(launch_decoder_start(d->m.embd_type, &token, &pos, 1u, d->state, d->m.tok_embd,
+                                          d->m.hidden, d->stream, rt_stream()),
+                     "decoder: state and first embedding");
 }
 
 int vbs_gfx950_decoder_step(void *handle, uint32_t token, uint32_t pos, float *logits) {
@@ -533,11 +640,11 @@ int vbs_gfx950_decoder_step(void *handle, uint32_t token, uint32_t pos, float *l
     if (!set_state(d, token, pos)) return 0;
     hipStream_t s = rt_stream();
     if (!rt_hip_ok(hipGraphLaunch(d->exec, s), "decoder_step: graph launch")) return 0;
-    if (logits &&
-        !rt_hip_ok(hipMemcpyAsync(logits, d->logits, (size_t)d->m.vocab * 4, hipMemcpyDeviceToHost, s),
-                   "decoder_step: logits"))
+    Fetch f;
+    f.pinned = (uint8_t *)d->pinned;
+    if (logits && !rt_hip_ok(f.add(logits, d->logits, (size_t)d->m.vocab * 4, s), "decoder_step: logits"))
         return 0;
-    return rt_hip_ok(hipStreamSynchronize(s), "decoder_step");
+    return rt_hip_ok(f.finish(s), "decoder_step");
 }
 
 int vbs_gfx950_decoder_greedy(void *handle, uint32_t token, uint32_t pos, uint32_t n,
@@ -551,14 +658,11 @@ int vbs_gfx950_decoder_greedy(void *handle, uint32_t token, uint32_t pos, uint32
     hipStream_t s = rt_stream();
     for (uint32_t i = 0; i < n; i++)
         if (!rt_hip_ok(hipGraphLaunch(d->exec, s), "decoder_greedy: graph launch")) return 0;
-    if (!rt_hip_ok(hipMemcpyAsync(tokens, d->tokens, (size_t)n * 4, hipMemcpyDeviceToHost, s),
-                   "decoder_greedy: tokens"))
-        return 0;
-    if (margins &&
-        !rt_hip_ok(hipMemcpyAsync(margins, d->margins, (size_t)n * 4, hipMemcpyDeviceToHost, s),
-                   "decoder_greedy: margins"))
-        return 0;
-    return rt_hip_ok(hipStreamSynchronize(s), "decoder_greedy");
+    Fetch f;
+    f.pinned = (uint8_t *)d->pinned;
+    if (!rt_hip_ok(f.add(tokens, d->tokens, (size_t)n * 4, s), "decoder_greedy: tokens")) return 0;
+    if (margins && !rt_hip_ok(f.add(margins, d->margins, (size_t)n * 4, s), "decoder_greedy: margins")) return 0;
+    return rt_hip_ok(f.finish(s), "decoder_greedy");
 }
 
 int vbs_gfx950_decoder_greedy_eager(void *handle, uint32_t token, uint32_t pos, uint32_t n,
@@ -573,14 +677,11 @@ int vbs_gfx950_decoder_greedy_eager(void *handle, uint32_t token, uint32_t pos, 
     hipStream_t s = rt_stream();
     for (uint32_t i = 0; i < n; i++)
         if (!rt_hip_ok(enqueue_step(*d, s), "decoder_greedy_eager: step")) return 0;
-    if (!rt_hip_ok(hipMemcpyAsync(tokens, d->tokens, (size_t)n * 4, hipMemcpyDeviceToHost, s),
-                   "decoder_greedy_eager: tokens"))
-        return 0;
-    if (margins &&
-        !rt_hip_ok(hipMemcpyAsync(margins, d->margins, (size_t)n * 4, hipMemcpyDeviceToHost, s),
-                   "decoder_greedy_eager: margins"))
-        return 0;
-    return rt_hip_ok(hipStreamSynchronize(s), "decoder_greedy_eager");
+    Fetch f;
+    f.pinned = (uint8_t *)d->pinned;
+    if (!rt_hip_ok(f.add(tokens, d->tokens, (size_t)n * 4, s), "decoder_greedy_eager: tokens")) return 0;
+    if (margins && !rt_hip_ok(f.add(margins, d->margins, (size_t)n * 4, s), "decoder_greedy_eager: margins")) return 0;
+    return rt_hip_ok(f.finish(s), "decoder_greedy_eager");
 }
 
 int vbs_gfx950_decoder_attn_o_fallbacks(void *handle, uint32_t *count) {
@@ -672,6 +773,7 @@ struct BDecoder {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     void *arena = nullptr;
+    void *pinned = nullptr;  // Fetch
 };
 
 static hipError_t enqueue_step_batch(const BDecoder &d, hipStream_t s) {
@@ -764,6 +866,10 @@ static void bdecoder_free(BDecoder *d) {
     if (d->arena) {
         (void)hipStreamSynchronize(rt_stream());
         (void)hipFree(d->arena);
+    }
+    if (d->pinned) {
+        (void)hipStreamSynchronize(rt_stream());
+        (void)hipHostFree(d->pinned);
     }
     delete d;
 }
@@ -861,6 +967,7 @@ int vbs_gfx950_bdecoder_create(const vbs_gfx950_model_t *m, uint32_t batch, uint
         bdecoder_free(d);
         return 0;
     }
+    d->pinned = fetch_buffer(m->vocab, batch, d->max_steps);
     if (!rt_hip_ok(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture")) {
         bdecoder_free(d);
         return 0;
@@ -884,46 +991,37 @@ int vbs_gfx950_bdecoder_create(const vbs_gfx950_model_t *m, uint32_t batch, uint
 }
 
 static int bdecoder_run(void *handle, const uint32_t *tokens0, const uint32_t *pos0, uint32_t n,
-                        uint32_t *tokens, float *margins, bool eager, float *logits = nullptr) {
+                        uint32_t *tokens, float *margins, bool eager, float *logits = nullptr, bool step = false) {
     if (!rt_ready()) return 0;
     BDecoder *d = (BDecoder *)handle;
-    if (!d || !tokens0 || !pos0 || !tokens) return rt_fail("bdecoder_greedy: null argument");
+    if (!d || !tokens0 || !pos0 || !(tokens || step)) return rt_fail("bdecoder_greedy: null argument");
     if (n > d->max_steps) return rt_fail("bdecoder_greedy: %u steps > max_steps %u", n, d->max_steps);
     const uint32_t B = d->batch;
-    std::vector<uint32_t> st(3 * B, 0u);
     for (uint32_t b = 0; b < B; b++) {
         if (tokens0[b] >= d->m.vocab)
             return rt_fail("bdecoder_greedy: token %u >= vocab %u", tokens0[b], d->m.vocab);
         if ((uint64_t)pos0[b] + n > d->m.max_ctx)
             return rt_fail("bdecoder_greedy: sequence %u: context exhausted", b);
-        st[b] = tokens0[b];
-        st[B + b] = pos0[b];
     }
     hipStream_t s = rt_stream();
-    if (!rt_hip_ok(hipMemcpyAsync(d->state, st.data(), st.size() * 4, hipMemcpyHostToDevice, s),
-                   "bdecoder_greedy: state") ||
-        !rt_hip_ok(launch_dequant_rows(d->m.embd_type, (const uint8_t *)d->m.tok_embd, d->state, 0,
-                                       B, d->m.hidden, d->x, s),
-                   "bdecoder_greedy: first embeddings"))
+    if (!rt_hip_ok(launch_decoder_start(d->m.embd_type, tokens0, pos0, B, d->state, d->m.tok_embd,
+                                        d->m.hidden, d->x, s),
+                   "bdecoder_greedy: state and first embeddings"))
         return 0;
     for (uint32_t i = 0; i < n; i++) {
         if (!rt_hip_ok(eager ? enqueue_step_batch(*d, s) : hipGraphLaunch(d->exec, s),
                        "bdecoder_greedy: step"))
             return 0;
     }
-    if (!rt_hip_ok(hipMemcpyAsync(tokens, d->tokens, (size_t)n * B * 4, hipMemcpyDeviceToHost, s),
-                   "bdecoder_greedy: tokens"))
+    Fetch f;
+    f.pinned = (uint8_t *)d->pinned;
+    if (tokens && !rt_hip_ok(f.add(tokens, d->tokens, (size_t)n * B * 4, s), "bdecoder_greedy: tokens"))
         return 0;
-    if (margins &&
-        !rt_hip_ok(hipMemcpyAsync(margins, d->margins, (size_t)n * B * 4, hipMemcpyDeviceToHost, s),
-                   "bdecoder_greedy: margins"))
+    if (margins && !rt_hip_ok(f.add(margins, d->margins, (size_t)n * B * 4, s), "bdecoder_greedy: margins"))
         return 0;
-    if (logits &&
-        !rt_hip_ok(hipMemcpyAsync(logits, d->logits, (size_t)B * d->m.vocab * 4, hipMemcpyDeviceToHost,
-                                  s),
-                   "bdecoder_step: logits"))
+    if (logits && !rt_hip_ok(f.add(logits, d->logits, (size_t)B * d->m.vocab * 4, s), "bdecoder_step: logits"))
         return 0;
-    return rt_hip_ok(hipStreamSynchronize(s), "bdecoder_greedy");
+    return rt_hip_ok(f.finish(s), "bdecoder_greedy");
 }
 
 int vbs_gfx950_bdecoder_greedy(void *handle, const uint32_t *tokens0, const uint32_t *pos0,
@@ -940,8 +1038,7 @@ int vbs_gfx950_bdecoder_step(void *handle, const uint32_t *tokens, const uint32_
                              float *logits) {
     BDecoder *d = (BDecoder *)handle;
     if (!d) return rt_fail("bdecoder_step: null argument");
-    std::vector<uint32_t> next(d->batch);
-    return bdecoder_run(handle, tokens, pos, 1, next.data(), nullptr, false, logits);
+    return bdecoder_run(handle, tokens, pos, 1, nullptr, nullptr, false, logits, true);
 }
 
 int vbs_gfx950_bdecoder_destroy(void *handle) {
