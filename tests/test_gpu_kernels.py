@@ -313,6 +313,40 @@ def test_gate_up_fused_equals_ops_one_by_one(dev, host, mem, t, rows, cols, norm
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), name
 
 
+@pytest.mark.parametrize("t", [V.Q4_K, V.Q6_K], ids=["q4k", "q6k"])
+@pytest.mark.parametrize("rows,cols", [(16, 256), (48, 1280), (4096, 2048), (4112, 2048),
+                                       (272, 2304), (4080, 4096), (32, 4352)])
+def test_small_fused_plans(dev, host, oracle, mem, t, rows, cols):
+    """Gate/up and RMSNorm + matvec at the edges of the one-block-per-wave
+    plan (rows of 1, 8, 9, 16 and 17 blocks, up to and past one workgroup per
+    CU): the bits of the ops one by one, and the matvec
+    within the oracle's tolerance."""
+    eps = 1e-5
+    wg = V.synth_matrix(host, t, rows, cols, SEED, 171)
+    wu = V.synth_matrix(host, t, rows, cols, SEED, 172)
+    x, nw = synth_x(host, cols, 173) * 2.0, synth_x(host, cols, 174)
+    pg, pu, px, pnw = mem.up(wg), mem.up(wu), mem.up(x), mem.up(nw)
+    ref = dict(xn=mem.zeros(cols), gate=mem.zeros(rows), up=mem.zeros(rows), hid=mem.zeros(rows))
+    fus = dict(xn=mem.zeros(cols), gate=mem.zeros(rows), up=mem.zeros(rows), hid=mem.zeros(rows))
+    one = dict(xn=mem.zeros(cols), gate=mem.zeros(rows))
+    dev.rms_norm(px, pnw, ref["xn"], cols, eps)
+    dev.linear(t, pg, ref["xn"], ref["gate"], cols, rows)
+    dev.linear(t, pu, ref["xn"], ref["up"], cols, rows)
+    dev.silu_mul(ref["gate"], ref["up"], ref["hid"], rows)
+    assert dev.gate_up_fused(t, pg, pu, px, cols, rows, pnw, eps, fus["xn"], fus["gate"],
+                             fus["up"], fus["hid"])
+    assert dev.linear_fused(t, pg, px, one["gate"], cols, rows, norm_w=pnw, norm_eps=eps,
+                            x_normed=one["xn"])
+    for got in (fus, one):
+        for name, p in got.items():
+            n = cols if name == "xn" else rows
+            a, b = dev.download(ref[name], n, np.float32), dev.download(p, n, np.float32)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), name
+    xn = dev.download(ref["xn"], cols, np.float32)
+    want = oracle.linear(t, wg, xn, cols, rows, threads=8)
+    assert lin_err(dev.download(fus["gate"], rows, np.float32), want) <= LIN_TOL
+
+
 def test_linear_fused_declines_and_rejects(dev, host, mem):
     """Combinations no fused kernel takes come back as 2 (nothing launched,
     y untouched); half-given neighbours are errors."""

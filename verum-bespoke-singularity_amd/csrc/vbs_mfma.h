@@ -976,10 +976,13 @@ static hipError_t launch_ks(const MvArgs &a, const MvPlan &p, uint32_t wgs, hipS
     }
     // rows of 65-112 blocks (70B down: 112), one tile per workgroup; rows of
     // at most 16 blocks over few tiles, one block per wave
-    if constexpr ((EPI == E_STORE || EPI == E_ACC) && TPW == 1 && !NORM) {
-        if (p.ks == 14u) VBS_MV(14, 512);
+    if constexpr ((EPI == E_STORE || EPI == E_ACC) && TPW == 1) {
+        if constexpr (!NORM)
+            if (p.ks == 14u) VBS_MV(14, 512);
         if (p.ks == 1u) VBS_MV(1, 1024);
     }
+    if constexpr (EPI == E_SILU && TPW == 2)
+        if (p.ks == 1u) VBS_MV(1, 1024);
     if constexpr (EPI == E_QKV) {  // the Q/K/V plans of launch_plan
         if (TPW == 2u && p.ks == 1u) VBS_MV(1, 1024);
         if (TPW == 1u && p.ks == 1u) VBS_MV(1, 1024);
@@ -1004,6 +1007,23 @@ static hipError_t launch_plan(const MvArgs &a, hipStream_t s) {
     if constexpr ((EPI == E_STORE || EPI == E_ACC) && !NORM) {
         const uint32_t nblk = a.cols / 256u;
         if (nblk <= 16u && (total <= 384u || (T::BYTES == 210u && total < 1024u))) {
+            p.ks = 1u;
+            p.nw = nblk;
+        }
+    }
+    // Fused RMSNorm + matvec (rows of at most 8 blocks) and gate/up (at most
+    // 16) over no more workgroups than CUs, as in small models: one block per
+    // wave too. Bound by one wave's serial chain of loads, unpacking and MFMAs:
+    // with two or four items per wave a workgroup runs the spare ones as well.
+    // us of a launch of 1024 rows, before -> after: norm Q4_K x 256 3.1 -> 2.7,
+    // x 2048 3.3 -> 3.1, x 4096 4.1 -> 4.7 (hence 8; Q6_K x 2048 4.5 -> 4.0,
+    // x 4096 equal); gate/up Q4_K x 256 4.8 -> 3.1, x 2048 5.3 -> 3.4, x 4096
+    // 5.5 -> 5.4, Q6_K x 256 7.6 -> 4.0, x 4096 9.5 -> 7.5. Past one workgroup
+    // per CU the launch is bound by the weight stream, which wants the longer
+    // queue of loads per wave.
+    if constexpr ((EPI == E_STORE && NORM) || EPI == E_SILU) {
+        const uint32_t nblk = a.cols / 256u, wgs = EPI == E_SILU ? a.tile_end[0] : total;
+        if (nblk <= (EPI == E_SILU ? 16u : 8u) && wgs <= device_cus()) {
             p.ks = 1u;
             p.nw = nblk;
         }
