@@ -313,6 +313,22 @@ def test_gate_up_fused_equals_ops_one_by_one(dev, host, mem, t, rows, cols, norm
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), name
 
 
+@pytest.mark.parametrize("t", [V.Q4_0, V.Q4_1], ids=["q4_0", "q4_1"])
+@pytest.mark.parametrize("rows,cols", [(1, 8448), (4096, 8448), (4097, 8448), (33, 12288),
+                                       (33, 8192), (33, 12544)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_nibble_block_wave_split(dev, host, oracle, mem, t, rows, cols, accumulate):
+    """Q4_0 and Q4_1 at the edges of the four-blocks-per-wave plan: rows of
+    32, 33, 48 and 49 units of 256 columns, up to and past a tile per CU."""
+    w, x = V.synth_matrix(host, t, rows, cols, SEED, 181), synth_x(host, cols, 182)
+    y0 = synth_x(host, rows, 183)
+    y = mem.up(y0)
+    dev.linear(t, mem.up(w), mem.up(x), y, cols, rows, accumulate=accumulate)
+    want = oracle.linear(t, w, x, cols, rows, y=y0.copy() if accumulate else None,
+                         accumulate=accumulate, threads=8)
+    assert lin_err(dev.download(y, rows, np.float32), want) <= LIN_TOL
+
+
 @pytest.mark.parametrize("t", [V.Q4_K, V.Q6_K], ids=["q4k", "q6k"])
 @pytest.mark.parametrize("rows,cols", [(16, 256), (48, 1280), (4096, 2048), (4112, 2048),
                                        (272, 2304), (4080, 4096), (32, 4352)])

@@ -1011,6 +1011,20 @@ static hipError_t launch_plan(const MvArgs &a, hipStream_t s) {
             p.nw = nblk;
         }
     }
+    // Q4_0 and Q4_1 rows of 33-48 blocks over at most one tile per CU: four
+    // blocks on nine to twelve waves instead of six on eight, since one wave's chain of
+    // unpacking bounds it (us, weights from HBM, before -> after: Q4_0 4096 x
+    // 11008 9.82 -> 9.35, 4096 x 9216 9.36 -> 8.85, 1000 x 11008 8.68 -> 8.09,
+    // 2048 x 12288 9.49 -> 8.92, Q4_1 2 to 7% as well). With more tiles the
+    // smaller workgroups overlap better (Q4_0 5120 x 10240 13.6 against 14.5),
+    // as for Q8_0 at any count (4096 x 11008 13.4 against 13.6).
+    if constexpr (T::SCRATCH != 0u && T::BYTES <= 160u) {
+        const uint32_t nblk = a.cols / 256u;
+        if (nblk > 32u && nblk <= 48u && total <= device_cus()) {
+            p.ks = 4u;
+            p.nw = (nblk + 3u) / 4u;
+        }
+    }
     // Fused RMSNorm + matvec (rows of at most 8 blocks) and gate/up (at most
     // 16) over no more workgroups than CUs, as in small models: one block per
     // wave too. Bound by one wave's serial chain of loads, unpacking and MFMAs:
