@@ -758,6 +758,44 @@ def test_attention_chunk_limits(dev, host, oracle, mem, hd, nqh, nkh, seq):
     assert np.max(np.abs(got)) <= 1.001 * np.max(np.abs(vc.view(np.float16).astype(np.float32)))
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96])
+@pytest.mark.parametrize("nqh,nkh", [(4, 2), (8, 1), (35, 5)])
+@pytest.mark.parametrize("seq", [1, 41, 250, 300, 4500])
+@pytest.mark.parametrize("what", ["key", "value", "last_value", "nan_key"])
+def test_attention_non_finite_cache(dev, host, oracle, mem, hd, nqh, nkh, seq, what):
+    """Cache entries that the f16 store rounded to inf, and NaN: a -inf score
+    weighs nothing and leaves the head finite, a +inf or NaN score makes it
+    NaN, an infinite value of positive weight gives inf in its dim. In one
+    launch and over several chunks, also at the last position, which fills the
+    tile's idle positions: the oracle's NaN, inf and finite outputs."""
+    max_ctx, layer, kvd, inf = seq + 5, 1, nkh * hd, 0x7C00
+    kc = V.synth_normal_f16(host, 2 * max_ctx * kvd, SEED, 161)
+    vc = V.synth_normal_f16(host, 2 * max_ctx * kvd, SEED, 162)
+    k, v = (c.reshape(2, max_ctx, nkh, hd)[layer] for c in (kc, vc))
+    q = synth_x(host, nqh * hd, 163)
+    if what == "key":
+        k[seq // 3, :, 5] = 0x8000 | inf
+        k[seq // 2, 0, hd - 1] = inf
+    elif what == "value":
+        v[seq // 3, :, 3] = inf
+        v[seq // 2, 0, hd - 2] = 0x8000 | inf
+        v[0, nkh - 1, 9] = 0x7E00
+    elif what == "last_value":
+        v[seq - 1, :, [0, hd - 1]] = inf
+    else:
+        k[seq // 2, 0, 7] = 0x7E00
+    scale = np.float32(1.0 / math.sqrt(hd))
+    po = mem.zeros(nqh * hd)
+    dev.attention(mem.up(q), mem.up(kc), mem.up(vc), po, seq, layer, max_ctx, nqh, nkh, hd, scale)
+    got = dev.download(po, nqh * hd, np.float32)
+    want = oracle.attention(q, kc, vc, seq, layer, max_ctx, nqh, nkh, hd, scale)
+    assert not np.all(np.isfinite(want))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fine = np.isfinite(want)
+    assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-4 * np.abs(want[fine]))
+
+
 @pytest.mark.parametrize("qscale", [1e-6, 1e4])
 def test_attention_q_magnitude(dev, host, oracle, mem, qscale):
     """q far from unit scale (the matrix-core kernel rescales each head's q

@@ -418,6 +418,112 @@ __device__ __forceinline__ void attn_mfma_store(float *pk, uint32_t stride, uint
     }
 }
 
+// The heads of a chunk whose sums are not finite once more, whole (head sizes
+// but 128): an infinite score or value meets the hi and lo halves as inf - inf
+// or 0 * inf. Here, as in the sequential softmax, -inf scores weigh 0, +inf and
+// NaN give NaN, and an infinite value of positive weight gives inf. Scores are
+// double dots, a lane per position; values a lane per DPL dims. m, l, a: what
+// attn_mfma_store has just stored. The test hides behind those stores (under 1%
+// of a launch); a head taken again costs about 2.5 us per 64 positions of a chunk.
+template <uint32_t HD>
+__device__ __forceinline__ void attn_heads_again(const float *__restrict__ q, const uint16_t *__restrict__ kc,
+                                                 const uint16_t *__restrict__ vc, uint64_t layer_off, uint32_t s0,
+                                                 uint32_t valid, uint32_t nkh, uint32_t kvh, uint32_t group,
+                                                 float scale, uint32_t lane, float *pk, uint32_t stride,
+                                                 uint32_t chunk, float l0, const float (&a)[HD / 16][4]) {
+    constexpr uint32_t DPL = HD / 16u, NP = kMfmaLmax / 64u;  // positions per lane
+    const uint32_t n = lane & 15u, g = lane >> 4;
+    float t[4] = {0.f, 0.f, 0.f, 0.f};  // NaN where a head's sums are not finite
+#pragma unroll
+    for (uint32_t dt = 0; dt < DPL; dt++)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) t[r] = fmaf(a[dt][r], 0.f, t[r]);
+    if (__builtin_expect(!__ballot(fmaf(l0, 0.f, (t[0] + t[1]) + (t[2] + t[3])) != 0.f), 1)) return;
+    const uint64_t rstride = (uint64_t)nkh * HD, base = layer_off + (uint64_t)s0 * rstride + (uint64_t)kvh * HD;
+#pragma unroll 1
+    for (uint32_t hh = 0; hh < group; hh++) {
+        bool bad = (n & 7u) == hh && !(fabsf(l0) <= 3.4028235e38f);
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) bad |= 4u * (g & 1u) + r == hh && t[r] != 0.f;
+        if (!__ballot(bad)) continue;
+        const float *qh = q + ((uint64_t)kvh * group + hh) * HD;
+        float sc[NP], e[NP], mt = -INFINITY, l = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < NP; i++) {
+            const uint32_t p = lane + 64u * i;
+            double d = 0.0;
+            if (64u * i < valid) {
+                const uint16_t *kr = kc + base + (uint64_t)min(p, valid - 1u) * rstride;
+#pragma unroll
+                for (uint32_t c = 0; c < HD; c += 8u) {
+                    const au4 kw = *reinterpret_cast<const au4 *>(kr + c);
+#pragma unroll
+                    for (uint32_t k = 0; k < 8u; k++)
+                        d = fma((double)qh[c + k], (double)hcvt(kw[k >> 1] >> (16u * (k & 1u))), d);
+                }
+            }
+            sc[i] = p < valid ? __fmul_rn((float)d, scale) : -INFINITY;
+            mt = fmaxf(mt, __fmul_rn(sc[i], 1.44269504088896341f));
+        }
+        const float mn = ceilf(wave_max(mt));  // (a whole power of two, as attn_mfma_wave's)
+#pragma unroll
+        for (uint32_t i = 0; i < NP; i++) {
+            const float p = __fmul_rn(sc[i], 1.44269504088896341f), r = rintf(p);
+            const float err = fmaf(sc[i], 1.92596299e-8f, fmaf(sc[i], 1.44269504088896341f, -p));
+            e[i] = ldexpf(exp2_fast((p - r) + __builtin_amdgcn_fmed3f(err, -0.5f, 0.5f)), (int)(r - mn));
+            if (sc[i] == -INFINITY) e[i] = 0.f;
+            l += e[i];
+        }
+        l = wave_sum(l);
+        float o[DPL];
+#pragma unroll
+        for (uint32_t dt = 0; dt < DPL; dt++) o[dt] = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < NP; i++)
+            for (uint32_t p0 = 64u * i; p0 < min(valid, 64u * (i + 1u)); p0 += 8u) {
+                uint16_t vr[8][DPL];  // (eight rows requested at a time)
+#pragma unroll
+                for (uint32_t k = 0; k < 8u; k++)
+#pragma unroll
+                    for (uint32_t dt = 0; dt < DPL; dt++)
+                        vr[k][dt] = vc[base + (uint64_t)min(p0 + k, valid - 1u) * rstride + DPL * n + dt];
+#pragma unroll
+                for (uint32_t k = 0; k < 8u; k++) {
+                    const float w = __shfl(e[i], (int)((p0 + k) & 63u), 64);
+                    if (p0 + k < valid) {
+#pragma unroll
+                        for (uint32_t dt = 0; dt < DPL; dt++) o[dt] = fmaf(w, hcvt(vr[k][dt]), o[dt]);
+                    }
+                }
+            }
+        // (by the lanes that stored the head's row before)
+        float *dst = pk + ((uint64_t)hh * stride + chunk) * part_row<HD>;
+        if (g == hh >> 2) {
+#pragma unroll
+            for (uint32_t i = 0; i < DPL / 2u; i++)
+                reinterpret_cast<float2 *>(dst + 2u + DPL * n)[i] = make_float2(o[2 * i], o[2 * i + 1]);
+        }
+        if (g == 0u && n == hh) {
+            dst[0] = mn;
+            dst[1] = l;
+        }
+    }
+}
+
+// A chunk from its positions to its partials row.
+template <uint32_t HD>
+__device__ __forceinline__ void attn_mfma_chunk(const float *__restrict__ q, const uint16_t *__restrict__ kc,
+                                                const uint16_t *__restrict__ vc, uint64_t layer_off, uint32_t s0,
+                                                uint32_t valid, uint32_t nt, uint32_t nkh, uint32_t kvh,
+                                                uint32_t group, float scale, uint32_t lane, float *pk,
+                                                uint32_t stride, uint32_t chunk) {
+    float m, l, a[HD / 16][4];
+    attn_mfma_wave<HD>(q, kc, vc, layer_off, s0, valid, nt, nkh, kvh, group, scale, lane, m, l, a);
+    attn_mfma_store<HD>(pk, stride, chunk, group, lane, m, l, a);
+    if constexpr (HD != 128u)
+        attn_heads_again<HD>(q, kc, vc, layer_off, s0, valid, nkh, kvh, group, scale, lane, pk, stride, chunk, l, a);
+}
+
 template <uint32_t HD>
 __global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
                                                   const uint16_t *__restrict__ kc,
@@ -443,11 +549,8 @@ __global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
     const AttnSplit sp = attn_split(seq_len, nkh, kMfmaGran, kMfmaLmax, target);
     if (chunk >= sp.n) return;  // past the sequence (the grid covers the longest split)
     const uint32_t s0 = chunk * sp.len, valid = min(sp.len, seq_len - s0);
-    float m, l, a[HD / 16][4];
-    attn_mfma_wave<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale,
-                   lane, m, l, a);
-    attn_mfma_store<HD>(part + (uint64_t)kvh * group * stride_chunks * part_row<HD>, stride_chunks, chunk,
-                        group, lane, m, l, a);
+    attn_mfma_chunk<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane,
+                        part + (uint64_t)kvh * group * stride_chunks * part_row<HD>, stride_chunks, chunk);
 }
 
 // Short sequences (at most kOneChunks chunks) in one launch: workgroup kvh
@@ -467,10 +570,8 @@ __global__ __launch_bounds__(64 * kOneChunks) void k_attn_one(
     const AttnSplit sp = attn_split(seq_len, nkh, kMfmaGran, kMfmaLmax, kMfmaTargetWgs);
     if (wave < sp.n) {
         const uint32_t s0 = wave * sp.len, valid = min(sp.len, seq_len - s0);
-        float m, l, a[HD / 16][4];
-        attn_mfma_wave<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane,
-                           m, l, a);
-        attn_mfma_store<HD>(part, kOneChunks, wave, group, lane, m, l, a);
+        attn_mfma_chunk<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane, part,
+                            kOneChunks, wave);
     }
     __syncthreads();
     for (uint32_t h = wave; h < group; h += nw) {
