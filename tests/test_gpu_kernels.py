@@ -700,6 +700,27 @@ def test_general_linear(dev, host, oracle, mem, t, rows, cols, batch):
     assert lin_err(dev.download(py, rows, np.float32), y0 + want[0]) <= LIN_TOL
 
 
+@pytest.mark.parametrize("t,base", [(V.Q4_K, 2), (V.Q4_K, 8), (V.Q6_K, 1), (V.Q4_K, 0), (V.Q6_K, 0)],
+                         ids=["q4k_base2", "q4k_base8", "q6k_base1", "q4k", "q6k"])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (513, 768), (3074, 2304), (6, 33024)])
+@pytest.mark.parametrize("batch", [1, 3, 9])
+def test_general_linear_kquants(dev, host, oracle, mem, t, base, rows, cols, batch):
+    """K-quant matrices that the matrix-core kernels do not take (a base off
+    their alignment, rows past 32768 columns) on the general kernel: every
+    sub-block of a block, scales from both halves of the packed scale bytes."""
+    w = V.synth_matrix(host, t, rows, cols, SEED, 191)
+    X = np.stack([synth_x(host, cols, 192 + b) for b in range(batch)])
+    pw = mem.up(np.concatenate([np.zeros(base, np.uint8), w.reshape(-1), np.zeros(16, np.uint8)])) + base
+    py = mem.zeros(batch * rows)
+    if batch == 1:
+        dev.linear(t, pw, mem.up(X), py, cols, rows)
+    else:
+        dev.linear_batch(t, pw, mem.up(X), cols, py, rows, cols, rows, batch)
+    got = dev.download(py, (batch, rows), np.float32)
+    for b in range(batch):
+        assert lin_err(got[b], oracle.linear(t, w, X[b], cols, rows, threads=8)) <= LIN_TOL, b
+
+
 def _attention_draws(n=12, seed=SEED + 6):
     rng = np.random.default_rng(seed)
     out = []
