@@ -700,6 +700,33 @@ def test_general_linear(dev, host, oracle, mem, t, rows, cols, batch):
     assert lin_err(dev.download(py, rows, np.float32), y0 + want[0]) <= LIN_TOL
 
 
+@pytest.mark.parametrize("t", [V.Q4_0, V.Q8_0, V.F16, V.F32, V.LNS8], ids=lambda t: V.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols", [(3, 32), (3075, 64), (513, 96), (512, 512), (3072, 480), (3073, 512),
+                                       (3072, 1056), (40, 2080), (6147, 96)])
+@pytest.mark.parametrize("batch", [1, 2, 3, 8, 13])
+def test_general_linear_short_rows(dev, host, oracle, mem, t, rows, cols, batch):
+    """Rows of at most four 512-element steps, on both sides of each limit of
+    the split (64, 512, 1024 and 2048 elements; 512 and 3072 rows; 2, 4, 8 and
+    16 sums per row), and one element past for F16 and F32."""
+    cols += t in (V.F16, V.F32) and rows % 3 == 0
+    if t == V.LNS8:
+        rng = np.random.default_rng(SEED)
+        w = rng.integers(0, 12, size=(rows, cols // 32, 36), dtype=np.uint8)
+        w[:, :, 32:36] = rng.random((rows, cols // 32, 1), np.float32).view(np.uint8)
+        w = w.reshape(rows, -1)
+    else:
+        w = V.synth_matrix(host, t, rows, cols, SEED, 201)
+    X = np.stack([synth_x(host, cols, 202 + b) for b in range(batch)])
+    py = mem.zeros(batch * rows)
+    if batch == 1:
+        dev.linear(t, mem.up(w), mem.up(X), py, cols, rows)
+    else:
+        dev.linear_batch(t, mem.up(w), mem.up(X), cols, py, rows, cols, rows, batch)
+    got = dev.download(py, (batch, rows), np.float32)
+    for b in range(batch):
+        assert lin_err(got[b], oracle.linear(t, w, X[b], cols, rows)) <= LIN_TOL, b
+
+
 @pytest.mark.parametrize("t,base", [(V.Q4_K, 2), (V.Q4_K, 8), (V.Q6_K, 1), (V.Q4_K, 0), (V.Q6_K, 0)],
                          ids=["q4k_base2", "q4k_base8", "q6k_base1", "q4k", "q6k"])
 @pytest.mark.parametrize("rows,cols", [(1, 256), (513, 768), (3074, 2304), (6, 33024)])

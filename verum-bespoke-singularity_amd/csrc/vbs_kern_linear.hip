@@ -185,6 +185,42 @@ template <> struct Row8<kF32> {
     }
 };
 
+// The value that lane l ^ M holds.
+template <uint32_t M>
+__device__ __forceinline__ float xor_lane(float v) {
+    if constexpr (M >= 16u) {
+        return lane_xor<(int)M>(v);
+    } else if constexpr (M == 4u) {  // (lanes of even quads from above, of odd ones from below)
+        const int i = __builtin_bit_cast(int, v);
+        const int t = __builtin_amdgcn_update_dpp(0, i, 0x104, 0xF, 0x5, false);
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(t, i, 0x114, 0xF, 0xA, false));
+    } else {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                     M == 8u ? 0x128 : M == 2u ? 0x4E : 0xB1, 0xF, 0xF,
+                                                                     false));
+    }
+}
+// wave_sum of each of N values (a power of two), bit for bit: every lane of the
+// k-th group of 64 / N gets the k-th sum. Each step halves the values a lane
+// carries, so N of them take about 2 N exchanges instead of 6 N.
+template <uint32_t N, uint32_t M = 32>
+__device__ __forceinline__ float wave_sums(const float (&v)[N], uint32_t lane) {
+    if constexpr (M == 0u) {
+        return v[0];
+    } else if constexpr (N == 1u) {
+        const float t[1] = {v[0] + xor_lane<M>(v[0])};
+        return wave_sums<1u, M / 2u>(t, lane);
+    } else {
+        float t[N / 2u];
+#pragma unroll
+        for (uint32_t i = 0; i < N / 2u; i++) {
+            const float own = lane & M ? v[i + N / 2u] : v[i], send = lane & M ? v[i] : v[i + N / 2u];
+            t[i] = own + xor_lane<M>(send);
+        }
+        return wave_sums<N / 2u, M / 2u>(t, lane);
+    }
+}
+
 // R rows and NB vectors per group of S waves (S = 1: every wave has rows of its
 // own; else the workgroup's S waves split the row's steps and add their sums
 // in wave order). A step is 512 elements of a row; U steps' loads go out
@@ -205,11 +241,17 @@ __global__ __launch_bounds__(S > 4 ? 64 * S : 256) void k_rows(const uint8_t *__
                                                                uint32_t batch, int accumulate) {
     typedef Row8<T> P;
     constexpr uint32_t kWaves = S > 4u ? S : 4u, kGroups = kWaves / S, L = P::E / 8u;  // lanes per block
+    // rows on one wave (short ones): all NB vectors are formed, without a branch
+    // between their loads; those past the batch repeat its last and are dropped
+        constexpr bool kAll = NB > 1u && R <= 2u && S == 1u;
+
     __shared__ float red[S > 1 ? kWaves : 1][R * NB];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t part = S > 1u ? wave % S : 0u;
     const uint32_t row0 = (blockIdx.x * kGroups + (S > 1u ? wave / S : wave)) * R;
-    const uint32_t q = lane % L, nu = cols / P::E;  // whole blocks (cols of F16 / F32 may have a tail)
+    // whole blocks; cols of F16 / F32 may have a tail (rows of at most 64 elements
+    // are all tail: a lane per element)
+    const uint32_t q = lane % L, nu = P::E == 8u && cols <= 64u ? 0u : cols / P::E;
     const uint8_t *rp[R];
 #pragma unroll
     for (uint32_t r = 0; r < R; r++) rp[r] = w + (uint64_t)min(row0 + r, rows - 1u) * rb;
@@ -242,12 +284,12 @@ __global__ __launch_bounds__(S > 4 ? 64 * S : 256) void k_rows(const uint8_t *__
                 for (uint32_t r = 0; r < R; r++) P::value(raw[k][r], wv[r]);
 #pragma unroll
                 for (uint32_t b = 0; b < NB; b++) {
-                    if (NB > 1u && b >= batch) break;  // (uniform)
+                    if (NB > 1u && !kAll && b >= batch) break;  // (uniform)
                     v4f a, c;
                     if constexpr (NB == 1u) {
                         a = xa[k], c = xb[k];
                     } else {
-                        const float *xp = x + (uint64_t)b * xs + P::E * u;
+                        const float *xp = x + (uint64_t)(kAll ? min(b, batch - 1u) : b) * xs + P::E * u;
                         a = *reinterpret_cast<const f4u *>(xp + P::lo(q));
                         c = *reinterpret_cast<const f4u *>(xp + P::hi(q));
                     }
@@ -262,40 +304,37 @@ __global__ __launch_bounds__(S > 4 ? 64 * S : 256) void k_rows(const uint8_t *__
                 }
             }
         }
-        if (P::E == 8u && part == 0u) {  // the tail of F16 / F32 rows: up to seven elements
+        if (P::E == 8u && part == 0u) {  // the tail of F16 / F32 rows
             const uint32_t c = 8u * nu + lane;
-            if (lane < 8u && c < cols) {
+            if (c < cols) {
+                float wv[R];
 #pragma unroll
-                for (uint32_t r = 0; r < R; r++)
+                for (uint32_t r = 0; r < R; r++) wv[r] = deq_elem<T>(rp[r], c);
 #pragma unroll
-                    for (uint32_t b = 0; b < NB; b++)
-                        if (NB == 1u || b < batch)
-                            acc[r][b] = fmaf(deq_elem<T>(rp[r], c), x[(uint64_t)b * xs + c], acc[r][b]);
+                for (uint32_t b = 0; b < NB; b++) {
+                    if (NB > 1u && !kAll && b >= batch) break;
+                    const float xv = x[(uint64_t)(kAll ? min(b, batch - 1u) : b) * xs + c];
+#pragma unroll
+                    for (uint32_t r = 0; r < R; r++) acc[r][b] = fmaf(wv[r], xv, acc[r][b]);
+                }
             }
         }
     }
-    // row r of vector b ends in lane r NB + b (R NB <= 64), or in LDS first
-    float mine = 0.f;
+    // row r of vector b ends in the lanes of group r NB + b (R NB <= 64), or in LDS first
+    float v[R * NB];
 #pragma unroll
-    for (uint32_t r = 0; r < R; r++)
-#pragma unroll
-        for (uint32_t b = 0; b < NB; b++) {
-            if (NB > 1u && b >= batch) break;
-            const float t = wave_sum(acc[r][b]);
-            if (S > 1u) {
-                if (lane == 0u) red[wave][r * NB + b] = t;
-            } else if (lane == r * NB + b) {
-                mine = t;
-            }
-        }
+    for (uint32_t k = 0; k < R * NB; k++) v[k] = acc[k / NB][k % NB];
+    float mine = wave_sums<R * NB>(v, lane);
+    constexpr uint32_t kGroup = 64u / (R * NB);
+    const uint32_t k = lane / kGroup, r = k / NB, b = k % NB;
     if (S > 1u) {
+        if (lane % kGroup == 0u) red[wave][k] = mine;
         __syncthreads();
         if (part != 0u) return;
-        if (lane < R * NB)
-            for (uint32_t k = 0; k < S; k++) mine += red[wave + k][lane];
+        mine = 0.f;
+        for (uint32_t i = 0; i < S; i++) mine += red[wave + i][k];
     }
-    const uint32_t r = lane / NB, b = lane % NB;
-    if (lane < R * NB && row0 + r < rows && b < batch) {
+    if (lane % kGroup == 0u && row0 + r < rows && b < batch) {
         float *dst = y + (uint64_t)b * ys + row0 + r;
         *dst = accumulate ? *dst + mine : mine;
     }
@@ -318,22 +357,48 @@ hipError_t launch_rows_t(const uint8_t *w, const float *x, uint32_t xs, float *y
 // (32000 x 1056 Q4_0 12.0 us against 14.6). Several vectors alike: 4, 16 vectors,
 // F32 256 x 4128 4.1, 7.3 us (a wave per row 10.5, 24.8), 1000 x 10528 13.5, 38.7
 // (29.1, 100), 11008 x 4128 42.1, 115 (55.9, 147).
+// Rows of no more steps than that split has waves leave waves idle, so short
+// rows take fewer: one wave at a step (512 elements; two for one vector and
+// 513-3072 rows), two rows a wave past 3072 rows, with as many sums as there are
+// vectors (us, before the split went by length -> now: F32 32000 x 32, 16 vectors
+// 99.9 -> 9.4, x 256 104 -> 24.1, 5000 x 96, 8 vectors 11.8 -> 4.2; Q4_0 512 x 96
+// one vector 2.69 -> 2.27, 1000 x 544 2.92 -> 2.56; one and four rows a wave
+// at 32000 x 256 F32, 8 vectors 24.9 and 17.0, two 16.7), four at up to four
+// steps of few rows (512 x 1024 F32, 16 vectors 7.2 -> 4.7; one wave 7.2).
 template <int T>
 hipError_t launch_rows(const uint8_t *w, const float *x, uint32_t xs, float *y, uint32_t ys, uint32_t cols,
                        uint32_t rows, uint32_t batch, int accumulate, hipStream_t s) {
 #define VBS_ROWS(R, NB, S, U) \
     return launch_rows_t<T, R, NB, S, U>(w, x, xs, y, ys, cols, rows, batch, accumulate, s)
     if (batch == 1u) {
+        if (cols <= (rows <= 512u ? 512u : rows <= 3072u ? 1024u : 0u)) VBS_ROWS(1, 1, 1, 1);
+        if (rows <= 512u && cols <= 2048u) VBS_ROWS(1, 1, 4, 1);
         if (rows <= 512u) VBS_ROWS(1, 1, 16, 1);
+        if (rows <= 3072u && cols <= 2048u) VBS_ROWS(2, 1, 4, 1);
         if (rows <= 3072u) VBS_ROWS(2, 1, 4, 2);
+        if (cols <= 512u) VBS_ROWS(2, 1, 1, 1);
         if (cols < 2048u) VBS_ROWS(4, 1, 1, 1);
         VBS_ROWS(4, 1, 4, 1);
     }
+    if (cols <= 512u) {
+        if (rows <= 3072u) {
+            if (batch == 2u) VBS_ROWS(1, 2, 1, 1);
+            if (batch <= 4u) VBS_ROWS(1, 4, 1, 1);
+            if (batch <= 8u) VBS_ROWS(1, 8, 1, 1);
+            VBS_ROWS(1, 16, 1, 1);
+        }
+        if (batch == 2u) VBS_ROWS(2, 2, 1, 1);
+        if (batch <= 4u) VBS_ROWS(2, 4, 1, 1);
+        if (batch <= 8u) VBS_ROWS(2, 8, 1, 1);
+        VBS_ROWS(2, 16, 1, 1);
+    }
     if (batch <= 4u) {
+        if (rows <= 512u && cols <= 2048u) VBS_ROWS(1, 4, 4, 1);
         if (rows <= 512u) VBS_ROWS(1, 4, 16, 1);
         if (rows <= 3072u) VBS_ROWS(2, 4, 4, 1);
         VBS_ROWS(4, 4, 1, 1);
     }
+    if (rows <= 512u && cols <= 2048u) VBS_ROWS(1, 16, 4, 1);
     if (rows <= 512u) VBS_ROWS(1, 16, 16, 1);
     VBS_ROWS(2, 16, 4, 1);
 #undef VBS_ROWS
