@@ -118,6 +118,25 @@ def test_hot_matvec_tile_edges(dev, host, orc, t, rows, cols):
         assert same_bits(got, orc.hot_matvec(t, w, rows, c, xq, qd, qs, x[:c].copy())), c
 
 
+@pytest.mark.parametrize("t", [V.Q8_0, V.Q4_0, V.Q4_1], ids=["Q8_0", "Q4_0", "Q4_1"])
+@pytest.mark.parametrize("rows,cols", [(1, 64), (7, 480), (6, 512), (5, 544), (9, 992), (3, 1024), (2, 1056)])
+def test_hot_matvec_few_blocks(dev, host, orc, t, rows, cols):
+    """Rows of one to three 16-block steps, whole and partly filled, also of
+    terms that are all zero, with an infinite scale or a NaN one."""
+    w = V.synth_matrix(host, t, rows, cols, 95 + t, 1)
+    w[0, :2] = np.array([0x8000], np.uint16).view(np.uint8)
+    if rows > 2:
+        w[1, -V.GEOMETRY[t][1]:][:2] = np.array([0x7C00], np.uint16).view(np.uint8)
+        w[2, :2] = np.array([0x7E01], np.uint16).view(np.uint8)
+    x = edge_activations(host, cols, 96 + t)
+    xq, qd, qs = orc.quantize_q8(x)
+    got = dev_hot(dev, t, w, rows, cols, xq, qd, qs, x)
+    want = orc.hot_matvec(t, w, rows, cols, xq, qd, qs, x)
+    fine = ~np.isnan(want)
+    assert np.array_equal(np.isnan(got), ~fine)
+    assert same_bits(got[fine], want[fine])
+
+
 @pytest.mark.parametrize("t", [V.F32, V.F16], ids=["F32", "F16"])
 def test_hot_matvec_ragged_float_rows(dev, host, orc, t):
     rows, cols = 9, 1000  # F32 / F16 rows need not be whole blocks

@@ -66,6 +66,10 @@ __device__ __forceinline__ float add_in_order(float sum, const float *t, uint32_
     return sum;
 }
 
+__device__ __forceinline__ float lane_f(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
 // f16 bits -> f32: the hardware's conversion but for inf and NaN (h2f's bits).
 __device__ __forceinline__ float hot_h2f(uint16_t h) {
     const float v = (float)__builtin_bit_cast(_Float16, h);
@@ -75,14 +79,17 @@ __device__ __forceinline__ float hot_h2f(uint16_t h) {
 // Block types: a row per wave, four rows per workgroup, so that the sums of
 // some workgroups run under the loads of others. A lane takes a quarter of a
 // block (as k_rows, vbs_kern_linear.hip), sixteen blocks per step, the quads
-// add their integer dots, and kHotBlocks blocks' terms at a time wait in LDS.
+// add their integer dots, and kHotBlocks blocks' terms at a time wait in LDS;
+// rows of one or two steps (REG) need no LDS and no barrier: the wave adds its
+// row's terms from the lanes that hold them, those past the row as +0, which
+// leaves a sum that began at +0 its bits.
 // Bound: the loads' latency, then HBM. Q8_0 4096 x 4096 10.2 -> 7.6 us (2.3
 // TB/s), 1000 x 11008 17.9 -> 7.9, Q4_0 4096 x 4096 9.2 -> 6.2, Q4_1 11008 x 4096
 // 26.2 -> 11.1 against the kernel before, which took a whole block per lane, in
 // 2-byte pieces, and added every term on all lanes through lane reads.
 constexpr uint32_t kHotBlocks = 512;
 
-template <int K, uint32_t U>
+template <int K, uint32_t U, bool REG>
 __global__ __launch_bounds__(256) void k_hot_blocks(const uint8_t *__restrict__ w, uint32_t rows,
                                                     uint32_t nblk, const int8_t *__restrict__ xq,
                                                     const float *__restrict__ qd,
@@ -91,7 +98,7 @@ __global__ __launch_bounds__(256) void k_hot_blocks(const uint8_t *__restrict__ 
     constexpr uint32_t kBytes = K == HK_Q8_0 ? 34u : K == HK_Q4_0 ? 18u : 20u;
     constexpr uint32_t N = K == HK_Q4_1 ? 2u : 1u;  // terms per block
     constexpr uint32_t kSize = kHotBlocks * N;
-    __shared__ __align__(16) float terms[4][kSize + 4u];
+    __shared__ __align__(16) float terms[REG ? 1 : 4][REG ? 4 : kSize + 4u];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, q = lane & 3u;
     const uint32_t row = blockIdx.x * 4u + wave;
     const uint8_t *const rp = w + (uint64_t)min(row, rows - 1u) * nblk * kBytes;
@@ -143,17 +150,32 @@ __global__ __launch_bounds__(256) void k_hot_blocks(const uint8_t *__restrict__ 
                 dot = dpp_add_i<0xB1>(dot);  // the block's four lanes
                 dot = dpp_add_i<0x4E>(dot);
                 const float t0 = __fmul_rn(__fmul_rn(hot_h2f(d[k]), xd[k]), (float)dot);
-                if (q == 0u && b < n) {
+                if constexpr (REG) {
+                    if (16u * k >= n) break;
+                    float t1 = 0.0f;
+                    if constexpr (K == HK_Q4_1) t1 = b < n ? __fmul_rn(hot_h2f(m[k]), xs[k]) : 0.0f;
+                    const float t = b < n ? t0 : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        sum = __fadd_rn(sum, lane_f(t, 4 * i));
+                        if constexpr (K == HK_Q4_1) sum = __fadd_rn(sum, lane_f(t1, 4 * i));
+                    }
+                } else if (q == 0u && b < n) {
                     terms[wave][N * b] = t0;
                     if constexpr (K == HK_Q4_1) terms[wave][2u * b + 1u] = __fmul_rn(hot_h2f(m[k]), xs[k]);
                 }
             }
         }
+        if constexpr (REG) break;
         __syncthreads();
         if (threadIdx.x < 4u) sum = add_in_order(sum, terms[threadIdx.x], N * n, kSize);
         if (c0 + kHotBlocks < nblk) __syncthreads();
     }
-    if (threadIdx.x < 4u && blockIdx.x * 4u + threadIdx.x < rows) y[blockIdx.x * 4u + threadIdx.x] = sum;
+    if constexpr (REG) {
+        if (lane == 0u && row < rows) y[row] = sum;
+    } else if (threadIdx.x < 4u && blockIdx.x * 4u + threadIdx.x < rows) {
+        y[blockIdx.x * 4u + threadIdx.x] = sum;
+    }
 }
 
 // F32 and F16: a term per element, so a row's sum is a chain of `cols` adds
@@ -216,10 +238,14 @@ __global__ __launch_bounds__(320) void k_hot_float(const uint8_t *__restrict__ w
                     }
                     load(min(t + kHotAhead, full - 1u), wv[k], xv[k]);
                 } else if (t < tiles) {
-                    for (uint32_t e = lane; e < tail; e += 64u)
-                        for (uint32_t r = 0; r < 4u; r++)
-                            terms[t & 1u][mr + r][e] =
-                                __fmul_rn(value(rp[r][t * kHotCols + e]), x[t * kHotCols + e]);
+                    for (uint32_t e = lane; e < tail; e += 64u) {
+                        const float xe = x[t * kHotCols + e];
+                        E v[4];
+#pragma unroll
+                        for (uint32_t r = 0; r < 4u; r++) v[r] = rp[r][t * kHotCols + e];
+#pragma unroll
+                        for (uint32_t r = 0; r < 4u; r++) terms[t & 1u][mr + r][e] = __fmul_rn(value(v[r]), xe);
+                    }
                 }
             } else if (t > 0u && lane < kHotRows) {
                 sum = add_in_order(sum, terms[(t - 1u) & 1u][lane], t <= full ? kHotCols : tail, kHotCols);
@@ -317,20 +343,24 @@ int vbs_gfx950_hot_matvec(int type, const void *w, uint32_t rows, uint32_t cols,
         const dim3 grid((rows + 3u) / 4u), block(256);
         const int8_t *xq = static_cast<const int8_t *>(act);
         // loads of U steps of 16 blocks together: no more than short rows have (16000
-        // x 320 Q8_0 6.3 us with one, 13.2 with eight; 4096 x 4096 12.9 / 7.6)
-#define VBS_HOT(K)                                                                                         \
-    do {                                                                                                   \
-        if (cols <= 512u)                                                                                  \
-            hipLaunchKernelGGL((k_hot_blocks<K, 1>), grid, block, 0, s, wb, rows, cols / 32u, xq, qd, qsum, y); \
-        else if (cols <= 2048u)                                                                            \
-            hipLaunchKernelGGL((k_hot_blocks<K, 4>), grid, block, 0, s, wb, rows, cols / 32u, xq, qd, qsum, y); \
-        else                                                                                               \
-            hipLaunchKernelGGL((k_hot_blocks<K, 8>), grid, block, 0, s, wb, rows, cols / 32u, xq, qd, qsum, y); \
+        // x 320 Q8_0 6.3 us with one, 13.2 with eight; 4096 x 4096 12.9 / 7.6; 16000 x
+        // 544 5.9 with two, 8.5 with four). Terms added from the lanes against LDS:
+        // Q8_0 1 x 32 2.06 / 2.25, 16000 x 320 4.29 / 5.65, 4096 x 1024 3.17 / 3.53; but
+        // of 64 blocks Q4_0 8000 x 2048 5.70 / 5.30, and of Q4_1's two terms a block
+        // 16000 x 544 7.6 / 6.0 (256 x 544 2.47 / 2.68)
+#define VBS_HOT_L(K, U, R) hipLaunchKernelGGL((k_hot_blocks<K, U, R>), grid, block, 0, s, wb, rows, cols / 32u, xq, qd, qsum, y)
+#define VBS_HOT(K)                                               \
+    do {                                                         \
+        if (cols <= 512u) VBS_HOT_L(K, 1, true);                 \
+        else if (cols <= 1024u) VBS_HOT_L(K, 2, K != HK_Q4_1);   \
+        else if (cols <= 2048u) VBS_HOT_L(K, 4, false);          \
+        else VBS_HOT_L(K, 8, false);                             \
     } while (0)
         if (kind == HK_Q8_0) VBS_HOT(HK_Q8_0);
         else if (kind == HK_Q4_0) VBS_HOT(HK_Q4_0);
         else VBS_HOT(HK_Q4_1);
 #undef VBS_HOT
+#undef VBS_HOT_L
     } else {
         const dim3 grid((rows + kHotRows - 1u) / kHotRows), block(320);
         const float *x = static_cast<const float *>(act);
