@@ -844,6 +844,36 @@ def test_attention_non_finite_cache(dev, host, oracle, mem, hd, nqh, nkh, seq, w
     assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-4 * np.abs(want[fine]))
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96])
+@pytest.mark.parametrize("nqh,nkh", [(1, 1), (5, 1), (4, 2), (16, 4), (3, 3), (24, 8)])
+@pytest.mark.parametrize("seq", [257, 4097, 8200, 12300, 33000])
+def test_attention_long_splits(dev, host, oracle, mem, hd, nqh, nkh, seq):
+    """The chunk splits of longer contexts: at most 128 chunks per kv head up to
+    32768 positions and more past them, chunks of one to eight tiles on one to
+    four waves, the last one short; one q head per kv head on the vector ALU.
+    Then with an infinite and a NaN value and a -inf score near the end."""
+    max_ctx, layer = seq + 3, 1
+    kc = V.synth_normal_f16(host, 2 * max_ctx * nkh * hd, SEED, 171)
+    vc = V.synth_normal_f16(host, 2 * max_ctx * nkh * hd, SEED, 172)
+    q = synth_x(host, nqh * hd, 173)
+    scale = np.float32(1.0 / math.sqrt(hd))
+    for bad in (False, True):
+        if bad:
+            k, v = (c.reshape(2, max_ctx, nkh, hd)[layer] for c in (kc, vc))
+            k[seq - 40, 0, 4] = 0xFC00
+            v[seq - 2, nkh - 1, 1] = 0x7C00
+            v[seq - 33, nkh - 1, 2] = 0x7E00
+        po = mem.zeros(nqh * hd)
+        dev.attention(mem.up(q), mem.up(kc), mem.up(vc), po, seq, layer, max_ctx, nqh, nkh, hd, scale)
+        got = dev.download(po, nqh * hd, np.float32)
+        want = oracle.attention(q, kc, vc, seq, layer, max_ctx, nqh, nkh, hd, scale)
+        fine = np.isfinite(want)
+        assert fine.all() != bad
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-4 * np.abs(want[fine]))
+
+
 @pytest.mark.parametrize("qscale", [1e-6, 1e4])
 def test_attention_q_magnitude(dev, host, oracle, mem, qscale):
     """q far from unit scale (the matrix-core kernel rescales each head's q

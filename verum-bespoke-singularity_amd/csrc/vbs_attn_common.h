@@ -12,8 +12,8 @@
 
 namespace vbs {
 
-// One-wave workgroups the matrix-core split aims for per sequence. The chunk
-// kernel holds 192 registers (157 VGPRs and the MFMA accumulators): two waves
+// One-wave workgroups the matrix-core split aims for per sequence. At head_dim
+// 128 the chunk kernel holds 192 registers (157 VGPRs and the MFMA accumulators): two waves
 // per SIMD, 2048 on the chip at once. At 70B, batch 8, a target of 1024 made
 // 5504 of them (2.7 rounds of waves), 640 makes 4160 (2.03). Measured chunk +
 // merge with 640 against 1024: 70B batch 8 51.2 against 52.3-55.7 us, 70B
@@ -47,6 +47,19 @@ __host__ __device__ inline AttnSplit attn_split(uint32_t seq, uint32_t nkh, uint
 __host__ __device__ inline uint32_t mfma_chunks(uint32_t seq, uint32_t nkh,
                                                 uint32_t target = kMfmaTargetWgs) {
     return attn_split(seq, nkh, kMfmaGran, kMfmaLmax, target).n;
+}
+
+// The same for any head size. At head sizes but 128 a kv head has at most
+// kFineChunks chunks for as long as kMfmaLmax allows: the merge takes that many
+// in one round trip, and few kv heads have many short chunks (8 q heads over one
+// kv head, head_dim 32, 16000 positions: 500 chunks 20.1 us, 125 8.7).
+constexpr uint32_t kFineChunks = 128, kFineWaves = 4;
+template <uint32_t HD>
+__host__ __device__ inline AttnSplit mfma_split(uint32_t seq, uint32_t nkh, uint32_t target = kMfmaTargetWgs) {
+    const AttnSplit a = attn_split(seq, nkh, kMfmaGran, kMfmaLmax, target);
+    if (HD == 128u) return a;
+    const AttnSplit b = attn_split(seq, 1u, kMfmaGran, kMfmaLmax, kFineChunks);
+    return a.len > b.len ? a : b;
 }
 
 // e^x as 2^(x log2 e) on the hardware exponential (a few ulp; the scores

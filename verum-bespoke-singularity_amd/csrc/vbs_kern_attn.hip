@@ -11,14 +11,15 @@
 // log-sum-exp rescaling: out = sum_c acc_c * e^(m_c-M) / sum_c l_c * e^(m_c-M).
 // The chunk length follows the sequence (attn_split) so that about
 // kMfmaTargetWgs (vbs_attn_common.h) workgroups of the matrix-core kernel, or
-// kTargetWgs of the generic one, share it at any length. A second kernel
-// merges (a hand-off inside one kernel, through device-scope stores, loads and
-// an arrival count, measured slower than the kernel boundary on this part);
-// short sequences take one launch that does both, the chunks of a kv head
-// on the waves of one workgroup (k_attn_one).
+// kTargetWgs of k_attn_solo, share it at any length; the generic kernel's is
+// kChunk. A second kernel merges (a hand-off inside one kernel, through
+// device-scope stores, loads and an arrival count, measured slower than the
+// kernel boundary on this part); short sequences take one launch that does
+// both, the chunks of a kv head on the waves of one workgroup (k_attn_one).
 //
 // head_dim 32, 64, 96 and 128 with at most eight q heads per kv head take the
-// matrix-core chunk kernel; other shapes the generic one (double dot, one
+// matrix-core chunk kernel, but one q head per kv head of 32 or 64 dims past the
+// one-launch lengths k_attn_solo; other shapes the generic one (double dot, one
 // position per four threads).
 #include "vbs_attn_common.h"
 #include "vbs_dev_common.h"
@@ -28,7 +29,7 @@ namespace vbs {
 
 constexpr uint32_t kChunk = 64;  // positions per workgroup of the generic kernel
 constexpr uint32_t kMaxGroup = 16;
-constexpr uint32_t kTargetWgs = 512;      // workgroups the generic kernel's split aims for
+constexpr uint32_t kTargetWgs = 512;      // workgroups k_attn_solo's split aims for
 
 // (attn_split, the matrix-core split's constants and the exponentials: vbs_attn_common.h)
 // Chunks per kv head of any split of a sequence of at most max_seq (every
@@ -138,6 +139,171 @@ __global__ __launch_bounds__(256) void k_attn_partial(const float *__restrict__ 
 }
 
 
+// ---- one q head per kv head (head_dim 32, 64) on the vector ALU -----------------
+// Four waves; lanes of a wave split a position's head_dim into 8-element slices
+// (16-byte K and V loads), so one wave step covers 64 / (HD / 8) positions
+// ("slots"). A wave loads kSteps steps at a time (up to kBatches such batches;
+// the next batch's K rows are requested once the scores are taken, its V rows
+// once they are used). The partial dot of a slice is an fp32 FMA chain and the
+// slices are added with DPP row operations, which leaves every lane of a slot
+// with its score. Each slot keeps a running softmax state (max, sum, acc); the
+// slots of a wave are combined with lane shuffles and the four waves in LDS.
+// With a single q head the matrix cores' columns stand empty and its scores and
+// weights cost the same as eight heads': past the one-launch lengths this
+// kernel is ahead (8 heads of 64, 300, 3001 and 9000 positions 6.6, 7.2 and 9.0 us
+// against 6.9, 8.3 and 11.0; 32 heads 3001 8.3 against 11.5; at two q heads per
+// kv head the matrix cores are, 16 over 8 3001 8.5 against 9.4).
+constexpr uint32_t kWaves = 4, kSteps = 4, kBatches = 4;
+template <uint32_t HD>
+struct ChunkShape {
+    static constexpr uint32_t LPP = HD / 8, PPW = 64 / LPP, GRAN = kWaves * PPW,
+                              LMAX = kBatches * kSteps * GRAN;
+};
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                     CTRL, 0xF, 0xF, false));
+}
+// Sum over each aligned group of L lanes (L = 4, 8), for every lane of it.
+template <uint32_t L>
+__device__ __forceinline__ float group_sum(float v) {
+    v = dpp_add<0xB1>(v);                         // quad_perm [1,0,3,2]
+    v = dpp_add<0x4E>(v);                         // quad_perm [2,3,0,1]
+    if constexpr (L >= 8) v = dpp_add<0x141>(v);  // row_half_mirror
+    return v;
+}
+
+template <uint32_t HD>
+__global__ __launch_bounds__(64 * kWaves) void k_attn_solo(
+    const float *__restrict__ q, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,
+    float *__restrict__ part, uint32_t seq_len, const uint32_t *__restrict__ pos_dev, uint64_t layer_off,
+    uint32_t nh, float scale, uint32_t stride_chunks) {
+    using S = ChunkShape<HD>;
+    constexpr uint32_t LPP = S::LPP, PPW = S::PPW;
+    __shared__ __align__(16) float red[kWaves][HD];
+    __shared__ float sm[kWaves], sl[kWaves];
+    const uint32_t chunk = blockIdx.x, h = blockIdx.y, t = threadIdx.x;
+    const uint32_t wave = t >> 6, lane = t & 63u, slot = lane / LPP, c = lane % LPP;
+    if (pos_dev) seq_len = pos_dev[0] + 1u;  // graph replay: the device holds the position
+    const AttnSplit sp = attn_split(seq_len, nh, S::GRAN, S::LMAX, kTargetWgs);
+    if (chunk >= sp.n) return;  // past the sequence (the grid covers the longest split)
+    const uint32_t s0 = chunk * sp.len, valid = min(sp.len, seq_len - s0);
+    const uint32_t pw = sp.len / kWaves, ns = pw / PPW;  // positions and steps per wave
+    const uint32_t nb = (ns + kSteps - 1u) / kSteps;     // batches of kSteps steps
+    const uint64_t rstride = (uint64_t)nh * HD;
+    const uint64_t base = layer_off + (uint64_t)s0 * rstride + (uint64_t)h * HD + 8u * c;
+
+    // position of step i of this lane's slot; positions past the chunk re-read
+    // its last row and are masked (score -inf, v zero)
+    auto pos_of = [&](uint32_t i) { return wave * pw + i * PPW + slot; };
+    uint4 kr[kSteps], vr[kSteps];
+    auto load_k = [&](uint32_t bi) {
+#pragma unroll
+        for (uint32_t b = 0; b < kSteps; b++)
+            if (bi * kSteps + b < ns)
+                kr[b] = *reinterpret_cast<const uint4 *>(
+                    kc + base + (uint64_t)min(pos_of(bi * kSteps + b), valid - 1u) * rstride);
+    };
+    auto load_v = [&](uint32_t bi) {
+#pragma unroll
+        for (uint32_t b = 0; b < kSteps; b++) {
+            const uint32_t i = bi * kSteps + b;
+            if (i < ns) {
+                vr[b] = *reinterpret_cast<const uint4 *>(vc + base + (uint64_t)min(pos_of(i), valid - 1u) * rstride);
+                if (pos_of(i) >= valid) vr[b] = make_uint4(0u, 0u, 0u, 0u);
+            }
+        }
+    };
+    load_k(0);
+    load_v(0);
+    float qv[8];
+    {
+        const float4 *qp = reinterpret_cast<const float4 *>(q + (uint64_t)h * HD + 8u * c);
+        const float4 a = qp[0], b = qp[1];
+        qv[0] = a.x, qv[1] = a.y, qv[2] = a.z, qv[3] = a.w;
+        qv[4] = b.x, qv[5] = b.y, qv[6] = b.z, qv[7] = b.w;
+    }
+
+    // per slot: running max m, sum l of e^(s - m), acc of e^(s - m) v
+    float m = -INFINITY, l = 0.f, acc[8] = {};
+    for (uint32_t bi = 0; bi < nb; bi++) {
+        float sc[kSteps];  // every lane of a slot holds its position's score
+#pragma unroll
+        for (uint32_t b = 0; b < kSteps; b++) {
+            const uint32_t i = bi * kSteps + b;
+            float p = 0.f;
+            if (i < ns) {
+                const uint32_t kw[4] = {kr[b].x, kr[b].y, kr[b].z, kr[b].w};
+#pragma unroll
+                for (uint32_t j = 0; j < 8; j++) p = fmaf(qv[j], hcvt(kw[j >> 1] >> (16u * (j & 1u))), p);
+                p = group_sum<LPP>(p);
+            }
+            sc[b] = i < ns && pos_of(i) < valid ? __fmul_rn(p, scale) : -INFINITY;
+        }
+        if (bi + 1u < nb) load_k(bi + 1u);  // the K registers are free again
+        float mb = sc[0];
+#pragma unroll
+        for (uint32_t b = 1; b < kSteps; b++) mb = fmaxf(mb, sc[b]);
+        const float mn = fmaxf(m, mb);
+        const float r = m == -INFINITY ? 0.f : fast_exp(__fsub_rn(m, mn));
+        l *= r;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++) acc[j] *= r;
+#pragma unroll
+        for (uint32_t b = 0; b < kSteps; b++) {
+            if (bi * kSteps + b < ns) {
+                const float e = sc[b] == -INFINITY ? 0.f : fast_exp(__fsub_rn(sc[b], mn));
+                const uint32_t vw[4] = {vr[b].x, vr[b].y, vr[b].z, vr[b].w};
+                l += e;
+#pragma unroll
+                for (uint32_t j = 0; j < 8; j++) acc[j] = fmaf(e, hcvt(vw[j >> 1] >> (16u * (j & 1u))), acc[j]);
+            }
+        }
+        m = mn;
+        if (bi + 1u < nb) load_v(bi + 1u);
+    }
+
+    // the wave's slots combined (lanes of equal c): M = max m, weights e^(m - M)
+    // (0 for an empty slot), then sums; slot 0 stores them
+    float M = m;
+#pragma unroll
+    for (uint32_t off = LPP; off < 64u; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    const float f = m == -INFINITY ? 0.f : fast_exp(__fsub_rn(m, M));
+    float L = l * f;
+#pragma unroll
+    for (uint32_t j = 0; j < 8; j++) acc[j] *= f;
+#pragma unroll
+    for (uint32_t off = LPP; off < 64u; off <<= 1) {
+        L += __shfl_xor(L, off, 64);
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++) acc[j] += __shfl_xor(acc[j], off, 64);
+    }
+    if (slot == 0) {
+        float4 *dst = reinterpret_cast<float4 *>(&red[wave][8u * c]);
+        dst[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        dst[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+        if (c == 0) sm[wave] = M, sl[wave] = L;
+    }
+    __syncthreads();
+
+    // the waves combined: M = max m_w, weights e^(m_w - M) (0 for empty waves)
+    if (t < HD) {
+        float Mw = sm[0], a = 0.f, Lw = 0.f;
+#pragma unroll
+        for (uint32_t w = 1; w < kWaves; w++) Mw = fmaxf(Mw, sm[w]);
+#pragma unroll
+        for (uint32_t w = 0; w < kWaves; w++) {
+            const float fw = sm[w] == -INFINITY ? 0.f : fast_exp(__fsub_rn(sm[w], Mw));
+            a = fmaf(red[w][t], fw, a);
+            Lw = fmaf(sl[w], fw, Lw);
+        }
+        float *dst = part + ((uint64_t)h * stride_chunks + chunk) * (HD + 2u);
+        dst[2u + t] = a;
+        if (t == 0) dst[0] = Mw, dst[1] = Lw;
+    }
+}
+
 // ---- matrix-core chunk kernel (head_dim 32, 64, 96, 128; group <= 8) -------------
 // One wave per chunk of up to kMfmaTiles tiles of 32 positions, on
 // v_mfma_f32_16x16x32_f16:
@@ -170,13 +336,19 @@ __global__ __launch_bounds__(256) void k_attn_partial(const float *__restrict__ 
 // replay reads the position on the device, so the grid covers every
 // position up to max_seq, and workgroups beyond the current split exit at
 // once (each costs dispatch time, so the grid is no larger than this).
+template <uint32_t HD = 128>
 inline uint32_t mfma_grid_chunks(uint32_t max_seq, uint32_t nkh, uint32_t target = kMfmaTargetWgs) {
     uint32_t best = 0;
     for (uint32_t k = 1; k <= kMfmaTiles; k++) {
-        const uint64_t hi = k < kMfmaTiles ? (uint64_t)kMfmaGran * k * target / nkh : max_seq;
+        uint64_t hi = max_seq;
+        if (k < kMfmaTiles) {
+            hi = (uint64_t)kMfmaGran * k * target / nkh;
+            const uint64_t cap = (uint64_t)kMfmaGran * k * kFineChunks;
+            if (HD != 128u && hi > cap) hi = cap;
+        }
         const uint32_t s = (uint32_t)(hi < max_seq ? hi : max_seq);
         if (s == 0) continue;
-        const uint32_t c = attn_split(s, nkh, kMfmaGran, kMfmaLmax, target).n;
+        const uint32_t c = mfma_split<HD>(s, nkh, target).n;
         best = c > best ? c : best;
     }
     return best;
@@ -418,84 +590,97 @@ __device__ __forceinline__ void attn_mfma_store(float *pk, uint32_t stride, uint
     }
 }
 
-// The heads of a chunk whose sums are not finite once more, whole (head sizes
-// but 128): an infinite score or value meets the hi and lo halves as inf - inf
-// or 0 * inf. Here, as in the sequential softmax, -inf scores weigh 0, +inf and
-// NaN give NaN, and an infinite value of positive weight gives inf. Scores are
-// double dots, a lane per position; values a lane per DPL dims. m, l, a: what
-// attn_mfma_store has just stored. The test hides behind those stores (under 1%
-// of a launch); a head taken again costs about 2.5 us per 64 positions of a chunk.
+// Head sizes but 128: one q head (qh) over `valid` <= kMfmaLmax positions from
+// base on, in whole f32 products: scores as double dots, a lane per position;
+// on return o[dt] = the sum of 2^(s log2 e - m) v[DPL n + dt] in every lane group.
+// For heads whose sums are not finite: an infinite score or value meets the hi
+// and lo halves of attn_mfma_wave as inf - inf or 0 * inf. Here, as in the
+// sequential softmax, -inf scores weigh 0, +inf and NaN give NaN, and an infinite
+// value of positive weight gives inf. About 2.5 us per 64 positions.
+template <uint32_t HD>
+__device__ __forceinline__ void attn_head_whole(const float *__restrict__ qh, const uint16_t *__restrict__ kc,
+                                                const uint16_t *__restrict__ vc, uint64_t base, uint32_t valid,
+                                                uint64_t rstride, float scale, uint32_t lane, float &m_out,
+                                                float &l_out, float (&o)[HD / 16]) {
+    constexpr uint32_t DPL = HD / 16u, NP = kMfmaLmax / 64u;  // positions per lane
+    const uint32_t n = lane & 15u;
+    float sc[NP], e[NP], mt = -INFINITY, l = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < NP; i++) {
+        const uint32_t p = lane + 64u * i;
+        double d = 0.0;
+        if (64u * i < valid) {
+            const uint16_t *kr = kc + base + (uint64_t)min(p, valid - 1u) * rstride;
+#pragma unroll
+            for (uint32_t c = 0; c < HD; c += 8u) {
+                const au4 kw = *reinterpret_cast<const au4 *>(kr + c);
+#pragma unroll
+                for (uint32_t k = 0; k < 8u; k++)
+                    d = fma((double)qh[c + k], (double)hcvt(kw[k >> 1] >> (16u * (k & 1u))), d);
+            }
+        }
+        sc[i] = p < valid ? __fmul_rn((float)d, scale) : -INFINITY;
+        mt = fmaxf(mt, __fmul_rn(sc[i], 1.44269504088896341f));
+    }
+    const float mn = ceilf(wave_max(mt));  // (a whole power of two, as attn_mfma_wave's)
+#pragma unroll
+    for (uint32_t i = 0; i < NP; i++) {
+        const float p = __fmul_rn(sc[i], 1.44269504088896341f), r = rintf(p);
+        const float err = fmaf(sc[i], 1.92596299e-8f, fmaf(sc[i], 1.44269504088896341f, -p));
+        e[i] = ldexpf(exp2_fast((p - r) + __builtin_amdgcn_fmed3f(err, -0.5f, 0.5f)), (int)(r - mn));
+        if (sc[i] == -INFINITY) e[i] = 0.f;
+        l += e[i];
+    }
+    m_out = mn;
+    l_out = wave_sum(l);
+#pragma unroll
+    for (uint32_t dt = 0; dt < DPL; dt++) o[dt] = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < NP; i++)
+        for (uint32_t p0 = 64u * i; p0 < min(valid, 64u * (i + 1u)); p0 += 8u) {
+            uint16_t vr[8][DPL];  // (eight rows requested at a time)
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++)
+#pragma unroll
+                for (uint32_t dt = 0; dt < DPL; dt++)
+                    vr[k][dt] = vc[base + (uint64_t)min(p0 + k, valid - 1u) * rstride + DPL * n + dt];
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) {
+                const float w = __shfl(e[i], (int)((p0 + k) & 63u), 64);
+                if (p0 + k < valid) {
+#pragma unroll
+                    for (uint32_t dt = 0; dt < DPL; dt++) o[dt] = fmaf(w, hcvt(vr[k][dt]), o[dt]);
+                }
+            }
+        }
+}
+
+// The heads of a chunk whose sums (l, a: what attn_mfma_store has just stored) are
+// not finite once more. The test hides behind those stores.
 template <uint32_t HD>
 __device__ __forceinline__ void attn_heads_again(const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                                  const uint16_t *__restrict__ vc, uint64_t layer_off, uint32_t s0,
                                                  uint32_t valid, uint32_t nkh, uint32_t kvh, uint32_t group,
                                                  float scale, uint32_t lane, float *pk, uint32_t stride,
-                                                 uint32_t chunk, float l0, const float (&a)[HD / 16][4]) {
-    constexpr uint32_t DPL = HD / 16u, NP = kMfmaLmax / 64u;  // positions per lane
+                                                 uint32_t chunk, float l, const float (&a)[HD / 16][4]) {
+    constexpr uint32_t DPL = HD / 16u;
     const uint32_t n = lane & 15u, g = lane >> 4;
     float t[4] = {0.f, 0.f, 0.f, 0.f};  // NaN where a head's sums are not finite
 #pragma unroll
     for (uint32_t dt = 0; dt < DPL; dt++)
 #pragma unroll
         for (uint32_t r = 0; r < 4; r++) t[r] = fmaf(a[dt][r], 0.f, t[r]);
-    if (__builtin_expect(!__ballot(fmaf(l0, 0.f, (t[0] + t[1]) + (t[2] + t[3])) != 0.f), 1)) return;
+    if (__builtin_expect(!__ballot(fmaf(l, 0.f, (t[0] + t[1]) + (t[2] + t[3])) != 0.f), 1)) return;
     const uint64_t rstride = (uint64_t)nkh * HD, base = layer_off + (uint64_t)s0 * rstride + (uint64_t)kvh * HD;
 #pragma unroll 1
     for (uint32_t hh = 0; hh < group; hh++) {
-        bool bad = (n & 7u) == hh && !(fabsf(l0) <= 3.4028235e38f);
+        bool bad = (n & 7u) == hh && !(fabsf(l) <= 3.4028235e38f);
 #pragma unroll
         for (uint32_t r = 0; r < 4; r++) bad |= 4u * (g & 1u) + r == hh && t[r] != 0.f;
         if (!__ballot(bad)) continue;
-        const float *qh = q + ((uint64_t)kvh * group + hh) * HD;
-        float sc[NP], e[NP], mt = -INFINITY, l = 0.f;
-#pragma unroll
-        for (uint32_t i = 0; i < NP; i++) {
-            const uint32_t p = lane + 64u * i;
-            double d = 0.0;
-            if (64u * i < valid) {
-                const uint16_t *kr = kc + base + (uint64_t)min(p, valid - 1u) * rstride;
-#pragma unroll
-                for (uint32_t c = 0; c < HD; c += 8u) {
-                    const au4 kw = *reinterpret_cast<const au4 *>(kr + c);
-#pragma unroll
-                    for (uint32_t k = 0; k < 8u; k++)
-                        d = fma((double)qh[c + k], (double)hcvt(kw[k >> 1] >> (16u * (k & 1u))), d);
-                }
-            }
-            sc[i] = p < valid ? __fmul_rn((float)d, scale) : -INFINITY;
-            mt = fmaxf(mt, __fmul_rn(sc[i], 1.44269504088896341f));
-        }
-        const float mn = ceilf(wave_max(mt));  // (a whole power of two, as attn_mfma_wave's)
-#pragma unroll
-        for (uint32_t i = 0; i < NP; i++) {
-            const float p = __fmul_rn(sc[i], 1.44269504088896341f), r = rintf(p);
-            const float err = fmaf(sc[i], 1.92596299e-8f, fmaf(sc[i], 1.44269504088896341f, -p));
-            e[i] = ldexpf(exp2_fast((p - r) + __builtin_amdgcn_fmed3f(err, -0.5f, 0.5f)), (int)(r - mn));
-            if (sc[i] == -INFINITY) e[i] = 0.f;
-            l += e[i];
-        }
-        l = wave_sum(l);
-        float o[DPL];
-#pragma unroll
-        for (uint32_t dt = 0; dt < DPL; dt++) o[dt] = 0.f;
-#pragma unroll
-        for (uint32_t i = 0; i < NP; i++)
-            for (uint32_t p0 = 64u * i; p0 < min(valid, 64u * (i + 1u)); p0 += 8u) {
-                uint16_t vr[8][DPL];  // (eight rows requested at a time)
-#pragma unroll
-                for (uint32_t k = 0; k < 8u; k++)
-#pragma unroll
-                    for (uint32_t dt = 0; dt < DPL; dt++)
-                        vr[k][dt] = vc[base + (uint64_t)min(p0 + k, valid - 1u) * rstride + DPL * n + dt];
-#pragma unroll
-                for (uint32_t k = 0; k < 8u; k++) {
-                    const float w = __shfl(e[i], (int)((p0 + k) & 63u), 64);
-                    if (p0 + k < valid) {
-#pragma unroll
-                        for (uint32_t dt = 0; dt < DPL; dt++) o[dt] = fmaf(w, hcvt(vr[k][dt]), o[dt]);
-                    }
-                }
-            }
+        float mw, lw, o[DPL];
+        attn_head_whole<HD>(q + ((uint64_t)kvh * group + hh) * HD, kc, vc, base, valid, rstride, scale, lane, mw, lw,
+                            o);
         // (by the lanes that stored the head's row before)
         float *dst = pk + ((uint64_t)hh * stride + chunk) * part_row<HD>;
         if (g == hh >> 2) {
@@ -504,8 +689,8 @@ __device__ __forceinline__ void attn_heads_again(const float *__restrict__ q, co
                 reinterpret_cast<float2 *>(dst + 2u + DPL * n)[i] = make_float2(o[2 * i], o[2 * i + 1]);
         }
         if (g == 0u && n == hh) {
-            dst[0] = mn;
-            dst[1] = l;
+            dst[0] = mw;
+            dst[1] = lw;
         }
     }
 }
@@ -524,8 +709,11 @@ __device__ __forceinline__ void attn_mfma_chunk(const float *__restrict__ q, con
         attn_heads_again<HD>(q, kc, vc, layer_off, s0, valid, nkh, kvh, group, scale, lane, pk, stride, chunk, l, a);
 }
 
-template <uint32_t HD>
-__global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
+// A chunk per workgroup: one wave, or (MULTI, head sizes but 128) the chunk's
+// tiles split over up to kFineWaves waves, whose sums are joined in LDS: their
+// maxima are whole powers of two, so the weights are exact.
+template <uint32_t HD, bool MULTI = false>
+__global__ __launch_bounds__(MULTI ? 64 * kFineWaves : 64) void k_attn_mfma(const float *__restrict__ q,
                                                   const uint16_t *__restrict__ kc,
                                                   const uint16_t *__restrict__ vc,
                                                   float *__restrict__ part, uint32_t seq_len,
@@ -536,7 +724,7 @@ __global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
                                                   uint64_t part_bstride, uint32_t target,
                                                   uint32_t *__restrict__ clear, uint32_t nclear,
                                                   uint32_t clear_stride) {
-    const uint32_t chunk = blockIdx.x, kvh = blockIdx.y, lane = threadIdx.x, bz = blockIdx.z;
+    const uint32_t chunk = blockIdx.x, kvh = blockIdx.y, lane = threadIdx.x & 63u, bz = blockIdx.z;
     // the merging launch that follows (k_mvl_attn) starts from cleared flags
     if (clear && chunk == 0u && kvh == 0u && bz == 0u)
         for (uint32_t i = lane; i < nclear; i += 64u) clear[(uint64_t)i * clear_stride] = 0u;
@@ -546,11 +734,42 @@ __global__ __launch_bounds__(64) void k_attn_mfma(const float *__restrict__ q,
     vc += bz * kv_bstride;
     part += bz * part_bstride;
     if (pos_dev) seq_len = pos_dev[bz] + 1u;  // graph replay: the device holds the position
-    const AttnSplit sp = attn_split(seq_len, nkh, kMfmaGran, kMfmaLmax, target);
+    const AttnSplit sp = mfma_split<HD>(seq_len, nkh, target);
     if (chunk >= sp.n) return;  // past the sequence (the grid covers the longest split)
     const uint32_t s0 = chunk * sp.len, valid = min(sp.len, seq_len - s0);
-    attn_mfma_chunk<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane,
-                        part + (uint64_t)kvh * group * stride_chunks * part_row<HD>, stride_chunks, chunk);
+    float *const pk = part + (uint64_t)kvh * group * stride_chunks * part_row<HD>;
+    if constexpr (!MULTI) {
+        attn_mfma_chunk<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane, pk,
+                            stride_chunks, chunk);
+    } else {
+        extern __shared__ __align__(16) float joint[];  // [group][waves][HD + 2]
+        const uint32_t nw = blockDim.x >> 6, wave = threadIdx.x >> 6;
+        const uint32_t tiles = (valid + kMfmaGran - 1u) / kMfmaGran, tpw = (tiles + nw - 1u) / nw;
+        const uint32_t used = (tiles + tpw - 1u) / tpw, w0 = kMfmaGran * tpw * wave;
+        if (wave < used) {
+            const uint32_t v = min(kMfmaGran * tpw, valid - w0);
+            attn_mfma_chunk<HD>(q, kc, vc, layer_off, s0 + w0, v, (v + kMfmaGran - 1u) / kMfmaGran, nkh, kvh, group,
+                                scale, lane, joint, nw, wave);
+        }
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < group * (HD / 2u); i += blockDim.x) {
+            const uint32_t hh = i / (HD / 2u), d = 2u * (i % (HD / 2u));
+            const float *row = joint + hh * nw * part_row<HD>;
+            float M = row[0];
+            for (uint32_t w = 1; w < used; w++) M = fmaxf(M, row[w * part_row<HD>]);
+            float l = 0.f, ax = 0.f, ay = 0.f;
+            for (uint32_t w = 0; w < used; w++) {
+                const float *rw = row + w * part_row<HD>;
+                const float wt = rw[0] == -INFINITY ? 0.f : ldexpf(1.f, (int)(rw[0] - M));
+                l = fmaf(rw[1], wt, l);
+                ax = fmaf(rw[2u + d], wt, ax);
+                ay = fmaf(rw[3u + d], wt, ay);
+            }
+            float *dst = pk + ((uint64_t)hh * stride_chunks + chunk) * part_row<HD>;
+            *reinterpret_cast<float2 *>(dst + 2u + d) = make_float2(ax, ay);
+            if (d == 0u) *reinterpret_cast<float2 *>(dst) = make_float2(M, l);
+        }
+    }
 }
 
 // Short sequences (at most kOneChunks chunks) in one launch: workgroup kvh
@@ -567,17 +786,44 @@ __global__ __launch_bounds__(64 * kOneChunks) void k_attn_one(
     extern __shared__ __align__(16) float part[];  // [group][kOneChunks][HD + 2]
     const uint32_t nw = blockDim.x >> 6, kvh = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     if (pos_dev) seq_len = pos_dev[0] + 1u;
+    // (mfma_split's bound on the chunk count is not met at such lengths)
     const AttnSplit sp = attn_split(seq_len, nkh, kMfmaGran, kMfmaLmax, kMfmaTargetWgs);
     if (wave < sp.n) {
         const uint32_t s0 = wave * sp.len, valid = min(sp.len, seq_len - s0);
-        attn_mfma_chunk<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane, part,
-                            kOneChunks, wave);
+        float m, l, a[HD / 16][4];
+        attn_mfma_wave<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane, m, l, a);
+        attn_mfma_store<HD>(part, kOneChunks, wave, group, lane, m, l, a);
     }
     __syncthreads();
+    uint32_t again = 0;  // heads whose results are not finite (attn_head_whole)
     for (uint32_t h = wave; h < group; h += nw) {
         const float2 o = merge_one_wave<kOneChunks, HD>(part + h * kOneChunks * part_row<HD>, sp.n, lane);
         if (HD == 128u || lane < HD / 2u)
             *reinterpret_cast<float2 *>(out + ((uint64_t)kvh * group + h) * HD + 2u * lane) = o;
+        if (HD != 128u && __ballot(lane < HD / 2u && fmaf(o.x, 0.f, o.y * 0.f) != 0.f)) again |= 1u << h;
+    }
+    if constexpr (HD != 128u) {
+        if (__builtin_expect(again != 0u, 0)) {
+            constexpr uint32_t DPL = HD / 16u;
+            // dims 2 lane and 2 lane + 1 go to the lane that stored them before
+            const uint32_t at = 2u * (lane % (HD / 2u)), src = at / DPL, d0 = at % DPL;
+#pragma unroll 1
+            for (uint32_t h = wave; h < group; h += nw) {
+                if (!((again >> h) & 1u)) continue;
+                float m, l, w[DPL];
+                attn_head_whole<HD>(q + ((uint64_t)kvh * group + h) * HD, kc, vc, layer_off + (uint64_t)kvh * HD,
+                                    seq_len, (uint64_t)nkh * HD, scale, lane, m, l, w);
+                float2 r = make_float2(0.f, 0.f);
+#pragma unroll
+                for (uint32_t i = 0; i < DPL / 2u; i++) {
+                    const float x = __shfl(w[2 * i], (int)src, 64), y = __shfl(w[2 * i + 1], (int)src, 64);
+                    if (d0 == 2u * i) r = make_float2(x, y);
+                }
+                if (lane < HD / 2u)
+                    *reinterpret_cast<float2 *>(out + ((uint64_t)kvh * group + h) * HD + 2u * lane) =
+                        make_float2(r.x / l, r.y / l);
+            }
+        }
     }
 }
 
@@ -594,18 +840,14 @@ __global__ __launch_bounds__(kMergeThreads) void k_attn_merge(const float *__res
                                                     float *__restrict__ out, uint32_t hd,
                                                     uint32_t n_chunks, uint32_t stride_chunks,
                                                     const uint32_t *__restrict__ pos_dev,
-                                                    uint32_t nkh, uint32_t gran, uint32_t lmax,
-                                                    uint32_t target, uint32_t q_bstride,
-                                                    uint64_t part_bstride) {
+                                                    uint32_t nkh, uint32_t gran, uint32_t lmax) {
     extern __shared__ __align__(16) uint8_t merge_lds[];
     float *w = reinterpret_cast<float *>(merge_lds);  // [stride_chunks]
     float *sl = w + stride_chunks;                    // [kMergeThreads]
     constexpr uint32_t NW = kMergeThreads / 64u;
     __shared__ float red[2 * NW];
-    const uint32_t h = blockIdx.x, t = threadIdx.x, lane = t & 63u, wave = t >> 6, bz = blockIdx.y;
-    part += bz * part_bstride;  // sequence bz of a batch
-    out += (uint64_t)bz * q_bstride;
-    if (pos_dev) n_chunks = attn_split(pos_dev[bz] + 1u, nkh, gran, lmax, target).n;  // seq = pos + 1
+    const uint32_t h = blockIdx.x, t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    if (pos_dev) n_chunks = attn_split(pos_dev[0] + 1u, nkh, gran, lmax, kTargetWgs).n;  // seq = pos + 1
     const float *ph = part + (uint64_t)h * stride_chunks * (hd + 2u);
     const uint32_t ns = kMergeThreads / hd;
     const uint32_t d = t % hd, s = t / hd;
@@ -682,7 +924,7 @@ __global__ __launch_bounds__(64 * kMergeRes) void k_attn_merge_hd(
     part += bz * part_bstride;
     out += (uint64_t)bz * q_bstride;
     if (pos_dev) seq_len = pos_dev[bz] + 1u;  // seq = pos + 1
-    const uint32_t nc = mfma_chunks(seq_len, nkh, target);
+    const uint32_t nc = mfma_split<HD>(seq_len, nkh, target).n;
     const float *ph = part + (uint64_t)h * stride_chunks * part_row<HD>;
     float2 av[kMergeBatch];
     merge_residue_load<HD>(ph, nc, wave, lane, av);  // with the (m, l) loads: one round trip
@@ -702,13 +944,24 @@ size_t attention_partial_bytes(uint32_t max_seq, uint32_t nqh, uint32_t nkh, uin
     return (size_t)nqh * attn_max_chunks(max_seq, nkh) * (hd + 2u) * sizeof(float);
 }
 
+// The general merge after k_attn_partial or k_attn_solo.
+static hipError_t launch_merge(const float *part, float *out, uint32_t seq_len, const uint32_t *pos_dev,
+                               uint32_t nqh, uint32_t nkh, uint32_t hd, uint32_t gran, uint32_t lmax,
+                               hipStream_t s) {
+    const uint32_t stride = attn_max_chunks(seq_len, nkh);
+    const size_t lds = ((size_t)stride + kMergeThreads) * sizeof(float);
+    k_attn_merge<<<nqh, kMergeThreads, lds, s>>>(part, out, hd, attn_split(seq_len, nkh, gran, lmax, kTargetWgs).n,
+                                                 stride, pos_dev, nkh, gran, lmax);
+    return hipGetLastError();
+}
+
 // The matrix-core path of one sequence: one launch up to kOneChunks chunks
 // (seq_len is the longest that the launch must cover), else chunks and merge.
 template <uint32_t HD>
 static hipError_t launch_mfma_hd(const float *q, const uint16_t *kc, const uint16_t *vc, float *out,
                                  float *part, uint32_t seq_len, const uint32_t *pos_dev, uint64_t layer_off,
                                  uint32_t nkh, uint32_t group, float scale, hipStream_t s) {
-    const uint32_t chunks = mfma_grid_chunks(seq_len, nkh), stride = attn_max_chunks(seq_len, nkh);
+    const uint32_t chunks = mfma_grid_chunks<HD>(seq_len, nkh), stride = attn_max_chunks(seq_len, nkh);
     // One launch: 41 positions of 8 kv heads 3.4-4.6 us (chunks and merge 6.5-9),
     // 256 of head_dim 64 4.8 (8.8); at head_dim 128 and eight q heads per kv head
     // 256 positions are too many for one workgroup (7.9 against 7.1), 96 alike.
@@ -719,8 +972,34 @@ static hipError_t launch_mfma_hd(const float *q, const uint16_t *kc, const uint1
                                                      scale);
         return hipGetLastError();
     }
-    k_attn_mfma<HD><<<dim3(chunks, nkh), 64, 0, s>>>(q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group,
-                                                    scale, stride, 0u, 0ull, 0ull, kMfmaTargetWgs, nullptr, 0u, 0u);
+    if constexpr (HD == 32u || HD == 64u) {
+        if (group == 1u) {  // (k_attn_solo: why)
+            using S = ChunkShape<HD>;
+            const uint32_t n = pos_dev ? stride : attn_split(seq_len, nkh, S::GRAN, S::LMAX, kTargetWgs).n;
+            k_attn_solo<HD><<<dim3(n, nkh), 64u * kWaves, 0, s>>>(q, kc, vc, part, seq_len, pos_dev, layer_off, nkh,
+                                                                  scale, stride);
+            const hipError_t e = hipGetLastError();
+            return e != hipSuccess ? e : launch_merge(part, out, seq_len, pos_dev, nkh, nkh, HD, S::GRAN, S::LMAX, s);
+        }
+    }
+    // Long chunks of few kv heads are split over waves (4 q heads over 2 kv heads,
+    // head_dim 64, 16000 positions 10.9 -> 9.0 us, 16 over 4 11.4 -> 10.6); with more
+    // workgroups than this the chip is full of waves (32 over 8 14.2, split 15.9).
+    // Two tiles pay for joining two waves' sums only below a workgroup per CU
+    // (6000 positions, 4 over 2 8.6 -> 8.2, 16 over 4 8.8 -> 9.6).
+    const uint32_t tiles = mfma_split<HD>(seq_len, nkh).len / kMfmaGran, wgs = chunks * nkh;
+    const bool multi = HD != 128u && tiles > 1u && wgs <= (tiles > 2u ? 512u : 256u);
+    if constexpr (HD != 128u) {
+        const uint32_t nw = tiles < kFineWaves ? tiles : kFineWaves;
+        if (multi)
+            k_attn_mfma<HD, true><<<dim3(chunks, nkh), 64u * nw, (size_t)group * nw * part_row<HD> * sizeof(float), s>>>(
+                q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group, scale, stride, 0u, 0ull, 0ull,
+                kMfmaTargetWgs, nullptr, 0u, 0u);
+    }
+    if (!multi)
+        k_attn_mfma<HD><<<dim3(chunks, nkh), 64, 0, s>>>(q, kc, vc, part, seq_len, pos_dev, layer_off, nkh, group,
+                                                        scale, stride, 0u, 0ull, 0ull, kMfmaTargetWgs, nullptr, 0u,
+                                                        0u);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     k_attn_merge_hd<HD><<<nkh * group, 64 * kMergeRes, 0, s>>>(part, out, stride, pos_dev, seq_len, nkh, 0u, 0ull,
@@ -762,11 +1041,7 @@ hipError_t launch_attention(const float *q, const uint16_t *kc, const uint16_t *
                                                        group, scale, stride);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const uint32_t n_chunks = attn_split(seq_len, nkh, kChunk, kChunk, kTargetWgs).n;
-    const size_t mlds = ((size_t)stride + kMergeThreads) * sizeof(float);
-    k_attn_merge<<<nqh, kMergeThreads, mlds, s>>>(part, out, hd, n_chunks, stride, pos_dev, nkh, kChunk, kChunk,
-                                                  kTargetWgs, 0u, 0ull);
-    return hipGetLastError();
+    return launch_merge(part, out, seq_len, pos_dev, nqh, nkh, hd, kChunk, kChunk, s);
 }
 
 uint32_t attention_chunk_stride(uint32_t max_seq, uint32_t nkh) { return attn_max_chunks(max_seq, nkh); }
