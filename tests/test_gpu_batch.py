@@ -228,6 +228,21 @@ def test_batch_block_types(dev, host, oracle, mem, t, shapes, cols, batch):
 
 
 @pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,batch", [
+    (3072, 8192, 2), (3072, 8192, 3), (3073, 3040, 2), (4096, 3072, 4), (3074, 2048, 4), (8209, 1056, 7), (3071, 1056, 8),
+    (3072, 544, 5), (24576, 512, 8), (24576, 32, 9), (8192, 64, 9), (1920, 4096, 8), (1919, 4096, 8), (2048, 2048, 16),
+    (1024, 8192, 12), (1023, 8192, 16), (1024, 8192, 5)])
+def test_batch_block_types_rule(dev, host, oracle, mem, t, rows, cols, batch):
+    """One matrix on both sides of each limit between the general kernel and the
+    matrix cores, there with one to three tiles per workgroup."""
+    w = V.synth_matrix(host, t, rows, cols, SEED, 184)
+    X = vectors(host, batch, cols, 195)
+    Y = run_batch(dev, mem, t, w, X, rows, cols)
+    for b in range(batch):
+        assert lin_err(Y[b], oracle.linear(t, w, X[b], cols, rows, threads=8)) <= LIN_TOL, b
+
+
+@pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
 def test_batch_block_types_non_finite(dev, host, oracle, mem, t):
     """inf and NaN in a vector and in a row's scales give the oracle's inf and
     NaN rows; the other vectors and rows stay within the bar."""

@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void k_attn_partial(const float *__restrict__ 
 // slots of a wave are combined with lane shuffles and the four waves in LDS.
 // With a single q head the matrix cores' columns stand empty and its scores and
 // weights cost the same as eight heads': past the one-launch lengths this
-// kernel is ahead (8 heads of 64, 300, 3001 and 9000 positions 6.6, 7.2 and 9.0 us
+// kernel is ahead (8 heads of 64, 300, 3001 and 9000 positions 6.6, 7.2 and 8.1 us
 // against 6.9, 8.3 and 11.0; 32 heads 3001 8.3 against 11.5; at two q heads per
 // kv head the matrix cores are, 16 over 8 3001 8.5 against 9.4).
 constexpr uint32_t kWaves = 4, kSteps = 4, kBatches = 4;

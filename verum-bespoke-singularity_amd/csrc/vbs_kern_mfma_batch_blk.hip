@@ -357,6 +357,36 @@ hipError_t launch_mvbb(const MbbArgs &a, hipStream_t s) {
     return launch_mvbb_t<P, 3, 1>(a, min(8u, nu), s);
 }
 
+// Where the general kernel's one launch (k_rows) ends before this path's two
+// for one matrix. Times of the general kernel over this path's, graph replays
+// with weights from HBM (Q4_0 / Q8_0 / F16):
+// * one vector: 0.2 to 0.8 at any size;
+// * two to four: 2048 x 14336 0.7-0.9 / 0.6-0.9 / 0.5-0.7, 5000 x 2048 0.9-1.0 /
+//   0.8-0.9 / 0.7-0.9 (Q4_1 1.0-1.15); but 4096 x 4096 1.2-1.4 / 1.2 / 0.9-1.0, 8192 x 11008 2.0-2.2 /
+//   1.5-1.6 / 0.9-1.0, 4096 x 14336 2.1-2.4 / 1.8-1.9 / 1.0-1.6;
+// * five to eight: up to 2048 x 2048 0.5-0.9, 1024 x 4096 0.7-0.8, 2048 x 4096 0.8-1.05;
+//   but 3072 x 1024 0.9-1.3, 4096 x 4096 1.2-1.8, 1024 x 11008 1.0-1.2 (F16 0.7-0.9);
+//   nine to sixteen: 1024 x 4096 0.8-1.0, 1536 x 4096 0.9-1.15, 8192 x 4096 1.7-2.7;
+// * rows of one step of the general kernel, five to eight vectors 16384 x 512
+//   0.8-0.9 / 0.8-0.9 / 1.0, 32000 x 512 1.3; more 4096 x 512 0.8-0.9 (F16 1.0), 8192 x
+//   512 1.1-1.2; F16 of 32 columns 32000 rows 0.9 and 1.3.
+bool general_sooner(int type, uint32_t rows, uint32_t cols, uint32_t batch) {
+    const bool f16 = type == kF16;
+    if (batch == 1u) return true;
+    if (batch <= 4u) {
+        if (f16 && batch == 2u) return true;
+        if (rows < 3072u || (rows == 3072u && (batch == 2u || cols < 8192u))) return true;
+        return cols < (f16 ? 8192u : type == kQ4_1 ? 2048u : 3072u);
+    }
+    if (cols <= 512u) {
+        if (f16) return cols < 64u ? batch <= 8u || rows < 24576u : rows < (batch <= 8u ? 16384u : 3072u);
+        return rows < (batch <= 8u ? 24576u : 8192u);
+    }
+    if (rows >= 3072u || (cols >= 2048u && rows * batch >= 32768u)) return false;
+    if (rows < 1024u || cols < 4096u) return true;
+    return rows * batch < (cols < 8192u ? 15360u : f16 ? 12288u : 5120u);
+}
+
 }  // namespace
 
 hipError_t launch_blk_linear_batch(int type, uint32_t nmat, const uint8_t *const w[], const uint32_t rows[],
@@ -379,16 +409,7 @@ hipError_t launch_blk_linear_batch(int type, uint32_t nmat, const uint8_t *const
         tiles += (rows[m] + 15u) / 16u;
         a.tile_end[m] = tiles;
     }
-    // One vector, or few rows, are done sooner by the general kernel's one launch
-    // (this path's two launches take 5 us at the least). Graph replays, matrix
-    // cores / general: one vector 4096 x 11008 Q8_0 17.7 / 15.0 us, F16 24.7 /
-    // 20.3; four, 2048 x 4096 Q8_0 9.3 / 7.5, 2048 x 11008 15.8 / 16.8, 4096 x
-    // 4096 10.0 / 15.8; eight, 512 x 11008 16.4 / 10.5, 1024 x 4096 9.4 / 8.5,
-    // 1024 x 11008 16.7 / 19.5, 2048 x 4096 9.8 / 11.1; sixteen, 512 x 4096 11.3 /
-    // 9.1, 1024 x 4096 11.3 / 12.5.
-    if (nmat == 1u && (batch == 1u || rows[0] <= (batch <= 4u ? 2048u : 512u) ||
-                       (batch <= 8u && rows[0] <= 1024u && cols <= 4096u)))
-        return hipErrorNotSupported;
+    if (nmat == 1u && general_sooner(type, rows[0], cols, batch)) return hipErrorNotSupported;
     const uint32_t pcols = (cols + 255u) & ~255u;
     hipError_t why;
     uint8_t *xp = static_cast<uint8_t *>(rt_scratch((size_t)((batch + kBatchMax - 1u) / kBatchMax) * xb_layout(pcols).bytes, s, &why));
