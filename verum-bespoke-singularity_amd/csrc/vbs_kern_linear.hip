@@ -359,7 +359,8 @@ hipError_t launch_rows_t(const uint8_t *w, const float *x, uint32_t xs, float *y
 // (29.1, 100), 11008 x 4128 42.1, 115 (55.9, 147).
 // Rows of no more steps than that split has waves leave waves idle, so short
 // rows take fewer: one wave at a step (512 elements; two for one vector and
-// 513-3072 rows), two rows a wave past 3072 rows, with as many sums as there are
+// 513-3072 rows), two rows a wave past 3072 rows (one vector past 16384 four:
+// 32000 x 96 F16 4.4 us, two 4.7), with as many sums as there are
 // vectors (us, before the split went by length -> now: F32 32000 x 32, 16 vectors
 // 99.9 -> 9.4, x 256 104 -> 24.1, 5000 x 96, 8 vectors 11.8 -> 4.2; Q4_0 512 x 96
 // one vector 2.69 -> 2.27, 1000 x 544 2.92 -> 2.56; one and four rows a wave
@@ -376,7 +377,7 @@ hipError_t launch_rows(const uint8_t *w, const float *x, uint32_t xs, float *y, 
         if (rows <= 512u) VBS_ROWS(1, 1, 16, 1);
         if (rows <= 3072u && cols <= 2048u) VBS_ROWS(2, 1, 4, 1);
         if (rows <= 3072u) VBS_ROWS(2, 1, 4, 2);
-        if (cols <= 512u) VBS_ROWS(2, 1, 1, 1);
+        if (cols <= 512u && rows <= 16384u) VBS_ROWS(2, 1, 1, 1);
         if (cols < 2048u) VBS_ROWS(4, 1, 1, 1);
         VBS_ROWS(4, 1, 4, 1);
     }
