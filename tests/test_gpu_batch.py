@@ -6,6 +6,7 @@ src/vbs_specializer.c:353-357), so the oracle of vbs_gfx950_linear_batch is
 every vector must meet the single matvec's bar, relative L2 <= 1e-5.
 """
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -312,3 +313,40 @@ def test_scratch_growth_keeps_captured_graphs(dev, host, oracle, mem):
     dev.linear_batch(t, pw, px, cols, py, rows, cols, rows, batch)
     Y = dev.download(py, (batch, rows), np.float32)
     assert lin_err(Y[0], want[0]) <= LIN_TOL
+
+
+def test_batch_calls_of_several_threads(dev, host, mem):
+    """Batched matvecs and a chunked attention issued by several threads at once
+    (they share the library's stream and scratch): every result has the bits
+    of the same call alone."""
+    calls = []
+    for i, (t, rows, cols, batch) in enumerate([(V.Q8_0, 3072, 1280, 8), (V.Q4_1, 4096, 1024, 16),
+                                                (V.F16, 3104, 2048, 6), (V.Q4_K, 512, 2048, 8)]):
+        pw, px = mem.up(V.synth_matrix(host, t, rows, cols, SEED, 210 + i)), mem.up(vectors(host, batch, cols, 220 + 20 * i))
+        py = mem.zeros(batch * rows)
+        calls.append((lambda a=(t, pw, px, cols, py, rows, cols, rows, batch): dev.linear_batch(*a), py, batch * rows))
+    nqh, nkh, hd, seq = 16, 2, 64, 3000
+    pk = mem.up(V.synth_normal_f16(host, seq * nkh * hd, SEED, 230))
+    pq, po = mem.up(synth_x(host, nqh * hd, 231)), mem.zeros(nqh * hd)
+    calls.append((lambda: dev.attention(pq, pk, pk, po, seq, 0, seq, nqh, nkh, hd, np.float32(0.125)), po, nqh * hd))
+    want = []
+    for call, p, n in calls:
+        call()
+        want.append(dev.download(p, n, np.float32))
+    for _ in range(10):
+        for _, p, n in calls:
+            dev.write(p, np.full(n, 7.0, np.float32))
+        go = threading.Barrier(len(calls))
+
+        def work(call):
+            go.wait()
+            for _ in range(20):
+                call()
+
+        threads = [threading.Thread(target=work, args=(c[0],)) for c in calls]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        for (_, p, n), w in zip(calls, want):
+            assert np.array_equal(dev.download(p, n, np.float32).view(np.uint32), w.view(np.uint32))

@@ -46,6 +46,9 @@ struct Runtime {
 
 Runtime g_rt;
 char g_err[512] = "not initialised";
+// Held by the entry points whose launches hand data to each other through the
+// library's scratch, so that calls of several threads don't come between them.
+std::mutex g_scratch_mu;
 
 int fail(const char *fmt, ...) {
     va_list ap;
@@ -526,6 +529,7 @@ int vbs_gfx950_linear_batch(int type, const void *w, const float *x, uint32_t x_
     if (batch > 16) return fail("linear_batch: batch %u exceeds 16", batch);
     if (x_stride < cols || y_stride < rows) return fail("linear_batch: stride smaller than row");
     if (!w || !x || !y) return fail("linear_batch: null pointer");
+    const std::lock_guard<std::mutex> together(g_scratch_mu);
     return hip_ok(launch_linear_batch(type, (const uint8_t *)w, x, x_stride, y, y_stride, cols,
                                       rows, batch, g_rt.stream),
                   "linear_batch");
@@ -554,6 +558,7 @@ int vbs_gfx950_linear_batch_multi(int type, uint32_t n_mat, const void *const *w
         rm[m] = rows[m];
         ysm[m] = y_stride[m];
     }
+    const std::lock_guard<std::mutex> together(g_scratch_mu);
     return hip_ok(launch_linear_batch_multi(type, n_mat, wm, rm, x, x_stride, ym, ysm, cols, batch,
                                             g_rt.stream),
                   "linear_batch_multi");
@@ -632,6 +637,7 @@ int vbs_gfx950_attention(const float *q, const uint16_t *kc, const uint16_t *vc,
     if (!ready_or_fail()) return 0;
     if (!attention_args_ok("attention", q, kc, vc, out, seq_len, max_ctx, nqh, nkh, hd)) return 0;
     uint64_t layer_off = (uint64_t)layer * max_ctx * nkh * hd;
+    const std::lock_guard<std::mutex> together(g_scratch_mu);
     return hip_ok(launch_attention(q, kc, vc, out, seq_len, nullptr, nullptr, layer_off, nqh, nkh,
                                    hd, scale, g_rt.stream),
                   "attention");
@@ -651,6 +657,7 @@ int vbs_gfx950_attention_noalloc(const float *q, const uint16_t *kc, const uint1
     // every partial the merge reads is written by the same call's chunk
     // kernels first, so the scratch needs no clearing between calls
     uint64_t layer_off = (uint64_t)layer * max_ctx * nkh * hd;
+    const std::lock_guard<std::mutex> together(g_scratch_mu);
     return hip_ok(launch_attention(q, kc, vc, out, seq_len, nullptr,
                                    static_cast<float *>(g_rt.noalloc_scratch), layer_off, nqh,
                                    nkh, hd, scale, g_rt.stream),
