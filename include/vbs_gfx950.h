@@ -253,15 +253,19 @@ int vbs_gfx950_checksum_variant(const void *p, size_t bytes, uint32_t *partials,
 /* The library's stream (a hipStream_t), for callers that time kernels with
  * HIP events or capture the stream into a graph.
  *
- * Capture and the library's scratch: vbs_gfx950_linear_batch (Q4_K / Q6_K; the
- * other types run without it where it cannot grow) and vbs_gfx950_attention keep intermediate results in a device scratch
- * that the library owns. It only grows, and a buffer that a larger call
- * replaces stays allocated until the process ends, so a captured graph keeps
- * valid memory whatever is called after the capture. Growing allocates, so a
- * call made while the stream is being captured fails (0, reason "operation
+ * Capture and the library's scratch: vbs_gfx950_linear_batch (Q4_K / Q6_K) and
+ * vbs_gfx950_attention keep intermediate results in a device scratch that the
+ * library owns. It only grows, and a buffer that a larger call replaces stays
+ * allocated until the process ends, so a captured graph keeps valid memory
+ * whatever is called after the capture; but graphs that use it must not run
+ * beside each other or beside such calls on another stream. Growing allocates,
+ * so a call made while the stream is being captured fails (0, reason "operation
  * not permitted when stream is capturing") if it needs more scratch than
  * earlier uncaptured calls have sized: make one uncaptured call of the
- * largest shape before capturing. */
+ * largest shape before capturing. Batched Q4_0, Q4_1, Q8_0 and F16 calls take
+ * memory of the graph's own while captured, at any size, which is given back
+ * with the graph and its executables: such graphs may run beside each other
+ * and beside any call. */
 void *vbs_gfx950_stream(void);
 
 /* ---- graph-replayed decode step (extension) -------------------------------

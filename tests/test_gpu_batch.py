@@ -350,3 +350,83 @@ def test_batch_calls_of_several_threads(dev, host, mem):
             th.join()
         for (_, p, n), w in zip(calls, want):
             assert np.array_equal(dev.download(p, n, np.float32).view(np.uint32), w.view(np.uint32))
+
+
+def test_batch_graphs_beside_each_other(dev, host, mem):
+    """Captured batched matvecs of the block types, replayed on two streams at
+    once and beside uncaptured calls: each keeps its prepared vectors in its
+    own graph's memory, so every result has the uncaptured call's bits."""
+    hip, stream = V.Hip(), dev.stream()
+    hip.h.hipStreamCreateWithFlags.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_uint]
+    hip.h.hipStreamSynchronize.argtypes = hip.h.hipStreamDestroy.argtypes = [ctypes.c_void_p]
+    calls, want, graphs, streams = [], [], [], []
+    for i, (t, rows, cols, batch) in enumerate([(V.Q8_0, 3072, 1280, 8), (V.Q4_1, 4096, 1280, 16),
+                                                (V.Q4_0, 3072, 1280, 5)]):
+        pw, px = mem.up(V.synth_matrix(host, t, rows, cols, SEED, 240 + i)), mem.up(vectors(host, batch, cols, 250 + 20 * i))
+        py = mem.zeros(batch * rows)
+        calls.append((lambda a=(t, pw, px, cols, py, rows, cols, rows, batch): dev.linear_batch(*a), py, batch * rows))
+        calls[-1][0]()
+        want.append(dev.download(py, batch * rows, np.float32))
+    try:
+        for call, _, _ in calls[:2]:
+            graphs.append(hip.capture(stream, lambda: [call() for _ in range(20)]))
+            s = ctypes.c_void_p()
+            assert hip.h.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+            streams.append(s.value)
+        for _ in range(10):
+            for _, p, n in calls:
+                dev.write(p, np.full(n, 7.0, np.float32))
+            dev.sync()
+            for g, s in zip(graphs, streams):
+                hip.launch(g, s)
+            for _ in range(20):
+                calls[2][0]()
+            for s in streams:
+                assert hip.h.hipStreamSynchronize(s) == 0
+            for (_, p, n), w in zip(calls, want):
+                assert np.array_equal(dev.download(p, n, np.float32).view(np.uint32), w.view(np.uint32))
+    finally:
+        for g in graphs:
+            hip.destroy(g)
+        for s in streams:
+            hip.h.hipStreamDestroy(s)
+
+
+def test_batch_capture_needs_no_sizing_call(dev, host, oracle, mem):
+    """A capture of calls whose prepared vectors (17 MB and 9 MB) no uncaptured
+    call has sized: the graph's bits are those of the calls alone, replay after
+    replay; captured again and again, its memory is given back."""
+    hip, stream = V.Hip(), dev.stream()
+    hip.h.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+
+    def free_bytes():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.h.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    t, rows, cols, batch = V.Q4_0, 1040, 262144, 16
+    w = V.synth_matrix(host, t, rows, cols, SEED, 280)
+    X = vectors(host, batch, cols, 281)
+    pw, px, py = mem.up(w), mem.up(X), mem.zeros(batch * rows)
+
+    def enqueue():
+        dev.linear_batch(t, pw, px, cols, py, rows, cols, rows, 8)  # (and a smaller one before it)
+        dev.linear_batch(t, pw, px, cols, py, rows, cols, rows, batch)
+
+    before, got = free_bytes(), []
+    for rep in range(12):
+        graph = hip.capture(stream, enqueue)
+        for _ in range(2):
+            dev.write(py, np.zeros(batch * rows, np.float32))
+            hip.launch(graph, stream)
+            got.append(dev.download(py, (batch, rows), np.float32))
+        hip.destroy(graph)
+        dev.sync()
+    assert before - free_bytes() <= 8 * (48 << 20)  # (the graphs', idle ones among them; each holds 16 + 32 MiB)
+    dev.linear_batch(t, pw, px, cols, py, rows, cols, rows, batch)
+    alone = dev.download(py, (batch, rows), np.float32)
+    for Y in got:
+        assert np.array_equal(Y.view(np.uint32), alone.view(np.uint32))
+    ws = np.ascontiguousarray(w[:32])
+    for b in (0, 9, 15):
+        assert lin_err(alone[b, :32], oracle.linear(t, ws, X[b], cols, 32)) <= LIN_TOL, b

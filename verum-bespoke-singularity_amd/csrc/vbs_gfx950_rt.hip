@@ -12,6 +12,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <new>
 #include <thread>
 
 #include "vbs_dev_common.h"
@@ -137,9 +138,106 @@ void *rt_scratch(size_t bytes, hipStream_t s, hipError_t *why) {
     return p;
 }
 
+// Scratch for the calls that a capture may record at any size. A graph may be
+// replayed beside other graphs and calls, on any stream, so what its nodes hand
+// to each other is memory of its own: one buffer per capture (its nodes on the
+// library's stream run one after the other), which a user object of the graph
+// gives back when the graph, its clones and its executables are gone. Given-back
+// buffers wait for later captures; uncaptured calls trim them to kIdleMax.
+struct CaptureBuffer {
+    void *p;
+    size_t bytes;
+    CaptureBuffer *next;
+};
+static std::mutex g_idle_mu;
+static CaptureBuffer *g_idle = nullptr;
+constexpr int kIdleMax = 8;
+
+static void capture_buffer_idle(void *b) {  // (the user object's destructor: no HIP calls here)
+    CaptureBuffer *c = static_cast<CaptureBuffer *>(b);
+    const std::lock_guard<std::mutex> lock(g_idle_mu);
+    c->next = g_idle;
+    g_idle = c;
+}
+
+// An idle buffer of `bytes`, the smallest there is; with trim, those past the first kIdleMax.
+static CaptureBuffer *idle_buffer(size_t bytes, bool trim) {
+    const std::lock_guard<std::mutex> lock(g_idle_mu);
+    CaptureBuffer **at = nullptr;
+    int n = 0;
+    for (CaptureBuffer **c = &g_idle; *c; c = &(*c)->next) {
+        if (trim ? n++ == kIdleMax : (*c)->bytes >= bytes && (!at || (*c)->bytes < (*at)->bytes)) at = c;
+    }
+    if (!at) return nullptr;
+    CaptureBuffer *c = *at;
+    *at = c->next;
+    return c;
+}
+
+void *rt_scratch_or_captured(size_t bytes, hipStream_t s, hipError_t *why) {
+    static unsigned long long cur_id = 0;  // the capture that `cur` belongs to
+    static CaptureBuffer *cur = nullptr;
+    static bool any = false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    hipGraph_t graph = nullptr;
+    const hipGraphNode_t *deps = nullptr;
+    size_t n_deps = 0;
+    *why = hipStreamGetCaptureInfo_v2(s, &st, &id, &graph, &deps, &n_deps);
+    if (*why != hipSuccess) return nullptr;
+    if (st == hipStreamCaptureStatusNone) {
+        while (any) {
+            CaptureBuffer *c = idle_buffer(0, true);
+            if (!c) break;
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+            (void)hipFree(c->p);
+            if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+            delete c;
+        }
+        return rt_scratch(bytes, s, why);
+    }
+    if (st != hipStreamCaptureStatusActive) {
+        *why = hipErrorStreamCaptureInvalidated;
+        return nullptr;
+    }
+    if (cur && cur_id == id && cur->bytes >= bytes) return cur->p;
+    size_t want = 1u << 16;
+    while (want < bytes) want *= 2;
+    CaptureBuffer *c = idle_buffer(want, false);
+    if (!c) {
+        void *p = nullptr;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (else an allocation ends the capture)
+        if ((*why = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return nullptr;
+        *why = hipMalloc(&p, want);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (*why != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        c = new (std::nothrow) CaptureBuffer{p, want, nullptr};
+        if (!c) {
+            *why = hipErrorOutOfMemory;  // (the buffer is lost with the host's memory)
+            return nullptr;
+        }
+    }
+    hipUserObject_t owner = nullptr;
+    *why = hipUserObjectCreate(&owner, c, capture_buffer_idle, 1, hipUserObjectNoDestructorSync);
+    if (*why != hipSuccess) {
+        capture_buffer_idle(c);
+        return nullptr;
+    }
+    if ((*why = hipGraphRetainUserObject(graph, owner, 1, hipGraphUserObjectMove)) != hipSuccess) {
+        (void)hipUserObjectRelease(owner, 1);
+        return nullptr;
+    }
+    any = true;
+    cur_id = id;
+    cur = c;
+    return c->p;
+}
+
 hipStream_t rt_stream() { return g_rt.stream; }
-
-
 
 int rt_fail(const char *fmt, ...) {
     va_list ap;

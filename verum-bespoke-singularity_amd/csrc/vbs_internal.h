@@ -21,6 +21,9 @@ uint32_t block_elems(int type);
 // hipErrorStreamCaptureUnsupported while `s` is being captured (growing
 // allocates), hipErrorOutOfMemory otherwise.
 void *rt_scratch(size_t bytes, hipStream_t s, hipError_t *why);
+// The same, but while `s` is being captured a buffer of the capture's own, which
+// lives as long as its graph. The caller holds the entry points' scratch mutex.
+void *rt_scratch_or_captured(size_t bytes, hipStream_t s, hipError_t *why);
 
 // The library's stream, and the last-error writer of the C ABI.
 hipStream_t rt_stream();

@@ -412,8 +412,9 @@ hipError_t launch_blk_linear_batch(int type, uint32_t nmat, const uint8_t *const
     if (nmat == 1u && general_sooner(type, rows[0], cols, batch)) return hipErrorNotSupported;
     const uint32_t pcols = (cols + 255u) & ~255u;
     hipError_t why;
-    uint8_t *xp = static_cast<uint8_t *>(rt_scratch((size_t)((batch + kBatchMax - 1u) / kBatchMax) * xb_layout(pcols).bytes, s, &why));
-    if (!xp) return hipErrorNotSupported;  // (no room, or none to be had under capture)
+    const size_t need = (size_t)((batch + kBatchMax - 1u) / kBatchMax) * xb_layout(pcols).bytes;
+    uint8_t *xp = static_cast<uint8_t *>(rt_scratch_or_captured(need, s, &why));
+    if (!xp) return hipErrorNotSupported;  // (no memory for it: the general kernel needs none)
     a.nmat = nmat;
     a.xp = xp;
     a.x = x;
