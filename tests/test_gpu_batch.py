@@ -264,6 +264,73 @@ def test_batch_block_types_non_finite(dev, host, oracle, mem, t):
             assert lin_err(Y[b][fine], want[fine]) <= LIN_TOL, b
 
 
+def run_multi(dev, mem, t, ws, X, shapes, cols, base=0):
+    """Y of each matrix through one matrix-core launch, the matrices at a base
+    that is only `base` bytes past 16-byte alignment."""
+    batch = X.shape[0]
+    pws = [mem.up(np.concatenate([np.zeros(base, np.uint8), w.reshape(-1)])) + base for w in ws]
+    pys = [mem.zeros(batch * r) for r in shapes]
+    dev.linear_batch_multi(t, pws, shapes, mem.up(X), cols, pys, shapes, cols, batch)
+    return [dev.download(py, (batch, r), np.float32) for py, r in zip(pys, shapes)]
+
+
+# (test_batch_block_types' [1], [16], [300] and [4097] and the one matrix of
+# test_batch_block_types_non_finite run in the general kernel; several matrices
+# always take k_mvbb)
+@pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
+@pytest.mark.parametrize("batch", [1, 6, 11])
+def test_batch_mfma_non_finite(dev, host, oracle, mem, t, batch):
+    """Infinities and NaN on the matrix cores: in vectors, and as scales,
+    weights and Q4_1 mins, also in a row's partly filled last unit, give the
+    oracle's inf and NaN; every other result stays within the bar."""
+    shapes, cols = [40, 33], 1056
+    ws = [V.synth_matrix(host, t, r, cols, SEED, 260 + m) for m, r in enumerate(shapes)]
+    bb = V.GEOMETRY[t][1]
+    f16 = lambda v: np.array([v], np.uint16).view(np.uint8)  # noqa: E731
+    ws[0][3, :2], ws[0][39, -bb:][:2], ws[1][7, -bb:][:2] = f16(0x7C00), f16(0x7C00), f16(0x7E00)
+    if t == V.Q4_1:
+        ws[1][32, -bb + 2:][:2] = f16(0xFC00)
+    X = vectors(host, batch, cols, 270)
+    X[0, 300] = np.inf
+    if batch > 1:
+        X[2, 1040], X[4, 1055], X[batch - 1, 0] = np.nan, -np.inf, np.inf
+    for w, r, Y in zip(ws, shapes, run_multi(dev, mem, t, ws, X, shapes, cols)):
+        for b in range(batch):
+            with np.errstate(invalid="ignore"):
+                want = oracle.linear(t, w, X[b], cols, r)
+            fine = np.isfinite(want)
+            assert np.array_equal(np.isnan(Y[b]), np.isnan(want)), b
+            assert np.array_equal(Y[b][np.isinf(want)], want[np.isinf(want)]), b
+            if fine.any():
+                assert lin_err(Y[b][fine], want[fine]) <= LIN_TOL, b
+
+
+@pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
+@pytest.mark.parametrize("base", [0, 2, 6, 14])
+def test_batch_mfma_activation_edges(dev, host, oracle, mem, t, base):
+    """The per-unit scaling of the block types' vectors (all zero, 1e-30, 1e30,
+    outliers, zero and subnormal sub-blocks) with the matrices at every kind of
+    2-byte base (F16 off 16 bytes takes the general kernel)."""
+    shapes, cols = [70, 17], 1120
+    ws = [V.synth_matrix(host, t, r, cols, SEED, 290 + m) for m, r in enumerate(shapes)]
+    X = vectors(host, 8, cols, 300)
+    X[0] = 0.0
+    X[1] *= 1e-30
+    X[2] *= 1e30
+    X[3, 40] = 1.0e4
+    X[4, 0:32] = 0.0
+    X[4, 64:96] *= 1e-40
+    X[5, 96:128] *= 1e30
+    X[6, 7] = -0.0
+    X[7, 1100:] *= 1e-38
+    for w, r, Y in zip(ws, shapes, run_multi(dev, mem, t, ws, X, shapes, cols, base)):
+        assert np.all(Y[0] == 0.0)
+        for b in range(1, 8):
+            want = oracle.linear(t, w, X[b], cols, r)
+            assert np.all(np.isfinite(Y[b])), b
+            assert lin_err(Y[b], want) <= LIN_TOL, b
+
+
 def test_scratch_growth_keeps_captured_graphs(dev, host, oracle, mem):
     """The batched matvec keeps its prepared x in the library's scratch. A
     graph captured from the library's stream holds the scratch address of the

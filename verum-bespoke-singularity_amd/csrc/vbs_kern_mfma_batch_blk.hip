@@ -35,10 +35,13 @@
 // About 6 us of each is the fixed cost of the two launches.
 // Error against 64 bits 0.7 to 1.3e-7 (the VALU kernel's 1.0 to 2.4e-7).
 //
-// Values that are not finite (an inf or NaN in x makes its whole block's
-// planes NaN here) are computed again by the general kernel's arithmetic, so
-// such vectors and weights give what k_rows gives.
+// Results that are not finite (an inf or NaN in x makes its whole block's
+// planes NaN here) are computed again by a wave each in the general kernel's
+// arithmetic, a row on one wave: such vectors and weights give the oracle's inf
+// and NaN (a NaN in one of eight vectors: Q8_0 4096 x 4096 37 us; by one lane per
+// result it took 1163).
 #include "vbs_mfma_batch.h"
+#include "vbs_row8.h"
 
 namespace vbs {
 
@@ -77,8 +80,9 @@ __global__ __launch_bounds__(256) void k_xprep_r(const float *x, uint32_t xs, ui
 }
 
 // ---- weight types -----------------------------------------------------------------------
-template <int TYPE>
+template <int BLK>
 struct BlkB {
+    static constexpr int TYPE = BLK;
     typedef KBlk<TYPE> K;
     static constexpr uint32_t BB = K::BB, QOFF = K::QOFF, BYTES = K::BYTES, CH = K::CH, NLD = K::NLD;
     static constexpr uint32_t SCRATCH = K::SCRATCH;
@@ -156,14 +160,12 @@ struct BlkB {
             }
         }
     }
-    __device__ static float weight(const uint8_t *row, uint32_t c) {
-        return deq_elem<TYPE>(row + (uint64_t)(c / 32u) * BB, c & 31u);
-    }
 };
 
 // F16 rows of a multiple of 8 elements at 16-byte alignment: the operands are
 // loaded where they are used, no LDS.
 struct F16B {
+    static constexpr int TYPE = kF16;
     static constexpr uint32_t BYTES = 512, NLD = 8, SCRATCH = 0;
     static constexpr bool MINS = false;
     __device__ static void load(const Src &src, uint32_t u, uint32_t cols, uint32_t n, uint32_t g,
@@ -195,8 +197,30 @@ struct F16B {
             acc[v][1] += S[2] + S[3];
         }
     }
-    __device__ static float weight(const uint8_t *row, uint32_t c) { return h2f(ld16(row + 2u * c)); }
 };
+
+// A row times x in f32 by the whole wave, as k_rows has a row on one wave.
+template <int T>
+__device__ __forceinline__ float row_whole(const uint8_t *row, const float *x, uint32_t cols, uint32_t lane) {
+    typedef Row8<T> R;
+    constexpr uint32_t L = R::E / 8u;
+    const uint32_t q = lane % L;
+    float acc = 0.f;
+#pragma unroll 2
+    for (uint32_t u = lane / L; u < cols / R::E; u += 64u / L) {
+        const f4u *x0 = reinterpret_cast<const f4u *>(x + R::E * u + R::lo(q));
+        const f4u *x1 = reinterpret_cast<const f4u *>(x + R::E * u + R::hi(q));
+        const typename R::Raw raw = R::raw(row, u, q);
+        const v4f a = *x0, b = *x1;
+        float w[8], s = 0.f;
+        R::value(raw, w);
+        const float xv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) s = fmaf(w[e], xv[e], s);
+        acc += s;
+    }
+    return wave_sum(acc);
+}
 
 template <class P, uint32_t T, uint32_t VG>
 __global__ __launch_bounds__(512) void k_mvbb(const MbbArgs a) {
@@ -308,24 +332,26 @@ __global__ __launch_bounds__(512) void k_mvbb(const MbbArgs a) {
             red[(j * nw + wave) * 128u + 2u * lane + 1u] = acc[j][v][1];
         }
         __syncthreads();
-        for (uint32_t q = threadIdx.x; q < T * 128u; q += blockDim.x) {
+        for (uint32_t q = threadIdx.x; q < T * 128u; q += blockDim.x) {  // (a wave's q are 64 in a row)
             const uint32_t j = q >> 7, l = (q >> 1) & 63u, tk = q & 1u;
             float s = 0.f;
             for (uint32_t w = 0; w < nw; w++) s += red[(j * nw + w) * 128u + 2u * l + tk];
             const uint32_t gt = blockIdx.x * T + j;
-            if (gt >= total) continue;
             const uint32_t m = (uint32_t)(gt >= a.tile_end[0]) + (uint32_t)(a.nmat > 2u && gt >= a.tile_end[1]);
             const uint32_t row = 16u * (gt - (m == 0u ? 0u : m == 1u ? a.tile_end[0] : a.tile_end[1])) + (l & 15u);
             const uint32_t rows = m == 0u ? a.rows[0] : m == 1u ? a.rows[1] : a.rows[2];
             const uint32_t t = kBatchMax * v + 2u * (l >> 4) + tk;
-            if (row >= rows || t >= a.batch) continue;
-            if (!(fabsf(s) <= 3.4028235e38f)) {
-                const uint8_t *const w = (m == 0u ? a.w[0] : m == 1u ? a.w[1] : a.w[2]) + (uint64_t)row * rb;
-                const float *const xt = a.x + (uint64_t)t * a.xs;
-                s = 0.f;
-                for (uint32_t c = 0; c < cols; c++) s = fmaf(P::weight(w, c), xt[c], s);
+            const bool ours = gt < total && row < rows && t < a.batch;
+            for (uint64_t bad = __ballot(ours && !(fabsf(s) <= 3.4028235e38f)); __builtin_expect(bad != 0u, 0); bad &= bad - 1u) {
+                const int who = __ffsll((unsigned long long)bad) - 1;
+                const uint32_t bm = __builtin_amdgcn_readlane(m, who), br = __builtin_amdgcn_readlane(row, who);
+                const uint32_t bt = __builtin_amdgcn_readlane(t, who);
+                const float again = row_whole<P::TYPE>((bm == 0u ? a.w[0] : bm == 1u ? a.w[1] : a.w[2]) + (uint64_t)br * rb,
+                                                       a.x + (uint64_t)bt * a.xs, cols, lane);
+                if ((int)lane == who) s = again;
             }
-            (m == 0u ? a.y[0] : m == 1u ? a.y[1] : a.y[2])[(uint64_t)t * (m == 0u ? a.ys[0] : m == 1u ? a.ys[1] : a.ys[2]) + row] = s;
+            if (ours)
+                (m == 0u ? a.y[0] : m == 1u ? a.y[1] : a.y[2])[(uint64_t)t * (m == 0u ? a.ys[0] : m == 1u ? a.ys[1] : a.ys[2]) + row] = s;
         }
     }
 }
