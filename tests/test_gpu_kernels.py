@@ -844,6 +844,32 @@ def test_attention_non_finite_cache(dev, host, oracle, mem, hd, nqh, nkh, seq, w
     assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-4 * np.abs(want[fine]))
 
 
+@pytest.mark.parametrize("hd,nqh,nkh,seq", [(64, 80, 80, 300), (32, 160, 80, 700), (64, 100, 100, 1500),
+                                            (32, 81, 81, 2048), (96, 160, 160, 512), (96, 330, 165, 1024)])
+def test_attention_non_finite_many_kv_heads(dev, host, oracle, mem, hd, nqh, nkh, seq):
+    """The one-launch kernel over more than 256 positions (many kv heads take
+    longer chunks): an infinite value and a -inf score near the end leave a
+    head the sums over all of its positions."""
+    kc = V.synth_normal_f16(host, seq * nkh * hd, SEED, 181)
+    vc = V.synth_normal_f16(host, seq * nkh * hd, SEED, 182)
+    k, v = (c.reshape(seq, nkh, hd) for c in (kc, vc))
+    k[3, ::2, 5] = 0xFC00
+    k[seq - 30, 1::2, 4] = 0x7C00
+    v[seq - 20, :, 3] = 0x7C00
+    v[9, ::3, hd - 1] = 0xFC00
+    q = synth_x(host, nqh * hd, 183)
+    scale = np.float32(1.0 / math.sqrt(hd))
+    po = mem.zeros(nqh * hd)
+    dev.attention(mem.up(q), mem.up(kc), mem.up(vc), po, seq, 0, seq, nqh, nkh, hd, scale)
+    got = dev.download(po, nqh * hd, np.float32)
+    want = oracle.attention(q, kc, vc, seq, 0, seq, nqh, nkh, hd, scale)
+    fine = np.isfinite(want)
+    assert fine.any() and np.isinf(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-4 * np.abs(want[fine]))
+
+
 @pytest.mark.parametrize("hd", [32, 64, 96])
 @pytest.mark.parametrize("nqh,nkh", [(1, 1), (5, 1), (4, 2), (16, 4), (3, 3), (24, 8)])
 @pytest.mark.parametrize("seq", [257, 4097, 8200, 12300, 33000])

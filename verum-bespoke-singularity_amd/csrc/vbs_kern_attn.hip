@@ -810,9 +810,22 @@ __global__ __launch_bounds__(64 * kOneChunks) void k_attn_one(
 #pragma unroll 1
             for (uint32_t h = wave; h < group; h += nw) {
                 if (!((again >> h) & 1u)) continue;
-                float m, l, w[DPL];
-                attn_head_whole<HD>(q + ((uint64_t)kvh * group + h) * HD, kc, vc, layer_off + (uint64_t)kvh * HD,
-                                    seq_len, (uint64_t)nkh * HD, scale, lane, m, l, w);
+                // (many kv heads have longer chunks, and more positions than attn_head_whole takes at once)
+                float m = -INFINITY, l = 0.f, w[DPL] = {};
+#pragma unroll 1
+                for (uint32_t p0 = 0; p0 < seq_len; p0 += kMfmaLmax) {
+                    float mp, lp, wp[DPL];
+                    attn_head_whole<HD>(q + ((uint64_t)kvh * group + h) * HD, kc, vc,
+                                        layer_off + ((uint64_t)p0 * nkh + kvh) * HD, min(kMfmaLmax, seq_len - p0),
+                                        (uint64_t)nkh * HD, scale, lane, mp, lp, wp);
+                    const float mn = fmaxf(m, mp);
+                    const float r = m == -INFINITY ? 0.f : ldexpf(1.f, (int)(m - mn));
+                    const float rp = mp == -INFINITY ? 0.f : ldexpf(1.f, (int)(mp - mn));
+                    m = mn;
+                    l = fmaf(lp, rp, l * r);
+#pragma unroll
+                    for (uint32_t dt = 0; dt < DPL; dt++) w[dt] = fmaf(wp[dt], rp, w[dt] * r);
+                }
                 float2 r = make_float2(0.f, 0.f);
 #pragma unroll
                 for (uint32_t i = 0; i < DPL / 2u; i++) {
