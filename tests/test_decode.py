@@ -17,6 +17,7 @@ vbs_oracle_forward_token, following src/vbs_specializer.c:231-349).
   pinned bit for bit on the CPU, and 32 teacher-forced positions against the
   oracle's logits.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -455,6 +456,49 @@ def test_gpu_graph_decoder_tiny_greedy_matches_oracle(host, backend, dev, tiny):
     assert np.array_equal(toks, want_toks)
     assert np.array_equal(etoks, toks)
     assert np.array_equal(emargins.view(np.uint32), margins.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("off", [0, 1, 4, 4093])
+def test_gpu_decoder_results_to_pinned_memory(host, backend, dev, tiny, off):
+    """Results in the caller's pinned memory, from any word of it on, are those
+    that a pageable destination gets, and the words beside them stay; also for
+    a batch, whose tokens, margins and logits go to one allocation, and where
+    the results run past the allocation's last whole block of four words."""
+    hip = V.Hip().h
+    hip.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+    hip.hipHostFree.argtypes = [ctypes.c_void_p]
+    d = V.Decoder(host, backend, tiny)
+    g, b, vocab = V.GraphDecoder(dev, d, max_steps=3), V.BatchDecoder(dev, d, 3, max_steps=3), tiny.cfg["vocab"]
+    total, p = off + 3 * vocab + 7, ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(p), 4 * total, 0) == 0
+    try:
+        words = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_uint32)), (total,))
+        at = p.value + 4 * off
+
+        def results(n):
+            got = words[off:off + n].copy()
+            assert np.all(words[:off] == 0xABCD1234) and np.all(words[off + n:] == 0xABCD1234)
+            words[:] = 0xABCD1234
+            return got
+
+        words[:] = 0xABCD1234
+        want = g.step(5, 0)
+        dev.check(dev._decoder_step(g.h, 5, 0, at), "decoder_step")
+        assert np.array_equal(results(vocab), want.view(np.uint32))
+        want = b.step([1, 2, 3], [0, 0, 0])
+        t, q = np.array([1, 2, 3], np.uint32), np.zeros(3, np.uint32)
+        dev.check(dev._bdecoder_step(b.h, t.ctypes.data, q.ctypes.data, at), "bdecoder_step")
+        assert np.array_equal(results(3 * vocab), want.reshape(-1).view(np.uint32))
+        toks, margins = b.greedy([1, 2, 3], [0, 0, 0], 3)
+        dev.check(dev._bdecoder_greedy(b.h, t.ctypes.data, q.ctypes.data, 3, at, at + 4 * 9), "bdecoder_greedy")
+        got = results(18)
+        assert np.array_equal(got[:9], toks.reshape(-1)) and np.array_equal(got[9:], margins.reshape(-1).view(np.uint32))
+    finally:
+        hip.hipHostFree(p)
+        b.close()
+        g.close()
+        d.close()
 
 
 @pytest.mark.gpu
