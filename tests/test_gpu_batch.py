@@ -244,6 +244,22 @@ def test_batch_block_types_rule(dev, host, oracle, mem, t, rows, cols, batch):
 
 
 @pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
+@pytest.mark.parametrize("shapes,cols,batch", [
+    ([1000, 24], 2080, 4), ([1000, 25], 2080, 4), ([2000, 48], 2048, 3), ([1025, 1024], 2048, 3), ([3000, 2000], 512, 4),
+    ([3000, 2000], 544, 4), ([1500, 548], 5120, 1), ([2000, 2096], 4096, 1), ([2000, 2096], 4128, 1), ([9000, 7400], 288, 1),
+    ([9000, 7384], 1056, 1), ([9000, 7384], 1056, 2), ([300, 212], 4096, 8), ([300, 213], 4096, 5), ([300, 70], 4096, 9),
+    ([300, 70, 142], 4096, 2), ([300, 70, 143], 4096, 1), ([300, 70, 20], 4096, 3), ([3000, 1000, 96], 4096, 1)])
+def test_batch_multi_rule(dev, host, oracle, mem, t, shapes, cols, batch):
+    """Two and three matrices on both sides of each limit between the general
+    kernel and the matrix cores."""
+    ws = [V.synth_matrix(host, t, r, cols, SEED, 186 + m) for m, r in enumerate(shapes)]
+    X = vectors(host, batch, cols, 197)
+    for w, r, Y in zip(ws, shapes, run_multi(dev, mem, t, ws, X, shapes, cols)):
+        for b in range(batch):
+            assert lin_err(Y[b], oracle.linear(t, w, X[b], cols, r, threads=8)) <= LIN_TOL, b
+
+
+@pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
 def test_batch_block_types_non_finite(dev, host, oracle, mem, t):
     """inf and NaN in a vector and in a row's scales give the oracle's inf and
     NaN rows; the other vectors and rows stay within the bar."""
@@ -275,15 +291,15 @@ def run_multi(dev, mem, t, ws, X, shapes, cols, base=0):
 
 
 # (test_batch_block_types' [1], [16], [300] and [4097] and the one matrix of
-# test_batch_block_types_non_finite run in the general kernel; several matrices
-# always take k_mvbb)
+# test_batch_block_types_non_finite run in the general kernel, as do two matrices
+# of few rows and at most four vectors; three of such rows take k_mvbb)
 @pytest.mark.parametrize("t", BLK, ids=lambda t: V.TYPE_NAMES[t])
 @pytest.mark.parametrize("batch", [1, 6, 11])
 def test_batch_mfma_non_finite(dev, host, oracle, mem, t, batch):
     """Infinities and NaN on the matrix cores: in vectors, and as scales,
     weights and Q4_1 mins, also in a row's partly filled last unit, give the
     oracle's inf and NaN; every other result stays within the bar."""
-    shapes, cols = [40, 33], 1056
+    shapes, cols = [40, 33, 5], 1056
     ws = [V.synth_matrix(host, t, r, cols, SEED, 260 + m) for m, r in enumerate(shapes)]
     bb = V.GEOMETRY[t][1]
     f16 = lambda v: np.array([v], np.uint16).view(np.uint8)  # noqa: E731

@@ -413,6 +413,34 @@ bool general_sooner(int type, uint32_t rows, uint32_t cols, uint32_t batch) {
     return rows * batch < (cols < 8192u ? 15360u : f16 ? 12288u : 5120u);
 }
 
+// The same for two or three matrices, a launch of the general kernel (or its own
+// matrix-core pair) each, against this path's two launches for all. Over their
+// times (us, of this path / one by one; two matrices of R rows each):
+// * two to four vectors: R = 512 x 14336 Q4_0 15.2 / 10.6 and 15.4 / 14.6, R = 1024 x
+//   2048 7.4 / 6.3 and 7.5 / 7.0, R = 4096 x 512 7.2 / 5.8 and 7.3 / 6.8; but R = 2048 x
+//   2048 7.7 / 7.4 and 7.7 / 7.9, R = 1024 x 8192 11.3 / 12.2 and 11.3 / 13.3; F16, two
+//   vectors R = 1024 x 8192 16.0 / 12.5, R = 8192 x 4096 38.5 / 30.7, R = 4096 x 4096 18.9 / 22.5;
+// * one vector: R = 1024 x 14336 16.9 / 14.1, R = 2048 x 4096 9.0 / 8.1, but R = 4096 x 4096
+//   11.6 / 12.7, R = 2048 x 8192 12.9 / 13.6; R = 8192 x 4096 23.0 / 18.2 (Q8_0 26.3 / 21.1),
+//   R = 28672 x 8192 94 / 97 (Q4_1 R = 11008 x 4096 23.7 / 25.1); F16 4.6 / 3.9 to 185 / 153;
+// * five to eight: R = 64 x 4096 8.1 / 6.8, R = 256 x 8192 11.4 / 9.7, but R = 512 x 8192 11.4 /
+//   14.5, R = 256 x 2048 6.8 / 6.7; nine and more 300 + 70 rows x 5664 11.4 / 12.6;
+// * three matrices: 300 + 70 + 20 rows x 8192, one to four vectors 11.4 / 8.5, 9.9, 11.8
+//   (F16 14.0 / 8.3, 10.0, 12.0), F16 of one vector 2048 + 512 + 512 x 2048 7.8 / 9.2, 8192 + 1024 + 1024 x 8192 40 / 35.
+bool general_sooner_multi(int type, uint32_t nmat, uint64_t rows, uint32_t cols, uint32_t batch) {
+    const bool f16 = type == kF16;
+    if (nmat == 3u) {
+        if (rows <= 512u && cols >= 4096u) return batch <= (f16 ? 4u : 2u);
+        return f16 && batch == 1u && rows >= 4096u && cols >= 4096u;
+    }
+    if (batch > 4u) return batch <= 8u && rows <= 512u && cols >= 4096u;
+    if (rows <= 1024u || cols <= 512u || (rows <= 2048u && (cols <= 2048u || (f16 && batch == 2u)))) return true;
+    if (batch == 1u)
+        return f16 || rows <= 2048u || (rows <= 4096u && cols <= 4096u) ||
+               (type != kQ4_1 && rows >= 16384u && cols <= 4096u);
+    return f16 && batch == 2u && rows >= 16384u;
+}
+
 }  // namespace
 
 hipError_t launch_blk_linear_batch(int type, uint32_t nmat, const uint8_t *const w[], const uint32_t rows[],
@@ -435,7 +463,10 @@ hipError_t launch_blk_linear_batch(int type, uint32_t nmat, const uint8_t *const
         tiles += (rows[m] + 15u) / 16u;
         a.tile_end[m] = tiles;
     }
-    if (nmat == 1u && general_sooner(type, rows[0], cols, batch)) return hipErrorNotSupported;
+    uint64_t all_rows = 0;
+    for (uint32_t m = 0; m < nmat; m++) all_rows += rows[m];
+    if (nmat == 1u ? general_sooner(type, rows[0], cols, batch) : general_sooner_multi(type, nmat, all_rows, cols, batch))
+        return hipErrorNotSupported;
     const uint32_t pcols = (cols + 255u) & ~255u;
     hipError_t why;
     const size_t need = (size_t)((batch + kBatchMax - 1u) / kBatchMax) * xb_layout(pcols).bytes;
