@@ -900,6 +900,27 @@ def test_attention_long_splits(dev, host, oracle, mem, hd, nqh, nkh, seq):
         assert np.all(np.abs(got[fine] - want[fine]) <= 1e-4 + 1e-4 * np.abs(want[fine]))
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("nqh,nkh", [(1, 1), (8, 1), (6, 2), (32, 8), (80, 80)])
+def test_attention_exact_weights(dev, host, mem, hd, nqh, nkh):
+    """One position weighs exactly 1: its value comes back in every bit, whatever its
+    score. So do equal values at positions of equal scores, over one tile
+    and several (counts that are powers of two, so that every sum is exact)."""
+    group = nqh // nkh
+    for seq in (1, 2, 32, 64, 128):
+        k = V.synth_normal_f16(host, nkh * hd, SEED, 187)
+        v = V.synth_normal_f16(host, nkh * hd, SEED, 188)
+        q = synth_x(host, nqh * hd, 189) * np.float32(7.3)
+        po = mem.zeros(nqh * hd)
+        dev.attention(mem.up(q), mem.up(np.tile(k, seq)), mem.up(np.tile(v, seq)), po, seq, 0, seq, nqh, nkh, hd,
+                      np.float32(0.31))
+        got = dev.download(po, nqh * hd, np.float32).reshape(nkh, group, hd)
+        want = v.view(np.float16).astype(np.float32).reshape(nkh, 1, hd)
+        if seq == 1 or (hd <= 64 and nkh <= 32):  # (the one launch, its scores against the joint maximum)
+            assert np.array_equal(got, np.broadcast_to(want, got.shape)), seq
+        assert np.all(np.abs(got - want) <= 1e-6 * np.abs(want)), seq
+
+
 @pytest.mark.parametrize("qscale", [1e-6, 1e4])
 def test_attention_q_magnitude(dev, host, oracle, mem, qscale):
     """q far from unit scale (the matrix-core kernel rescales each head's q

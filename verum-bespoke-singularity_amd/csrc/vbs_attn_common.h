@@ -203,7 +203,8 @@ __device__ __forceinline__ float2 merge_residue_sum(const float *ph, uint32_t nc
     return make_float2(ox, oy);
 }
 
-// The four residues in order, scaled by 1 / L.
+// The four residues in order, scaled by 1 / L (head sizes but 128: divided by L, one rounding less).
+template <uint32_t HD = 128>
 __device__ __forceinline__ float2 merge_finish(const float2 a[kMergeRes], float L) {
     float2 s = a[0];
 #pragma unroll
@@ -211,6 +212,7 @@ __device__ __forceinline__ float2 merge_finish(const float2 a[kMergeRes], float 
         s.x += a[r].x;
         s.y += a[r].y;
     }
+    if (HD != 128u) return make_float2(__fdiv_rn(s.x, L), __fdiv_rn(s.y, L));
     const float inv = __fdiv_rn(1.0f, L);
     return make_float2(__fmul_rn(s.x, inv), __fmul_rn(s.y, inv));
 }
@@ -257,7 +259,7 @@ __device__ __forceinline__ float2 merge_one_wave(const float *ph, uint32_t nc, u
     float2 a[kMergeRes];
 #pragma unroll
     for (uint32_t r = 0; r < kMergeRes; r++) a[r] = make_float2(ox[r], oy[r]);
-    return merge_finish(a, st.L);
+    return merge_finish<HD>(a, st.L);
 }
 
 }  // namespace vbs

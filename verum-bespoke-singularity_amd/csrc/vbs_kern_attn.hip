@@ -21,6 +21,8 @@
 // matrix-core chunk kernel, but one q head per kv head of 32 or 64 dims past the
 // one-launch lengths k_attn_solo; other shapes the generic one (double dot, one
 // position per four threads).
+#include <type_traits>
+
 #include "vbs_attn_common.h"
 #include "vbs_dev_common.h"
 #include "vbs_internal.h"
@@ -325,8 +327,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_attn_solo(
 // Bound: latency (one or a few tiles per wave) up to HBM at long contexts.
 // Measured (chunk + merge) against the vector-ALU kernel that took head_dim 32
 // and 64 before and the generic one that took 96: 32 q heads over 8 kv heads,
-// 3001 positions, head_dim 32 14.1 -> 8.1 us, 64 13.5 -> 9.0, 96 44.3 -> 10.4; 41
-// positions 9.2 -> 3.5, 8.8 -> 3.9, 28.4 -> 4.4 (one launch). Head_dim 128 over one
+// 3001 positions, head_dim 32 14.1 -> 8.5 us, 64 13.6 -> 9.1, 96 39.2 -> 9.9; 41
+// positions 9.3 -> 3.9, 8.7 -> 4.3, 28.5 -> 4.8 (one launch). Head_dim 128 over one
 // kv head, 16000 positions 37.4 -> 21.1 (the merge's later rows sixteen at a time).
 // The most chunks the matrix-core split gives any sequence of at most max_seq
 // positions: the chunk count grows with the sequence while the chunk length
@@ -363,16 +365,41 @@ typedef uint32_t au4 __attribute__((ext_vector_type(4)));
 // holds, for head n & 7 of its lane n = lane & 15, the chunk maximum m and
 // l = sum e^(s - m); and a[dt][r] = the sum of e^(s - m) v[HD / 16 n + dt] of head
 // 4 (lane >> 4) + r (rows hi + lo added; lane groups 0 and 1 carry them).
-template <uint32_t HD>
+__device__ __forceinline__ float score_max(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ double score_max(double a, double b) { return fmax(a, b); }
+template <int M>
+__device__ __forceinline__ float score_xor(float v) {
+    return lane_xor<M>(v);
+}
+template <int M>
+__device__ __forceinline__ double score_xor(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t h = lane_xor<M>((uint32_t)(b >> 32)), l = lane_xor<M>((uint32_t)b);
+    return __builtin_bit_cast(double, (uint64_t)h << 32 | l);
+}
+
+constexpr uint32_t kOneChunks = 8;  // k_attn_one's waves
+
+// JOINT (one tile per wave, head sizes but 128): the workgroup's n_joint waves
+// take one maximum per head over all their positions, through joint[wave][8]
+// and a barrier (none if n_joint is 0), so that its position and every chunk weigh
+// exactly 1. Short contexts are then as exact as whole f32 products, one position
+// exact: a whole power of two as the chunk's maximum left 6e-8 there (error figures
+// below). It takes 0.2 to 0.5 us (32 q heads over 8 kv heads of 64, 41 positions 3.9 ->
+// 4.25 us, 256 5.3 -> 6.0).
+template <uint32_t HD, bool JOINT = false>
 __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
                                                const uint16_t *__restrict__ kc,
                                                const uint16_t *__restrict__ vc, uint64_t layer_off,
                                                uint32_t s0, uint32_t valid, uint32_t nt,
                                                uint32_t nkh, uint32_t kvh, uint32_t group,
                                                float scale, uint32_t lane, float &m_out,
-                                               float &l_out, float (&a)[HD / 16][4]) {
+                                               float &l_out, float (&a)[HD / 16][4],
+                                               double (*joint)[8] = nullptr, uint32_t n_joint = 0,
+                                               uint32_t wave = 0) {
     constexpr uint32_t KK = HD / 32u, DPL = HD / 16u, VW = DPL / 2u;  // K slices; V dims and words per lane
     constexpr bool FINE = HD != 128u;
+    typedef std::conditional_t<FINE, double, float> Score;
     constexpr float PS = FINE ? 16384.f : 1.f;  // P's scale (f16 would drop lo bits of small weights)
     const uint32_t n = lane & 15u, g = lane >> 4;
     const uint64_t rstride = (uint64_t)nkh * HD;
@@ -436,13 +463,15 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
     const float csc = ldexpf(scale, -sq);
     // FINE (head sizes whose scores were double dots, or sums of eight dims per
     // lane, before this kernel took them): each dot is a double sum of one
-    // product per 16 dims, and the scores are kept times log2 e, s2 = c (dot)
-    // with c in two parts, the maximum rounded up to a whole number so that
-    // no bits of s2 are lost against it. Error against 64 bits, 32 q heads over 8
-    // kv heads, 300 and 3001 positions: head_dim 64 1.4e-7 and 1.8e-7 (1.5 and 1.8
-    // without; 2.1 and 1.9 before), 96 1.6 and 1.9 (2.2 and 2.3; 1.6 and 2.0).
-    const float c2 = FINE ? csc * 1.44269504088896341f : csc;
-    const float c2lo = fmaf(csc, 1.44269504088896341f, -c2) + csc * 1.92596299e-8f;
+    // product per 16 dims and of the hi and lo columns, the scores (times log2 e)
+    // stay double until the maximum is taken off them, that is rounded up to a whole
+    // number (or JOINT), and l adds the weights as they multiply V. Error against 64
+    // bits over 1 to 32 q heads (of the kernels before; of f32 scores -> now), at 2, 7, 45, 228,
+    // 3000 positions, in 1e-8: head_dim 32 6.3, 9.5, 13.4, 16.3, 19.3; 7.8, 10.1, 13.1, 15.7, 19.2
+    // -> 5.8, 8.3, 11.0, 13.0, 17.4; 64 6.5, 9.4, 12.6, 15.0, 18.3; 7.8, 9.7, 13.0, 14.7, 18.5 -> 5.8,
+    // 8.3, 10.5, 11.9, 17.0; 96 5.7, 8.2, 13.4, 15.8, 19.3; 7.9, 10.2, 13.5, 14.9, 19.1 -> 5.9, 8.7,
+    // 11.2, 12.6, 17.7.
+    const double c2 = (double)csc * 1.4426950408889634;
     ah8 Qb[KK];
 #pragma unroll
     for (uint32_t kk = 0; kk < KK; kk++)
@@ -454,7 +483,8 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
         }
 
 
-    float m = -INFINITY, l = 0.f;
+    Score m = -INFINITY;
+    float l = 0.f;
     af4 acc[DPL];
 #pragma unroll
     for (uint32_t t = 0; t < DPL; t++) acc[t] = af4{0.f, 0.f, 0.f, 0.f};
@@ -486,49 +516,61 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
         }
         if (t + 1u < nt) load_k(t + 1u);  // the K registers are free again
         // scores of positions p_j: hi + lo columns (lane n and n ^ 8), scaled, masked
-        float dot[8], sc[8], mt = -INFINITY;
+        Score sc[8], mt = -INFINITY;
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++) {
-            float v;
+            const bool in = pos_of(t, j) < valid;
             if constexpr (FINE) {
                 double d = 0.0;
 #pragma unroll
                 for (uint32_t k = 0; k < 2u * KK; k++) d += (double)S[j >> 2][k][j & 3u];
-                v = (float)d;
+                const uint64_t b = __builtin_bit_cast(uint64_t, d);
+                const uint32_t h = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x128, 0xF, 0xF, false);
+                const uint32_t l = __builtin_amdgcn_update_dpp(0, (int)b, 0x128, 0xF, 0xF, false);
+                sc[j] = in ? (d + __builtin_bit_cast(double, (uint64_t)h << 32 | l)) * c2 : -INFINITY;
             } else {
-                v = S[j >> 2][0][j & 3u];
+                const float v = S[j >> 2][0][j & 3u];
+                const float w = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                                                  0, __builtin_bit_cast(int, v), 0x128,
+                                                                  0xF, 0xF, false));  // row_ror:8
+                sc[j] = in ? __fmul_rn(w, csc) : -INFINITY;
             }
-            const float w = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                                                              0, __builtin_bit_cast(int, v), 0x128,
-                                                              0xF, 0xF, false));  // row_ror:8
-            const bool in = pos_of(t, j) < valid;
-            dot[j] = in ? w : 0.f;
-            sc[j] = in ? __fmul_rn(w, c2) : -INFINITY;
-            mt = fmaxf(mt, sc[j]);
+            mt = score_max(mt, sc[j]);
         }
-        mt = fmaxf(mt, lane_xor<16>(mt));
-        mt = fmaxf(mt, lane_xor<32>(mt));
-        if (FINE) mt = ceilf(mt);
-        const float mn = fmaxf(m, mt);
-        const float rs = m == -INFINITY ? 0.f : merge_exp<HD>(__fsub_rn(m, mn));
+        mt = score_max(mt, score_xor<16>(mt));
+        mt = score_max(mt, score_xor<32>(mt));
+        if constexpr (FINE) {
+            if (JOINT && n_joint) {
+                if (lane < 8u) joint[wave][lane] = mt;
+                __syncthreads();
+                double v[kOneChunks];
+#pragma unroll
+                for (uint32_t w = 0; w < kOneChunks; w++) v[w] = joint[w][n & 7u];
+#pragma unroll
+                for (uint32_t w = 0; w < kOneChunks; w++) mt = w < n_joint ? score_max(mt, v[w]) : mt;
+            } else if (fabs(mt) < 0x1p23) {  // (past that a float has no room for the difference)
+                mt = ceil(mt);
+            }
+        }
+        const Score mn = score_max(m, mt);
+        const float rs = m == -INFINITY ? 0.f : merge_exp<HD>((float)(m - mn));
         m = mn;
         l *= rs;
         ah8 P;
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++) {
             float e;
-            if constexpr (FINE) {  // s2 = n + x, |x| <= 1/2 and a bit: 2^x times an exact 2^(n - m)
-                const float p = __fmul_rn(dot[j], c2), n = rintf(p);
-                const float err = fmaf(dot[j], c2lo, fmaf(dot[j], c2, -p));
-                e = ldexpf(exp2_fast((p - n) + __builtin_amdgcn_fmed3f(err, -0.5f, 0.5f)), (int)(n - mn));
+            if constexpr (FINE) {  // 2^(n + x), |x| <= 1/2
+                const double d = sc[j] - mn, n = rint(d);
+                e = ldexpf(exp2_fast((float)(d - n)), (int)n);
             } else {
                 e = fast_exp(__fsub_rn(sc[j], mn));
             }
             if (sc[j] == -INFINITY) e = 0.f;
-            l += e;
             const float es = e * PS;
-            const _Float16 hi = (_Float16)es;
-            P[j] = n < 8u ? hi : (_Float16)(es - (float)hi);
+            const _Float16 hi = (_Float16)es, lo = (_Float16)(es - (float)hi);
+            l += FINE ? (float)hi + (float)lo : e;  // (FINE: the sum of the weights as they multiply V)
+            P[j] = n < 8u ? hi : lo;
         }
         // D rows 4 g + r of the P V accumulators belong to head (4 g + r) & 7
         float rsr[4];
@@ -560,8 +602,8 @@ __device__ __forceinline__ void attn_mfma_wave(const float *__restrict__ q,
     for (uint32_t dt = 0; dt < DPL; dt++)
 #pragma unroll
         for (uint32_t r = 0; r < 4; r++) a[dt][r] = (acc[dt][r] + lane_xor<32>(acc[dt][r])) * (1.f / PS);
-    m_out = m;
-    l_out = l;
+    m_out = (float)m;
+    l_out = l * (1.f / PS);
 }
 
 // A chunk's (m, l, acc) to its partials row (chunk rows `stride` apart per q
@@ -776,7 +818,6 @@ __global__ __launch_bounds__(MULTI ? 64 * kFineWaves : 64) void k_attn_mfma(cons
 // takes the kv head's chunks one per wave, as k_attn_mfma does (bit-identical:
 // the same split, arithmetic and merge), leaves the partials in LDS and merges
 // its q heads there.
-constexpr uint32_t kOneChunks = 8;
 
 template <uint32_t HD>
 __global__ __launch_bounds__(64 * kOneChunks) void k_attn_one(
@@ -788,11 +829,16 @@ __global__ __launch_bounds__(64 * kOneChunks) void k_attn_one(
     if (pos_dev) seq_len = pos_dev[0] + 1u;
     // (mfma_split's bound on the chunk count is not met at such lengths)
     const AttnSplit sp = attn_split(seq_len, nkh, kMfmaGran, kMfmaLmax, kMfmaTargetWgs);
+    __shared__ double joint[HD == 128u ? 1 : kOneChunks][8];
+    const bool is_joint = HD != 128u && sp.len == kMfmaGran;
     if (wave < sp.n) {
         const uint32_t s0 = wave * sp.len, valid = min(sp.len, seq_len - s0);
         float m, l, a[HD / 16][4];
-        attn_mfma_wave<HD>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane, m, l, a);
+        attn_mfma_wave<HD, HD != 128u>(q, kc, vc, layer_off, s0, valid, sp.len / kMfmaGran, nkh, kvh, group, scale, lane,
+                                       m, l, a, joint, is_joint ? sp.n : 0u, wave);
         attn_mfma_store<HD>(part, kOneChunks, wave, group, lane, m, l, a);
+    } else if (is_joint) {
+        __syncthreads();  // (attn_mfma_wave's)
     }
     __syncthreads();
     uint32_t again = 0;  // heads whose results are not finite (attn_head_whole)
@@ -949,7 +995,7 @@ __global__ __launch_bounds__(64 * kMergeRes) void k_attn_merge_hd(
 #pragma unroll
         for (uint32_t r = 0; r < kMergeRes; r++) a[r] = red[r][lane];
         if (HD == 128u || lane < HD / 2u)
-            *reinterpret_cast<float2 *>(out + (uint64_t)h * HD + 2u * lane) = merge_finish(a, st.L);
+            *reinterpret_cast<float2 *>(out + (uint64_t)h * HD + 2u * lane) = merge_finish<HD>(a, st.L);
     }
 }
 
@@ -975,8 +1021,8 @@ static hipError_t launch_mfma_hd(const float *q, const uint16_t *kc, const uint1
                                  float *part, uint32_t seq_len, const uint32_t *pos_dev, uint64_t layer_off,
                                  uint32_t nkh, uint32_t group, float scale, hipStream_t s) {
     const uint32_t chunks = mfma_grid_chunks<HD>(seq_len, nkh), stride = attn_max_chunks(seq_len, nkh);
-    // One launch: 41 positions of 8 kv heads 3.4-4.6 us (chunks and merge 6.5-9),
-    // 256 of head_dim 64 4.8 (8.8); at head_dim 128 and eight q heads per kv head
+    // One launch: 41 positions of 8 kv heads 3.7-4.8 us (chunks and merge 6.4-7.5),
+    // 256 of head_dim 64 5.4-6.0 (6.4-7.0); at head_dim 128 and eight q heads per kv head
     // 256 positions are too many for one workgroup (7.9 against 7.1), 96 alike.
     if (chunks <= (HD <= 64u ? kOneChunks : kOneChunks / 2u)) {
         const uint32_t nw = chunks > group ? chunks : group;  // a wave per chunk, then per q head
