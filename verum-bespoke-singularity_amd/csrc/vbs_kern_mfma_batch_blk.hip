@@ -15,7 +15,7 @@
 // group read 256 contiguous bytes). The operand is the bare quant, exact in
 // f16: q (Q8_0), nibble - 8 (Q4_0), nibble (Q4_1), the weight itself (F16). D
 // is then the block's dot with each plane in fp32 and the block's d multiplies
-// it: y += d D (F16: the unit's eight MFMAs chain into D instead). Q4_1's
+// it: y += d D (F16: the unit's eight D are added up). Q4_1's
 // d nib + m adds m times the block's sum of x by one more MFMA per unit, A the
 // unit's eight sub-block sums (x'/32, hi and lo planes), B the eight mins.
 //
@@ -163,7 +163,10 @@ struct BlkB {
 };
 
 // F16 rows of a multiple of 8 elements at 16-byte alignment: the operands are
-// loaded where they are used, no LDS.
+// loaded where they are used, no LDS. Each MFMA has a sum of its own, added in a
+// tree: chained, the rounding of short rows was larger than that of the VALU kernel
+// before (256 and 512 columns, error against 64 bits 7.8 and 8.6e-8 there, two chains
+// 9.5 and 9.9, now 8.2 and 8.7; the general kernel's 8.1 and 8.6), for no time.
 struct F16B {
     static constexpr int TYPE = kF16;
     static constexpr uint32_t BYTES = 512, NLD = 8, SCRATCH = 0;
@@ -179,20 +182,22 @@ struct F16B {
     __device__ static void dot(const u32x4 *r, const uint8_t *, const Src &, uint32_t u, uint32_t cols,
                                uint32_t, uint32_t g, const h8 (&A)[VG][8], const h8 (&)[VG],
                                float (&acc)[VG][2]) {
-        f4 D[VG][2];
-#pragma unroll
-        for (uint32_t v = 0; v < VG; v++) D[v][0] = D[v][1] = f4{0.f, 0.f, 0.f, 0.f};
+        f4 D[VG][8];
 #pragma unroll
         for (uint32_t m = 0; m < 8u; m++) {
             const u32x4 z = {0u, 0u, 0u, 0u};
             const h8 B = __builtin_bit_cast(h8, 256u * u + 32u * m + 8u * g < cols ? r[m] : z);
 #pragma unroll
             for (uint32_t v = 0; v < VG; v++)
-                D[v][m & 1u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[v][m], B, D[v][m & 1u], 0, 0, 0);
+                D[v][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[v][m], B, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         }
 #pragma unroll
         for (uint32_t v = 0; v < VG; v++) {
-            const f4 S = D[v][0] + D[v][1];
+#pragma unroll
+            for (uint32_t w = 4u; w; w /= 2u)
+#pragma unroll
+                for (uint32_t k = 0; k < w; k++) D[v][k] += D[v][k + w];
+            const f4 S = D[v][0];
             acc[v][0] += S[0] + S[1];
             acc[v][1] += S[2] + S[3];
         }
