@@ -73,8 +73,7 @@ __global__ __launch_bounds__(S > 4 ? 64 * S : 256) void k_rows(const uint8_t *__
     constexpr uint32_t kWaves = S > 4u ? S : 4u, kGroups = kWaves / S, L = P::E / 8u;  // lanes per block
     // rows on one wave (short ones): all NB vectors are formed, without a branch
     // between their loads; those past the batch repeat its last and are dropped
-        constexpr bool kAll = NB > 1u && R <= 2u && S == 1u;
-
+    constexpr bool kAll = NB > 1u && R <= 2u && S == 1u;
     __shared__ float red[S > 1 ? kWaves : 1][R * NB];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t part = S > 1u ? wave % S : 0u;

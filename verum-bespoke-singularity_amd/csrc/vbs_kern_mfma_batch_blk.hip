@@ -26,14 +26,16 @@
 // from the wave's LDS slot (two in flight cost registers and were slower:
 // 22016 x 4096 Q8_0 33.7 against 29.8 us).
 //
-// Bound: no one unit; a CU's two waves per SIMD add up L1 traffic (A and
-// weights), LDS and VALU work per item that overlap only in part. Measured
+// Bound: each wave's chain of load, LDS, unpack, MFMA and scale, with 1.3 to 1.6
+// waves per SIMD in flight (Q8_0, 8 vectors: vector ALU 26-37% busy, LDS 6-9%, matrix
+// cores 3-5%, 3.0 to 4.3 TB/s fetched). Measured
 // with its x preparation, weights from HBM, 8 vectors, against the VALU kernel
 // it replaced: Q8_0 4096 x 4096 72.5 -> 10.7 us, 11008 x 4096 251.7 -> 16.7
-// (2.9 TB/s), 4096 x 11008 199.2 -> 19.2; Q4_0 11008 x 4096 170.4 -> 14.5; F16
+// (2.9 TB/s), 4096 x 11008 199.2 -> 18.9; Q4_0 11008 x 4096 170.4 -> 14.5; F16
 // 11008 x 4096 315 -> 24.3 (3.7 TB/s); 16 vectors, Q8_0 11008 x 4096 445 -> 23.7.
 // About 6 us of each is the fixed cost of the two launches.
-// Error against 64 bits 0.7 to 1.3e-7 (the VALU kernel's 1.0 to 2.4e-7).
+// Error against 64 bits 0.7 to 1.3e-7 (the VALU kernel's 1.0 to 2.4e-7; F16 rows of 128
+// to 256 elements 5% over its, 7.8 -> 8.2e-8: the 22 bits of x).
 //
 // Results that are not finite (an inf or NaN in x makes its whole block's
 // planes NaN here) are computed again by a wave each in the general kernel's
